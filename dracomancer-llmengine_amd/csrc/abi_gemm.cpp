@@ -2,8 +2,8 @@
 //
 // m5_gemm_auto: src/m5/m5_gemm_fused.c:231-241 (0 = done, -1 = code not served,
 // the caller falls back); m5_gemm: src/m5/m5_gemm.c:249-272 (Y[T x n_out] =
-// X[T x n_in] . W^T).  Host pointers.  Q4_K / Q6_K run on the f16-MFMA GEMM
-// (gemmh.hip); Q8_0 and Q5_K run as one device GEMV per token.  The int8-MFMA kernels
+// X[T x n_in] . W^T).  Host pointers.  Q4_K, Q5_K, Q6_K and Q8_0 run on the
+// f16-MFMA GEMM (gemmh.hip).  The int8-MFMA kernels
 // of gemm.hip serve the grouped expert GEMMs of m6_moe_tok only.
 // m5_dequant_row: src/m5/m5_gemm.c:55-235, the GEMM library's row decoder.
 #include <stdio.h>
@@ -19,42 +19,67 @@ extern "C" int draco_repack(int code, const uint8_t* src, int n_out, int n_in, u
 
 using namespace draco;
 
-int draco_enqueue_gemm(const DracoMat& m, const float* X, int T, float* Y, uint8_t* digits, bool have_digits,
-                       hipStream_t st) {
-    if (m.L.code != DRACO_Q4_K && m.L.code != DRACO_Q6_K) {  // Q8_0 and the plain formats: one GEMV per token
-        for (int t = 0; t < T; t++)
-            if (draco_gemv_launch(m, X + (size_t)t * m.L.n_in, Y + (size_t)t * m.L.n_out, nullptr, 0, m.L.n_out, st))
-                return fail(-1, "gemm: gemv launch rejected");
+int draco_enqueue_gemms(const GemmTo* to, int n, const float* X, int T, uint8_t* digits, hipStream_t st) {
+    bool have = false;  // X's operands are in `digits`
+    GemmHArgs a = {};
+    for (int i = 0; i < n; i++) {
+        const DracoMat& m = *to[i].m;
+        if (!draco_gemmh_serves(m.L.code)) {  // the plain formats: one GEMV per token
+            for (int t = 0; t < T; t++)
+                if (draco_gemv_launch(m, X + (size_t)t * m.L.n_in, to[i].Y + (size_t)t * m.L.n_out, nullptr, 0, m.L.n_out, st))
+                    return fail(-1, "gemm: gemv launch rejected");
+            continue;
+        }
+        if (!have && draco_gemmh_x_launch(X, T, m.L.n_in, digits, st)) return fail(-1, "gemm: activation launch rejected");
+        have = true;
+        a.n_in = m.L.n_in;
+        a.T = T;
+        a.xh = digits;
+        GemmHSeg& s = a.seg[a.nseg++];
+        s.W = m.dev;
+        s.L = m.L;
+        s.Y = to[i].Y;
+        s.ldy = m.L.n_out;
+        // launched when full, or when the next matrix cannot join
+        bool more = a.nseg < 3 && i + 1 < n && draco_gemmh_serves(to[i + 1].m->L.code);
+        for (int k = 0; more && k < a.nseg; k++) more = draco_gemmh_mixes(a.seg[k].L.code, to[i + 1].m->L.code);
+        if (more) continue;
+        if (draco_gemmh_launch(a, st)) return fail(-1, "gemm: launch rejected");
+        a = GemmHArgs{};
+    }
+    // (a plain-format matrix in between leaves an unlaunched group)
+    if (a.nseg && draco_gemmh_launch(a, st)) return fail(-1, "gemm: launch rejected");
+    return 0;
+}
+
+int draco_enqueue_swiglu(const DracoMat& gate, const DracoMat& up, const float* X, int T, float* G, float* U,
+                         uint8_t* digits, hipStream_t st) {
+    if (!draco_gemmh_serves(gate.L.code) || gate.L.code != up.L.code || gate.L.n_out != up.L.n_out) {
+        const GemmTo to[2] = {{&gate, G}, {&up, U}};
+        if (int rc = draco_enqueue_gemms(to, 2, X, T, digits, st)) return rc;
+        dk_swiglu(G, U, T * gate.L.n_out, st);
         return 0;
     }
-    if (!have_digits && draco_gemmh_x_launch(X, T, m.L.n_in, digits, st))
-        return fail(-1, "gemm: activation launch rejected");
+    if (draco_gemmh_x_launch(X, T, gate.L.n_in, digits, st)) return fail(-1, "gemm: activation launch rejected");
     GemmHArgs a = {};
-    a.W = m.dev;
-    a.L = m.L;
-    a.n_in = m.L.n_in;
+    a.nseg = 2;
+    a.pair = 1;
+    a.n_in = gate.L.n_in;
     a.T = T;
     a.xh = digits;
-    a.Y = Y;
-    a.ldy = m.L.n_out;
-    const size_t pf = draco_gemmh_part_floats(m.L, T, a.ldy);
-    if (pf) {
-        // grow-only; callers that capture graphs enqueue once before capturing
-        a.part = (float*)scratch(12, sizeof(float) * pf);
-        if (!a.part) return -2;
-    }
+    a.seg[0] = {gate.dev, nullptr, gate.L, G, gate.L.n_out, 0, 0};
+    a.seg[1] = {up.dev, nullptr, up.L, nullptr, gate.L.n_out, 0, 0};
     if (draco_gemmh_launch(a, st)) return fail(-1, "gemm: launch rejected");
     return 0;
 }
 
 namespace {
 
-bool served(int code) {
-    return code == DRACO_Q4_K || code == DRACO_Q6_K || code == DRACO_Q8_0 || code == DRACO_Q5_K;
-}
+bool served(int code) { return draco_gemmh_serves(code); }
 
 int enqueue_gemm(const DracoMat& m, const float* X, int T, float* Y, uint8_t* digits, hipStream_t st) {
-    return draco_enqueue_gemm(m, X, T, Y, digits, false, st);
+    const GemmTo to = {&m, Y};
+    return draco_enqueue_gemms(&to, 1, X, T, digits, st);
 }
 
 int gemm_host(int code, const float* X, const uint8_t* W, int T, int n_out, int n_in, float* Y) {
@@ -68,8 +93,8 @@ int gemm_host(int code, const float* X, const uint8_t* W, int T, int n_out, int 
     hipStream_t st = stream();
     float* dx = (float*)scratch(0, sizeof(float) * (size_t)T * n_in);
     float* dy = (float*)scratch(1, sizeof(float) * (size_t)T * n_out);
-    uint8_t* dd = code == DRACO_Q8_0 ? nullptr : (uint8_t*)scratch(7, draco_gemm_digit_bytes(T, n_in));
-    if (!dx || !dy || (code != DRACO_Q8_0 && !dd)) return -2;
+    uint8_t* dd = (uint8_t*)scratch(7, draco_gemm_digit_bytes(T, n_in));
+    if (!dx || !dy || !dd) return -2;
     DRACO_HIP(hipMemcpyAsync(dx, X, sizeof(float) * (size_t)T * n_in, hipMemcpyHostToDevice, st));
     if (int rc = enqueue_gemm(*m, dx, T, dy, dd, st)) return rc;
     DRACO_HIP(hipGetLastError());
@@ -180,7 +205,7 @@ int m5_dequant_row(int code, const uint8_t* row, int n_in, float* out) {
 // GEMM kernel alone (digits computed once).
 int draco_bench_gemm(int code, const uint8_t* W, int n_out, int n_in, int T, int n_copies, int iters, float* out) {
     std::lock_guard<std::recursive_mutex> g(api_mutex());
-    if (code != DRACO_Q4_K && code != DRACO_Q6_K) return fail(-1, "bench gemm: code %d not on the MFMA path", code);
+    if (!served(code)) return fail(-1, "bench gemm: code %d not on the MFMA path", code);
     if (int rc = ensure_init()) return rc;
     DracoLayout L;
     if (draco_layout(code, n_out, n_in, &L) || T < 1) return fail(-1, "bench gemm: bad shape");
@@ -202,11 +227,9 @@ int draco_bench_gemm(int code, const uint8_t* W, int n_out, int n_in, int T, int
     DRACO_HIP(hipMalloc(&dd, draco_gemm_digit_bytes(T, n_in)));
     DRACO_HIP(hipMemcpy(dx, xh.data(), sizeof(float) * xh.size(), hipMemcpyHostToDevice));
     hipStream_t st = stream();
-    // one eager product first: it sizes the K-split scratch outside the capture
+    // one eager product first: it writes the activation operands
     if (enqueue_gemm(mats[0], dx, T, dy, dd, st)) return -1;
     DRACO_HIP(hipStreamSynchronize(st));
-    float* part = (float*)scratch(12, sizeof(float) * (draco_gemmh_part_floats(L, T, n_out) + 1));
-    if (!part) return -2;
     hipEvent_t e0, e1;
     DRACO_HIP(hipEventCreate(&e0));
     DRACO_HIP(hipEventCreate(&e1));
@@ -219,14 +242,11 @@ int draco_bench_gemm(int code, const uint8_t* W, int n_out, int n_in, int T, int
                 enqueue_gemm(mats[i % n_copies], dx, T, dy, dd, st);
             } else {
                 GemmHArgs b = {};
-                b.W = mats[i % n_copies].dev;
-                b.L = L;
+                b.nseg = 1;
                 b.n_in = n_in;
                 b.T = T;
                 b.xh = dd;
-                b.Y = dy;
-                b.ldy = n_out;
-                b.part = part;
+                b.seg[0] = {mats[i % n_copies].dev, nullptr, L, dy, n_out, 0, 0};
                 draco_gemmh_launch(b, st);
             }
         }

@@ -858,21 +858,17 @@ int enqueue_prefill_layer(DevModel* m, int l, int T, int pos0, int row0, float e
     const float* tab = rope_dev(a->rot, a->base, pos0 + T);
     if (!tab) return -2;
     if (!xn_ready && pf_rms(b.X, m->anorm[l], b.Xn, T, H, eps, st)) return fail(-1, "prefill: rms rejected");
-    // the digits of Xn are written by the first K-quant product and reused by the others
-    auto kquant = [](const DracoMat* x) { return x->L.code == DRACO_Q4_K || x->L.code == DRACO_Q6_K; };
-    if (draco_enqueue_gemm(*a->wq, b.Xn, T, b.Q, b.dig, false, st)) return -1;
-    if (draco_enqueue_gemm(*a->wk, b.Xn, T, b.K, b.dig, kquant(a->wq), st)) return -1;
-    if (draco_enqueue_gemm(*a->wv, b.Xn, T, b.V, b.dig, kquant(a->wq) || kquant(a->wk), st)) return -1;
+    const GemmTo qkv[3] = {{a->wq, b.Q}, {a->wk, b.K}, {a->wv, b.V}};
+    if (draco_enqueue_gemms(qkv, 3, b.Xn, T, b.dig, st)) return -1;
     if (pf_rope_append(b.Q, b.K, b.V, a->kc, a->vc, tab, pos0, row0, T, a->NH, a->NKV, a->HD, a->rot, st))
         return fail(-1, "prefill: rope rejected");
     if (pf_attention(b.Q, a->kc, a->vc, b.part, b.O, row0, T, a->NH, a->NKV, a->HD, a->scale, st))
         return fail(-1, "prefill: attention shape NH=%d NKV=%d HD=%d not served", a->NH, a->NKV, a->HD);
-    if (draco_enqueue_gemm(*a->wo, b.O, T, b.Y, b.dig, false, st)) return -1;
+    const GemmTo o = {a->wo, b.Y}, dn = {f->d, b.Y};
+    if (draco_enqueue_gemms(&o, 1, b.O, T, b.dig, st)) return -1;
     if (pf_add_rms(b.X, b.Y, m->fnorm[l], b.Xn, T, H, eps, st)) return fail(-1, "prefill: rms rejected");
-    if (draco_enqueue_gemm(*f->g, b.Xn, T, b.G, b.dig, false, st)) return -1;
-    if (draco_enqueue_gemm(*f->u, b.Xn, T, b.U, b.dig, kquant(f->g), st)) return -1;
-    dk_swiglu(b.G, b.U, T * f->FF, st);
-    if (draco_enqueue_gemm(*f->d, b.G, T, b.Y, b.dig, false, st)) return -1;
+    if (draco_enqueue_swiglu(*f->g, *f->u, b.Xn, T, b.G, b.U, b.dig, st)) return -1;
+    if (draco_enqueue_gemms(&dn, 1, b.G, T, b.dig, st)) return -1;
     // the residual; fused with the next layer's input RMSNorm when there is one
     if (l + 1 < m->n_layer) {
         if (pf_add_rms(b.X, b.Y, m->anorm[l + 1], b.Xn, T, H, eps, st)) return fail(-1, "prefill: rms rejected");

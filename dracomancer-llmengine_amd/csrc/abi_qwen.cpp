@@ -1029,14 +1029,17 @@ int qstack_positions(QStack* s, int pos0, int n) {
 // src/qwen35_prefill.py:209-239 (_gdn :110-135, _full :137-168), with the
 // projections as f16-MFMA GEMMs over the chunk and the scan token-serial
 int enqueue_qchunk(QStack* s, int T, int pos0, hipStream_t st) {
-    auto kq = [](const DracoMat* m) { return m->L.code == DRACO_Q4_K || m->L.code == DRACO_Q6_K; };
+    auto gemm = [&](const DracoMat* m, const float* X, float* Y) {
+        const GemmTo to = {m, Y};
+        return draco_enqueue_gemms(&to, 1, X, T, s->dig, st);
+    };
     for (int l = 0; l < s->n_layer; l++) {
         QLayer& q = s->L[l];
         if (q.desc.kind == 0) {
             const GdnDev& g = q.g;
             if (pf_rms(s->X, g.attn_norm, s->Xn, T, QH, QEPS, st)) return fail(-1, "qwen prefill: rms rejected");
-            if (draco_enqueue_gemm(*g.qkv, s->Xn, T, s->QKV, s->dig, false, st)) return -1;
-            if (draco_enqueue_gemm(*g.gate, s->Xn, T, s->Z, s->dig, kq(g.qkv), st)) return -1;
+            const GemmTo in2[2] = {{g.qkv, s->QKV}, {g.gate, s->Z}};
+            if (draco_enqueue_gemms(in2, 2, s->Xn, T, s->dig, st)) return -1;
             if (pf_gdn_gates(s->Xn, T, QH, g.bw, g.aw, g.ssm_dt, g.ssm_a, s->B, s->G, g.n_vh, st))
                 return fail(-1, "qwen prefill: gates rejected");
             GdnArgs a = {};
@@ -1056,28 +1059,25 @@ int enqueue_qchunk(QStack* s, int T, int pos0, hipStream_t st) {
             a.nspl = T == 1 ? 1 : draco_gdn_split(false);
             a.PSS = s->PPSS;
             if (draco_gdn_scan_launch(a, st)) return fail(-1, "qwen prefill: scan rejected");
-            if (draco_enqueue_gemm(*g.out, s->ON, T, s->Y, s->dig, false, st)) return -1;
+            if (gemm(g.out, s->ON, s->Y)) return -1;
             if (pf_add_rms(s->X, s->Y, g.post_norm, s->Xn, T, QH, QEPS, st)) return fail(-1, "qwen prefill: rms");
         } else {
             const FullDev& f = q.f;
             if (pf_rms(s->X, f.attn_norm, s->Xn, T, QH, QEPS, st)) return fail(-1, "qwen prefill: rms rejected");
-            if (draco_enqueue_gemm(*f.q, s->Xn, T, s->PQG, s->dig, false, st)) return -1;
-            if (draco_enqueue_gemm(*f.k, s->Xn, T, s->PK, s->dig, kq(f.q), st)) return -1;
-            if (draco_enqueue_gemm(*f.v, s->Xn, T, s->PV, s->dig, kq(f.q) || kq(f.k), st)) return -1;
+            const GemmTo in3[3] = {{f.q, s->PQG}, {f.k, s->PK}, {f.v, s->PV}};
+            if (draco_enqueue_gemms(in3, 3, s->Xn, T, s->dig, st)) return -1;
             dk_fa_prep_rows(s->PQG, f.nh * 2 * FHD, s->PQr, s->PK, s->PV, q.kc, q.vc, f.q_norm, f.k_norm, q.cs,
                             nullptr, pos0, pos0, f.nh, T, st);
             if (pf_attention256(s->PQr, q.kc, q.vc, s->Ppart, s->AO, pos0, T, f.nh, FNKV, 1.f / sqrtf((float)FHD),
                                 s->PQG + FHD, f.nh * 2 * FHD, 2 * FHD, st))
                 return fail(-1, "qwen prefill: attention rejected");
-            if (draco_enqueue_gemm(*f.o, s->AO, T, s->Y, s->dig, false, st)) return -1;
+            if (gemm(f.o, s->AO, s->Y)) return -1;
             if (pf_add_rms(s->X, s->Y, f.post_norm, s->Xn, T, QH, QEPS, st)) return fail(-1, "qwen prefill: rms");
         }
         // FFN of the chunk (input Xn = x2n rows, residual into X)
         if (q.desc.ffn_kind == QFFN_DENSE) {
-            if (draco_enqueue_gemm(*q.fg, s->Xn, T, s->PG, s->dig, false, st)) return -1;
-            if (draco_enqueue_gemm(*q.fu, s->Xn, T, s->PU, s->dig, kq(q.fg), st)) return -1;
-            dk_swiglu(s->PG, s->PU, T * q.FF, st);
-            if (draco_enqueue_gemm(*q.fd, s->PG, T, s->Y, s->dig, false, st)) return -1;
+            if (draco_enqueue_swiglu(*q.fg, *q.fu, s->Xn, T, s->PG, s->PU, s->dig, st)) return -1;
+            if (gemm(q.fd, s->PG, s->Y)) return -1;
             pf_add(s->X, s->Y, (size_t)T * QH, st);
         } else if (q.desc.ffn_kind == QFFN_MOE) {
             return fail(-1, "qwen prefill: MoE FFN layers are fed token by token");

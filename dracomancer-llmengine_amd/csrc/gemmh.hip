@@ -1,19 +1,26 @@
 // gemmh.hip -- chunked-prefill GEMM on f16 MFMA (gfx950): Y[t][n] = x_t . W_n
-// for Q4_K / Q6_K weights in the 16-row tile layout (formats.h).
+// for Q4_K, Q5_K, Q6_K and Q8_0 weights in their device layouts (formats.h).
 //
-// Exactness.  The weights enter the MFMA as f16 integers that carry their
-// sub-block scale: Q4_K sc*q (<= 63*15 = 945), Q6_K sh*(q-32) and sl*(q-32)
-// with sc = 8*sh + sl, sl in [0,7] (|values| <= 512); every one is an exact
-// f16.  Per (token, 256-value super-block) the activations are scaled by
-// 2^-e (e = ilogb(max|x|) - 14, so |x'| < 2^15) and split into two f16
-// (hi = f16(x'), lo = f16(x' - hi)); x' - hi - lo is below 2^-22 |x'|.
-// Every f16 x f16 product is exact in the MFMA's fp32 accumulation, so the
-// result differs from the reference's fp32 row dot only by fp32 summation
-// order and that 2^-22 representation step.  Per super-block and row:
+// Exactness.  The weights enter the MFMA as f16 integers: Q4_K sc*q (at most
+// 63*15), Q5_K sc*(q-16) (63*16), Q8_0 q, all exact; Q6_K sc*(q-32) (|.| <= 4096)
+// as its f16 rounding plus the rest (-1, 0 or 1).  Per (token, 256-value
+// super-block) the activations are scaled by 2^-e (e = ilogb(max|x|) - 14, so
+// |x'| < 2^15) and split into two f16 (hi = f16(x'), lo = f16(x' - hi));
+// x' - hi - lo is below 2^-22 |x'|, and so is the one product left out (Q6_K's
+// lo * rest).  f16 x f16 products are exact in the MFMA's fp32 accumulation.
+// Per super-block and row, with 2^e the token's scale:
 //   Q4_K: y += 2^e * (d * sum_k (sc*q)_k x'_k - 32 * dmin * sum_sb m_sb S'_sb)
 //         with S'_sb = 2^-5 * (sum of the sub-block's x'), itself on the MFMA
 //         (K = 8 sub-blocks, hi/lo);
-//   Q6_K: y += 2^e * d * (8 * sum (sh*(q-32)) x' + sum (sl*(q-32)) x').
+//   Q5_K: the same with q - 16 and 512 * d * sum_sb sc_sb S'_sb added;
+//   Q6_K: y += 2^e * d * sum (sc*(q-32)) x';
+//   Q8_0: y += 2^e * sum_blocks d_block * (sum q x').
+// The hi and the lo products accumulate apart: the lo sums are 2^-11 of the
+// hi ones, so their roundings vanish and the hi chain is half as long.
+// Relative error against 64 bits, 2048-wide rows: Q4_K 1.7e-7 (2.3e-7 in one
+// chain, the sub-block sums added in sequence), Q5_K 1.2e-7 (a GEMV with exact
+// integer dots 1.26e-7; not centred 1.8e-7), Q6_K 1.3e-7 (1.6e-7 in one chain),
+// Q8_0 1.05e-7 (its GEMV 1.25e-7).
 //
 // Operand order.  v_mfma_f32_32x32x16_f16: A lane l = row (token) l%32,
 // K 8*(l/32)..+7; B lane l = column (weight row) l%32, same K; C lane l =
@@ -22,16 +29,27 @@
 // lane half u supplies the 8 values 16*G + 8*(s&1) + i of group
 // G = 8*(s>>3) + 2*((s>>1)&3) + u -- for Q4_K the low (s>>1 even) or high
 // nibbles of quant vector (r = s>>3, gh = (s>>2)&1), for Q6_K fragment
-// (s>>1)&3 of lane slot s>>3.  k_gemmh_x writes the activations in the same
-// order, so one activation buffer serves both formats.
+// (s>>1)&3 of lane slot s>>3, for Q8_0 half u of block s>>1.  k_gemmh_x
+// writes the activations in the same order, so one activation buffer serves
+// every format.
 //
-// Blocking.  Block = 4 waves on 32 tokens x 4*RW row tiles of 32 rows; the
-// activation operands of one super-block (34944 B: 16 K-steps x hi/lo x 1 KB,
-// the min-term operands, the 32 token scales) are staged in LDS, double
-// buffered, and read by all four waves; each wave reads a K-step's A once and
-// runs it against its RW row tiles (independent accumulator chains).  Weights stream from global memory (non-temporal loads).
-// Tall-K products split K across blockIdx.z and a reduce kernel sums the
-// partials in a fixed order.
+// The kernel (k_gemmr).  A block is 8 waves on one 32-token tile: NSB
+// super-block slots x 8 / NSB row streams.  A wave holds its super-block's
+// activation operands, hi and lo of 16 K-steps, in 128 VGPRs and runs the
+// block's row tiles past them; a tile's weight registers refill with the next
+// tile's bytes as they fall free; the slots' sums meet in LDS.  So
+// activations are read once per block and pass instead of once per row tile,
+// no wave waits for another inside a tile, and there is no K split over
+// blocks with partials in memory.  What bounds it: issue -- about 365 VALU and
+// 34 MFMA instructions a (row tile, super-block) for Q4_K, which overlap only
+// in part (measured: 5.4k cycles a step of two waves against 2.2k of MFMA and
+// 2.9k of VALU); a 32-token tile re-forms the weights that the next one forms
+// too.  Against the kernel it replaced (activations staged in LDS super-block
+// by super-block, K split over the grid and a reduce launch), us a product
+// incl. reduce: T=256 2048x2048 Q4_K 14.7 -> 8.8, 8192x2048 34.9 -> 27.5,
+// 16384x2048 54.5 -> 49; T=64 12288x2048 20.2 -> 11.6, 2048x4096 13.2 -> 9.4;
+// T=256 512x2048 Q6_K 12.0 -> 6.5, 2048x8192 53.6 -> 47; T=31 Q8_0 960x960
+// 11.7 -> 6.4, 5120x960 13.8 -> 7.0; T=75 2048x2048 Q5_K 11.4 -> 6.8.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -49,30 +67,38 @@ typedef float v16f __attribute__((ext_vector_type(16)));
 constexpr int XH_A = 16 * 2 * 64 * 16;          // A operands of one super-block (bytes)
 constexpr int XH_M = 2 * 64 * 16;               // min-term A operands
 constexpr int XH_SB = XH_A + XH_M + 32 * 4;     // + 32 token scales = 34944 B per (token tile, super-block)
-constexpr int XH_V4 = XH_SB / 16;               // 2184 uint4 per super-block
 
 // ------------------------------------------------------------ activations --
 // Block (b, tt), 256 threads: thread (m = tid/8, sb = tid%8) owns the 32
-// values of sub-block sb of token 32*tt + m in super-block b.
+// values of sub-block sb of token 32*tt + m in super-block b; with `rows` the
+// token's values are row rows[token] of X (negative: zeros), else its own row.
+// Within each 8 the order is 0 2 1 3 4 6 5 7: the weights' bytes 0, 2 and 1, 3
+// of a dword are formed as pairs.  Rows whose
+// length is not a multiple of 256 (Q8_0) are padded with zeros.  An infinite
+// value keeps its sign in hi with lo = 0, so it meets a row's weights as the
+// fp32 dot would (inf * 0 = NaN included); a NaN stays NaN.
+__device__ __forceinline__ constexpr int kord(int i) { return (i & 4) + ((i & 1) << 1) + ((i >> 1) & 1); }
 __global__ __launch_bounds__(256) void k_gemmh_x(const float* __restrict__ X, int T, int n_in,
-                                                 uint8_t* __restrict__ xh) {
+                                                 const int* __restrict__ rows, uint8_t* __restrict__ xh) {
     const int b = blockIdx.x, tt = blockIdx.y, tid = threadIdx.x;
-    const int m = tid >> 3, sb = tid & 7, t = 32 * tt + m, nb = n_in >> 8;
+    const int m = tid >> 3, sb = tid & 7, t = 32 * tt + m, nb = (n_in + 255) >> 8;
     float v[32];
-    const float* src = X + (size_t)t * n_in + (size_t)b * 256 + 32 * sb;
+    const int row = t < T ? (rows ? rows[t] : t) : -1;
+    const bool live = row >= 0 && b * 256 + 32 * sb < n_in;  // whole 32-value blocks (n_in % 32 == 0)
+    const float* src = X + (size_t)max(row, 0) * n_in + (size_t)b * 256 + 32 * sb;
 #pragma unroll
     for (int i = 0; i < 32; i += 4) {
-        const float4 q = t < T ? ld4(src + i) : make_float4(0.f, 0.f, 0.f, 0.f);
+        const float4 q = live ? ld4(src + i) : make_float4(0.f, 0.f, 0.f, 0.f);
         v[i] = q.x; v[i + 1] = q.y; v[i + 2] = q.z; v[i + 3] = q.w;
     }
     float am = 0.f;
 #pragma unroll
     for (int i = 0; i < 32; i++) am = fmaxf(am, fabsf(v[i]));
     am = group_max<8>(am);  // the token's 8 threads are consecutive lanes
-    const int e = am > 0.f ? max(ilogbf(am) - 14, -100) : 0;
+    const int e = am > 0.f ? min(max(ilogbf(am) - 14, -100), 113) : 0;
     const float sdown = __builtin_bit_cast(float, (uint32_t)(127 - e) << 23);  // 2^-e (e in [-100, 113])
     uint8_t* base = xh + ((size_t)tt * nb + b) * XH_SB;
-    float ssum = 0.f;
+    float ssum[4];  // the sub-block's sum, pairwise: the min terms multiply its rounding
 #pragma unroll
     for (int gg = 0; gg < 2; gg++) {           // the two 16-value groups of this sub-block
         const int G = 2 * sb + gg, u = G & 1;
@@ -81,369 +107,592 @@ __global__ __launch_bounds__(256) void k_gemmh_x(const float* __restrict__ X, in
         for (int bh = 0; bh < 2; bh++) {
             const int s = 8 * (G >> 3) + 2 * ((G >> 1) & 3) + bh;
             v8h hi, lo;
+            float xv[8];
 #pragma unroll
             for (int i = 0; i < 8; i++) {
-                const float xs = v[16 * gg + 8 * bh + i] * sdown;
-                ssum += xs;
+                const float xs = v[16 * gg + 8 * bh + kord(i)] * sdown;
+                xv[i] = xs;
                 const _Float16 h = (_Float16)xs;
                 hi[i] = h;
-                lo[i] = (_Float16)(xs - (float)h);
+                lo[i] = fabsf(xs) < INFINITY ? (_Float16)(xs - (float)h) : (_Float16)0.f;
             }
+            ssum[2 * gg + bh] = ((xv[0] + xv[1]) + (xv[2] + xv[3])) + ((xv[4] + xv[5]) + (xv[6] + xv[7]));
             *reinterpret_cast<v8h*>(base + ((size_t)(2 * s) * 64 + lane) * 16) = hi;
             *reinterpret_cast<v8h*>(base + ((size_t)(2 * s + 1) * 64 + lane) * 16) = lo;
         }
     }
-    // min-term operand: lane m (u = 0) holds S'_sb for sb = 0..7 in its 8 K slots;
-    // lanes m + 32 (u = 1) hold zeros
-    const float s5 = ssum * 0.03125f;
+    // min-term operand: lane m (u = 0) holds S'_sb for sb = 0..7 in its 8 K slots
+    // (the same order); lanes m + 32 (u = 1) hold zeros
+    const float s5 = ((ssum[0] + ssum[1]) + (ssum[2] + ssum[3])) * 0.03125f;
     const _Float16 sh = (_Float16)s5;
-    const _Float16 sl = (_Float16)(s5 - (float)sh);
+    const _Float16 sl = fabsf(s5) < INFINITY ? (_Float16)(s5 - (float)sh) : (_Float16)0.f;
     _Float16* mh = reinterpret_cast<_Float16*>(base + XH_A);
     _Float16* ml = reinterpret_cast<_Float16*>(base + XH_A + 64 * 16);
-    mh[m * 8 + sb] = sh;
-    ml[m * 8 + sb] = sl;
-    mh[(m + 32) * 8 + sb] = (_Float16)0.f;
-    ml[(m + 32) * 8 + sb] = (_Float16)0.f;
+    const int so = kord(sb);  // its own inverse
+    mh[m * 8 + so] = sh;
+    ml[m * 8 + so] = sl;
+    mh[(m + 32) * 8 + so] = (_Float16)0.f;
+    ml[(m + 32) * 8 + so] = (_Float16)0.f;
     if (sb == 0) reinterpret_cast<float*>(base + XH_A + XH_M)[m] = __builtin_bit_cast(float, (uint32_t)(127 + e) << 23);
 }
 
-// f16 pairs of (bytes n0, n1) and (n2, n3) of w (each < 64) times c, exactly:
-// the pair (1024 + n) is built by a byte permute, then fma((1024 + n), c, -1024 c)
-// rounds once to the exact n*c (|n*c| <= 2048 by the callers' ranges)
-__device__ __forceinline__ void nib2h(uint32_t w, v2h c2, v2h off2, uint32_t& p01, uint32_t& p23) {
-    const uint32_t a = __builtin_amdgcn_perm(0x64646464u, w, 0x04010400u);
-    const uint32_t b = __builtin_amdgcn_perm(0x64646464u, w, 0x04030402u);
-    const v2h ha = __builtin_bit_cast(v2h, a), hb = __builtin_bit_cast(v2h, b);
-    p01 = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(ha, c2, off2));
-    p23 = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(hb, c2, off2));
-}
-
-__device__ __forceinline__ v8h pack8(uint32_t a, uint32_t b, uint32_t c, uint32_t d) {
-    typedef uint32_t v4u __attribute__((ext_vector_type(4)));
-    return __builtin_bit_cast(v8h, (v4u){a, b, c, d});
-}
-
-__device__ __forceinline__ v8h lds8(const uint8_t* p) { return *reinterpret_cast<const v8h*>(p); }
-
-// stage super-block b's activation block into LDS (all 256 threads)
-__device__ __forceinline__ void stage_load(const uint8_t* src, uint4 (&r)[9], int tid) {
-#pragma unroll
-    for (int k = 0; k < 9; k++) {
-        const int i = tid + 256 * k;
-        r[k] = i < XH_V4 ? *reinterpret_cast<const uint4*>(src + (size_t)i * 16) : make_uint4(0, 0, 0, 0);
-    }
-}
-__device__ __forceinline__ void stage_store(uint8_t* dst, const uint4 (&r)[9], int tid) {
-#pragma unroll
-    for (int k = 0; k < 9; k++) {
-        const int i = tid + 256 * k;
-        if (i < XH_V4) *reinterpret_cast<uint4*>(dst + (size_t)i * 16) = r[k];
-    }
-}
-
 // ------------------------------------------------------------------ GEMM --
-// Raw weight registers of one (32-row tile, super-block) for lane (n, u).
+__device__ __forceinline__ v8h pack8(uint32_t a, uint32_t b, uint32_t c, uint32_t d) {
+    return __builtin_bit_cast(v8h, (v4u32){a, b, c, d});
+}
+__device__ __forceinline__ v8h lds8(const uint8_t* p) { return *reinterpret_cast<const v8h*>(p); }
+__device__ __forceinline__ v2h h2(uint32_t w) { return __builtin_bit_cast(v2h, w); }
+__device__ __forceinline__ uint32_t u2(v2h h) { return __builtin_bit_cast(uint32_t, h); }
+__device__ __forceinline__ v2h splat(float v) { return (v2h){(_Float16)v, (_Float16)v}; }
+__device__ __forceinline__ v16f mfma16(v8h a, v8h b, v16f c) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
+}
+// (w & m) | k: with k = 0x64006400 the f16 pair (1024 + byte 0, 1024 + byte 2)
+// of w & m.  The constant is held in a VGPR (magic_k): v_and_or_b32 takes one scalar operand, and with two constants the
+// compiler uses two instructions (445 -> 365 VALU a tile).
+__device__ __forceinline__ uint32_t magic(uint32_t w, uint32_t m, uint32_t k) { return (w & m) | k; }
+__device__ __forceinline__ uint32_t magic_k(uint32_t k) {
+    asm volatile("" : "+v"(k));
+    return k;
+}
+// (byte 0, byte 2) and (byte 1, byte 3) of w as f16 pairs, plus 1024
+__device__ __forceinline__ void pairs(uint32_t w, uint32_t mk, v2h& a, v2h& b) {
+    a = h2(magic(w, 0x00FF00FFu, mk));
+    b = h2(magic(w >> 8, 0x00FF00FFu, mk));
+}
+
+// One wave's raw weights of a (32-row tile, super-block), lane (n, u): row n
+// of the tile, lane half u.  FM 1 = Q4_K, 2 = Q6_K, 3 = Q8_0, 4 = Q5_K.
 template <int FM>
 struct WFrag;
 template <>
-struct WFrag<1> {  // Q4_K: quant vectors (r, gh) = (v>>1, v&1), the row header
+struct WFrag<1> {  // quant vectors (r, gh) = (v>>1, v&1), the row header
     uint4 qv[4], h;
 };
 template <>
-struct WFrag<2> {  // Q6_K: ql A, ql B, qh and 4 scales of lane slots g2 = 0, 1; d
+struct WFrag<4> {  // the Q4_K ones, then the 16 fifth-bit bytes of half u
+    uint4 qv[4], h, qh;
+};
+template <>
+struct WFrag<2> {  // ql A, ql B, qh and 4 scales of lane slots g2 = 0, 1; d
     uint4 qa[2], qb[2], qh[2];
     uint32_t sc4[2];
     uint32_t d;
 };
+template <>
+struct WFrag<3> {  // the 16 quants of (block k, half u) of the 8 blocks, and the blocks' f16 scales
+    uint4 q[8];
+    uint32_t d[8];
+    int live;  // blocks that the row has from this super-block on
+};
 
-__device__ __forceinline__ void wload(const uint8_t* item, int j, int u, WFrag<1>& f) {
-#pragma unroll
-    for (int v = 0; v < 4; v++) f.qv[v] = ldnt4(item + (v >> 1) * 1024 + 16 * (j + 16 * (2 * (v & 1) + u)));
-    f.h = ldnt4(item + 2048 + 16 * j);
+// Super-block b of 32-row tile t through a buffer descriptor: one wave-uniform
+// base, the lane's offset fixed for the whole kernel (wlane), so walking tiles
+// forms no per-lane address.  Reads past the matrix return zero (the rows
+// after n_out).
+template <int FM>
+__device__ __forceinline__ int wlane(const DracoLayout& L, int n, int u) {
+    constexpr int IB = FM == 1 ? DRACO_Q4T_ITEM : FM == 2 ? DRACO_Q6T_ITEM : DRACO_Q5T_ITEM;
+    if constexpr (FM == 3) return n * L.nb * 32 + 16 * u;
+    else return (n >> 4) * L.nb * IB + 16 * ((n & 15) + 16 * u);
 }
-__device__ __forceinline__ void wload(const uint8_t* item, int j, int u, WFrag<2>& f) {
-#pragma unroll
-    for (int g2 = 0; g2 < 2; g2++) {
-        const int ls = j + 16 * (2 * g2 + u);
-        f.qa[g2] = ldnt4(item + 16 * ls);
-        f.qb[g2] = ldnt4(item + 1024 + 16 * ls);
-        f.qh[g2] = ldnt4(item + 2048 + 16 * ls);
-        f.sc4[g2] = *reinterpret_cast<const uint32_t*>(item + 3072 + 4 * ls);
-    }
-    f.d = *reinterpret_cast<const uint16_t*>(item + 3328 + 2 * j);
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc(const uint8_t* base, size_t bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(base), (short)0,
+                                             (int)(bytes > 0x7FFFFFFFu ? 0x7FFFFFFFu : (uint32_t)bytes), 0x00020000);
 }
-
-// RW (32-row tile, super-block) items against the staged activations `cur`:
-// each K-step reads its A operands (hi, lo) from LDS once and runs them
-// against every tile's B, so the LDS traffic per MFMA falls with RW and the
-// RW accumulator chains are independent.  Returns each tile's contribution
-// before the token scale, per C element.
-template <int RW>
-__device__ __forceinline__ void tiles_q4(const WFrag<1> (&f)[RW], const uint8_t* cur, int lane, int u,
-                                         float (&part)[RW][16]) {
-    v16f P[RW], Q[RW];
-    int sc[RW][8];
-    v8h Bm[RW];
-#pragma unroll
-    for (int r = 0; r < RW; r++) {
-        P[r] = (v16f){};
-        Q[r] = (v16f){};
-        // 6-bit scales and mins of the 8 sub-blocks (src/m5_kern_scalar.c:39-46)
-#pragma unroll
-        for (int s8 = 0; s8 < 8; s8++) {
-            int mn;
-            if (s8 < 4) {
-                sc[r][s8] = (f[r].h.y >> (8 * s8)) & 63;
-                mn = (f[r].h.z >> (8 * s8)) & 63;
-            } else {
-                const int s0 = s8 - 4;
-                sc[r][s8] = ((f[r].h.w >> (8 * s0)) & 15) | (((f[r].h.y >> (8 * s0 + 6)) & 3) << 4);
-                mn = ((f[r].h.w >> (8 * s0 + 4)) & 15) | (((f[r].h.z >> (8 * s0 + 6)) & 3) << 4);
-            }
-            // min term: B lane (n, 0) = m_0..m_7 of row n, lanes (n, 1) zero
-            Bm[r][s8] = u ? (_Float16)0.f : (_Float16)mn;
+__device__ __forceinline__ uint4 buf4(__amdgpu_buffer_rsrc_t r, int off) {
+    const v4u32 v = __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0);
+    return make_uint4(v.x, v.y, v.z, v.w);
+}
+template <int FM>
+struct WPtr {
+    __amdgpu_buffer_rsrc_t r, rd;  // rd: Q8_0 scales
+    int vo, n, u, live;
+    __device__ __forceinline__ WPtr(const uint8_t* W, const DracoLayout& L, int t, int b, int vo_, int n_, int u_)
+        : vo(vo_), n(n_), u(u_) {
+        if constexpr (FM == 3) {
+            const size_t e = (size_t)32 * t * L.nb + 8 * b, all = (size_t)L.n_out * L.nb;  // in blocks
+            r = rsrc(W + L.off[0] + e * 32, e < all ? (all - e) * 32 : 0);
+            rd = rsrc(W + L.off[1] + e * 2, e < all ? (all - e) * 2 : 0);
+            live = L.nb - 8 * b;
+        } else {
+            constexpr size_t IB = FM == 1 ? DRACO_Q4T_ITEM : FM == 2 ? DRACO_Q6T_ITEM : DRACO_Q5T_ITEM;
+            const size_t e = (size_t)2 * t * L.nb + b, all = (size_t)L.ntiles * L.nb;
+            r = rsrc(W + e * IB, e < all ? (all - e) * IB : 0);
         }
     }
+    // the pieces of WFrag<FM>, each loaded on its own so that a tile's
+    // registers refill with the next tile's bytes as they fall free
+    __device__ __forceinline__ void hdr(WFrag<FM>& f) const {
+        if constexpr (FM == 1 || FM == 4) f.h = buf4(r, vo + 2048 - 256 * u);
+        if constexpr (FM == 4) f.qh = buf4(r, vo + 2304);
+        if constexpr (FM == 2) {
+            const int j4 = 4 * ((n & 15) + 16 * u);  // this lane's slot, in 4-byte units
 #pragma unroll
-    for (int s = 0; s < 16; s++) {
-        const int v = s >> 2, nib = (s >> 1) & 1, bh = s & 1;
-        const int sbk = 4 * (s >> 3) + ((s >> 1) & 3);  // sub-block of this K-step
-        const v8h Ahi = lds8(cur + ((size_t)(2 * s) * 64 + lane) * 16);
-        const v8h Alo = lds8(cur + ((size_t)(2 * s + 1) * 64 + lane) * 16);
+            for (int g2 = 0; g2 < 2; g2++)
+                f.sc4[g2] = __builtin_amdgcn_raw_buffer_load_b32(r, vo - 3 * j4 + 3072 + 128 * g2, 0, 0);
+            f.d = __builtin_amdgcn_raw_buffer_load_b16(r, vo - 4 * j4 + 3328 + 2 * (n & 15), 0, 0);
+        }
+        if constexpr (FM == 3) {
+            const int vd = (vo - 16 * u) >> 4;
 #pragma unroll
-        for (int r = 0; r < RW; r++) {
-            const uint4 q = f[r].qv[v];
-            uint32_t w0 = bh ? q.z : q.x, w1 = bh ? q.w : q.y;
-            if (nib) {
-                w0 = ((w0 >> 4) & 0x0F0F0F0Fu) ^ 0x08080808u;  // stored XOR 0x80: high nibble u ^ 8
-                w1 = ((w1 >> 4) & 0x0F0F0F0Fu) ^ 0x08080808u;
-            } else {
-                w0 &= 0x0F0F0F0Fu;
-                w1 &= 0x0F0F0F0Fu;
-            }
-            const _Float16 c = (_Float16)sc[r][sbk], o = (_Float16)(-1024.f * (float)sc[r][sbk]);
-            uint32_t p0, p1, p2, p3;
-            nib2h(w0, (v2h){c, c}, (v2h){o, o}, p0, p1);
-            nib2h(w1, (v2h){c, c}, (v2h){o, o}, p2, p3);
-            const v8h B = pack8(p0, p1, p2, p3);
-            P[r] = __builtin_amdgcn_mfma_f32_32x32x16_f16(Ahi, B, P[r], 0, 0, 0);
-            P[r] = __builtin_amdgcn_mfma_f32_32x32x16_f16(Alo, B, P[r], 0, 0, 0);
+            for (int k = 0; k < 8; k++) f.d[k] = __builtin_amdgcn_raw_buffer_load_b16(rd, vd + 2 * k, 0, 0);
+            f.live = live;
         }
     }
-    const v8h Mhi = lds8(cur + XH_A + (size_t)lane * 16), Mlo = lds8(cur + XH_A + 1024 + (size_t)lane * 16);
+    // the quants of K-steps [4v, 4v + 4) (Q4_K, Q5_K, Q8_0) or, for even v, [4v, 4v + 8) (Q6_K)
+    __device__ __forceinline__ void quants(WFrag<FM>& f, int v) const {
+        if constexpr (FM == 1 || FM == 4) f.qv[v] = buf4(r, vo + (v >> 1) * 1024 + 512 * (v & 1));
+        if constexpr (FM == 2) {
+            if ((v & 1) == 0) {
+                f.qa[v >> 1] = buf4(r, vo + 512 * (v >> 1));
+                f.qb[v >> 1] = buf4(r, vo + 1024 + 512 * (v >> 1));
+                f.qh[v >> 1] = buf4(r, vo + 2048 + 512 * (v >> 1));
+            }
+        }
+        if constexpr (FM == 3) {
 #pragma unroll
-    for (int r = 0; r < RW; r++) {
-        Q[r] = __builtin_amdgcn_mfma_f32_32x32x16_f16(Mhi, Bm[r], Q[r], 0, 0, 0);
-        Q[r] = __builtin_amdgcn_mfma_f32_32x32x16_f16(Mlo, Bm[r], Q[r], 0, 0, 0);
-        const float dd = h2f((uint16_t)(f[r].h.x & 0xFFFF)), dm32 = -32.f * h2f((uint16_t)(f[r].h.x >> 16));
-#pragma unroll
-        for (int i = 0; i < 16; i++) part[r][i] = fmaf(dd, P[r][i], dm32 * Q[r][i]);
+            for (int k = 2 * v; k < 2 * v + 2; k++) f.q[k] = buf4(r, vo + 32 * k);
+        }
     }
-}
+};
 
-template <int RW>
-__device__ __forceinline__ void tiles_q6(const WFrag<2> (&f)[RW], const uint8_t* cur, int lane,
-                                         float (&part)[RW][16]) {
-    v16f P[RW], Q[RW];
+// A (row tile, super-block)'s contribution before the token scales, o[i] per C
+// element: hi / lo the wave's activation operands, mm its min-term operands
+// (LDS, hi then lo, 1 KB each), nx the tile that follows.  The next K-step's
+// weights are formed between this one's MFMAs (without the group barriers the
+// compiler puts them all before: 53.6 -> 49.0 us at T=256 16384x2048), and the
+// barrier per K-step keeps the live registers within two waves a SIMD.
+template <int FM>
+__device__ __forceinline__ void tile_mma(WFrag<FM>& f, const WPtr<FM>& nx, const v8h (&hi)[16], const v8h (&lo)[16],
+                                         const uint8_t* mm, int lane, float (&o)[16]) {
+    const uint32_t mk = magic_k(0x64006400u);
+    if constexpr (FM == 1 || FM == 4) {
+        const uint32_t mk5 = FM == 4 ? magic_k(0x50005000u) : 0u;
+        // 6-bit scales and mins (src/m5_kern_scalar.c:39-46), bytes of sub-blocks 0..3 and 4..7.
+        // Q4_K, low nibbles: (1024 + q) c - 1024 c; high nibbles stay in place: (1024 + 16 q) (c / 16) - 64 c.
+        // Q5_K: (32 + q) c - 48 c = (q - 16) c, with 16 sum_sb sc_sb S_sb beside the min term: centred, the
+        // weights' sum is not twice the size of what the min term leaves of it
+        const uint4 h = f.h;
+        uint4 qh = {};
+        if constexpr (FM == 4) qh = f.qh;
+        const uint32_t sb[2] = {h.y & 0x3F3F3F3Fu, (h.w & 0x0F0F0F0Fu) | ((h.y >> 2) & 0x30303030u)};
+        const uint32_t mb[2] = {h.z & 0x3F3F3F3Fu, ((h.w >> 4) & 0x0F0F0F0Fu) | ((h.z >> 2) & 0x30303030u)};
+        const float dd = h2f((uint16_t)(h.x & 0xFFFF)), dm = -32.f * h2f((uint16_t)(h.x >> 16));
+        v2h cl[2], ol[2], ch[2], oh[2];
 #pragma unroll
-    for (int r = 0; r < RW; r++) {
-        P[r] = (v16f){};
-        Q[r] = (v16f){};
-    }
+        for (int q = 0; q < 2; q++) {
+            v2h a, b;
+            pairs(sb[q], mk, a, b);
+            cl[q] = a - splat(1024.f);
+            b = b - splat(1024.f);
+            ch[q] = FM == 4 ? b : b * splat(0.0625f);
+            ol[q] = cl[q] * splat(FM == 4 ? -48.f : -1024.f);
+            oh[q] = b * splat(FM == 4 ? -48.f : -64.f);
+        }
+        nx.hdr(f);
+        auto bfrag = [&](int s) {  // the weights of K-step s
+            const int k = s >> 1, bh = s & 1, nib = k & 1;
+            const uint4 qv = f.qv[s >> 2];
+            const v2h cp = nib ? ch[k >> 2] : cl[k >> 2], op = nib ? oh[k >> 2] : ol[k >> 2];
+            const v2h c = (k & 2) ? (v2h){cp.y, cp.y} : (v2h){cp.x, cp.x};
+            const v2h of = (k & 2) ? (v2h){op.y, op.y} : (v2h){op.x, op.x};
+            uint32_t p[4];
 #pragma unroll
-    for (int s = 0; s < 16; s++) {
-        const int g2 = s >> 3, r6 = (s >> 1) & 3, bh = s & 1;
-        const v8h Ahi = lds8(cur + ((size_t)(2 * s) * 64 + lane) * 16);
-        const v8h Alo = lds8(cur + ((size_t)(2 * s + 1) * 64 + lane) * 16);
+            for (int q = 0; q < 2; q++) {
+                uint32_t w = q ? (bh ? qv.w : qv.y) : (bh ? qv.z : qv.x);
+                uint32_t a, b;
+                if constexpr (FM == 1) {
+                    w ^= 0x80808080u;  // stored XOR 0x80
+                    const uint32_t m = nib ? 0x00F000F0u : 0x000F000Fu;
+                    a = magic(w, m, mk);
+                    b = magic(w >> 8, m, mk);
+                } else {  // 32 + q: the nibble at bits 5..8, the fifth bit (value 32k + i: bit k of qh[i]) at bit 9
+                    const uint32_t H = q ? (bh ? qh.w : qh.y) : (bh ? qh.z : qh.x);
+                    a = magic(nib ? w << 1 : w << 5, 0x01E001E0u, mk5);
+                    b = magic(nib ? w >> 7 : w >> 3, 0x01E001E0u, mk5);
+                    a = magic(H << (9 - k), 0x02000200u, a);
+                    b = magic(k ? H >> (k - 1) : H << 1, 0x02000200u, b);
+                }
+                p[2 * q] = u2(__builtin_elementwise_fma(h2(a), c, of));
+                p[2 * q + 1] = u2(__builtin_elementwise_fma(h2(b), c, of));
+            }
+            return pack8(p[0], p[1], p[2], p[3]);
+        };
+        v16f P = {}, Q = {};
+        v8h B = bfrag(0), Bn = B;
 #pragma unroll
-        for (int r = 0; r < RW; r++) {
-            const uint4 A4 = f[r].qa[g2], B4 = f[r].qb[g2], H4 = f[r].qh[g2];
-            uint32_t wq[2];
+        for (int s = 0; s < 16; s++) {
+            __builtin_amdgcn_sched_barrier(0);
+            if (s < 15) Bn = bfrag(s + 1);
+            P = mfma16(hi[s], B, P);
+            Q = mfma16(lo[s], B, Q);
+            if ((s & 3) == 2) nx.quants(f, s >> 2);
+#pragma unroll
+            for (int g = 0; g < 2; g++) {
+                __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);  // one MFMA, then up to six VALU
+                __builtin_amdgcn_sched_group_barrier(0x2, 6, 0);
+            }
+            B = Bn;
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        const uint32_t keep = lane < 32 ? ~0u : 0u;  // min term: lanes (n, 1) hold zeros
+        uint32_t bm[4];
+#pragma unroll
+        for (int q = 0; q < 2; q++) {
+            v2h a, b;
+            pairs(mb[q], mk, a, b);
+            bm[2 * q] = u2(a - splat(1024.f)) & keep;
+            bm[2 * q + 1] = u2(b - splat(1024.f)) & keep;
+        }
+        const v8h Bm = pack8(bm[0], bm[1], bm[2], bm[3]);
+        const v8h mh = lds8(mm + lane * 16), ml = lds8(mm + 1024 + lane * 16);
+        const v16f M = mfma16(mh, Bm, mfma16(ml, Bm, (v16f){}));
+#pragma unroll
+        for (int i = 0; i < 16; i++) o[i] = fmaf(dd, P[i], dd * Q[i]);
+        if constexpr (FM == 4) {
+            const v8h Bs = pack8(u2(cl[0]) & keep, u2(ch[0]) & keep, u2(cl[1]) & keep, u2(ch[1]) & keep);
+            const v16f C = mfma16(mh, Bs, mfma16(ml, Bs, (v16f){}));
+            // the two large terms meet first
+#pragma unroll
+            for (int i = 0; i < 16; i++) o[i] += fmaf(dm, M[i], 512.f * dd * C[i]);
+        } else {
+#pragma unroll
+            for (int i = 0; i < 16; i++) o[i] = fmaf(dm, M[i], o[i]);
+        }
+    } else if constexpr (FM == 2) {
+        const float dd = h2f((uint16_t)f.d);
+        v2h c[2][2];
+#pragma unroll
+        for (int g = 0; g < 2; g++) {
+            pairs(f.sc4[g] ^ 0x80808080u, mk, c[g][0], c[g][1]);
+            c[g][0] = c[g][0] - splat(1152.f);
+            c[g][1] = c[g][1] - splat(1152.f);
+        }
+        nx.hdr(f);
+        auto bfrag = [&](int s, v8h& B, v8h& R) {  // rounding and rest of K-step s
+            const int g = s >> 3, r6 = (s >> 1) & 3, bh = s & 1;
+            const v2h cp = c[g][r6 & 1], cc = (r6 & 2) ? (v2h){cp.y, cp.y} : (v2h){cp.x, cp.x};
+            const uint4 A4 = f.qa[g], B4 = f.qb[g], H4 = f.qh[g];
+            uint32_t b[4], r[4];
 #pragma unroll
             for (int k = 0; k < 2; k++) {
-                const int qd = 2 * bh + k;  // dword of the 16-byte vectors
-                const uint32_t av = qd == 0 ? A4.x : (qd == 1 ? A4.y : (qd == 2 ? A4.z : A4.w));
-                const uint32_t bv = qd == 0 ? B4.x : (qd == 1 ? B4.y : (qd == 2 ? B4.z : B4.w));
-                const uint32_t hv = qd == 0 ? H4.x : (qd == 1 ? H4.y : (qd == 2 ? H4.z : H4.w));
+                const uint32_t av = bh ? (k ? A4.w : A4.z) : (k ? A4.y : A4.x);
+                const uint32_t bv = bh ? (k ? B4.w : B4.z) : (k ? B4.y : B4.x);
+                const uint32_t hv = bh ? (k ? H4.w : H4.z) : (k ? H4.y : H4.x);
                 // the GGUF 6-bit map of src/m5_kern_scalar.c:115-142 (as the GEMV's dot_q6)
-                if (r6 == 0) wq[k] = (av & 0x0F0F0F0Fu) | ((hv << 4) & 0x30303030u);
-                else if (r6 == 1) wq[k] = (bv & 0x0F0F0F0Fu) | ((hv << 2) & 0x30303030u);
-                else if (r6 == 2) wq[k] = ((av >> 4) & 0x0F0F0F0Fu) | (hv & 0x30303030u);
-                else wq[k] = ((bv >> 4) & 0x0F0F0F0Fu) | ((hv >> 2) & 0x30303030u);
-            }
-            const int scv = (int)(int8_t)(f[r].sc4[g2] >> (8 * r6));
-            const int shv = scv >> 3, slv = scv & 7;  // sc = 8*sh + sl
-            const _Float16 ch = (_Float16)shv, cl = (_Float16)slv;
-            const _Float16 oh = (_Float16)(-1056.f * (float)shv), ol = (_Float16)(-1056.f * (float)slv);
-            uint32_t p0, p1, p2, p3;
-            nib2h(wq[0], (v2h){ch, ch}, (v2h){oh, oh}, p0, p1);
-            nib2h(wq[1], (v2h){ch, ch}, (v2h){oh, oh}, p2, p3);
-            const v8h Bh = pack8(p0, p1, p2, p3);
-            nib2h(wq[0], (v2h){cl, cl}, (v2h){ol, ol}, p0, p1);
-            nib2h(wq[1], (v2h){cl, cl}, (v2h){ol, ol}, p2, p3);
-            const v8h Bl = pack8(p0, p1, p2, p3);
-            P[r] = __builtin_amdgcn_mfma_f32_32x32x16_f16(Ahi, Bh, P[r], 0, 0, 0);
-            P[r] = __builtin_amdgcn_mfma_f32_32x32x16_f16(Alo, Bh, P[r], 0, 0, 0);
-            Q[r] = __builtin_amdgcn_mfma_f32_32x32x16_f16(Ahi, Bl, Q[r], 0, 0, 0);
-            Q[r] = __builtin_amdgcn_mfma_f32_32x32x16_f16(Alo, Bl, Q[r], 0, 0, 0);
-        }
-    }
+                uint32_t w;
+                if (r6 == 0) w = (av & 0x0F0F0F0Fu) | ((hv << 4) & 0x30303030u);
+                else if (r6 == 1) w = (bv & 0x0F0F0F0Fu) | ((hv << 2) & 0x30303030u);
+                else if (r6 == 2) w = ((av >> 4) & 0x0F0F0F0Fu) | (hv & 0x30303030u);
+                else w = ((bv >> 4) & 0x0F0F0F0Fu) | ((hv >> 2) & 0x30303030u);
+                v2h q2[2];
+                pairs(w, mk, q2[0], q2[1]);
 #pragma unroll
-    for (int r = 0; r < RW; r++) {
-        const float dd = h2f((uint16_t)f[r].d);
-#pragma unroll
-        for (int i = 0; i < 16; i++) part[r][i] = dd * fmaf(8.f, P[r][i], Q[r][i]);
-    }
-}
-
-// FM 1 = Q4_K, 2 = Q6_K.  Grid (row blocks of 4*RW*32 rows, token tiles, K
-// splits).  The next super-block's weights are loaded into registers while
-// the current one is computed, as are its activations (then written to the
-// other LDS buffer).
-template <int FM, int RW>
-__global__ __launch_bounds__(256) void k_gemmh(const GemmHArgs a) {
-    extern __shared__ __align__(16) uint8_t sm[];  // [2][XH_SB]
-    const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int n = lane & 31, u = lane >> 5, j = n & 15;
-    const int tt = blockIdx.y, nb = a.n_in >> 8;
-    const int per = (nb + gridDim.z - 1) / gridDim.z;
-    const int b0 = blockIdx.z * per, b1 = min(nb, b0 + per);
-    const int rt0 = (4 * blockIdx.x + w) * RW;  // this wave's first 32-row tile
-    constexpr size_t IB = FM == 1 ? DRACO_Q4T_ITEM : DRACO_Q6T_ITEM;
-    const uint8_t* xsrc = a.xh + (size_t)tt * nb * XH_SB;
-    float y[RW][16];
-    const uint8_t* wrow[RW];  // item 0 of each row tile (tile index clamped in bounds)
-#pragma unroll
-    for (int r = 0; r < RW; r++) {
-#pragma unroll
-        for (int i = 0; i < 16; i++) y[r][i] = 0.f;
-        const int tile = min(2 * (rt0 + r) + (n >> 4), a.L.ntiles - 1);
-        wrow[r] = a.W + (size_t)tile * nb * IB;
-    }
-    if (b0 >= b1) return;  // uniform per block (empty K split)
-
-    WFrag<FM> wc[RW], wn[RW];
-#pragma unroll
-    for (int r = 0; r < RW; r++) wload(wrow[r] + (size_t)b0 * IB, j, u, wc[r]);
-    uint4 stg[9];
-    stage_load(xsrc + (size_t)b0 * XH_SB, stg, tid);
-    stage_store(sm, stg, tid);
-    __syncthreads();
-    for (int b = b0; b < b1; b++) {
-        const uint8_t* cur = sm + (size_t)((b - b0) & 1) * XH_SB;
-        uint8_t* nxt = sm + (size_t)((b - b0 + 1) & 1) * XH_SB;
-        const int bn = b + 1 < b1 ? b + 1 : b;  // the last step reloads its own (cached) data
-        stage_load(xsrc + (size_t)bn * XH_SB, stg, tid);
-#pragma unroll
-        for (int r = 0; r < RW; r++) wload(wrow[r] + (size_t)bn * IB, j, u, wn[r]);
-        float4 ts4[4];  // token scales of this lane's C rows 8q + 4u .. +3
-#pragma unroll
-        for (int q = 0; q < 4; q++) ts4[q] = *reinterpret_cast<const float4*>(cur + XH_A + XH_M + 4 * (8 * q + 4 * u));
-        if (32 * rt0 < a.L.n_out) {  // uniform per wave; no barrier inside.  Tiles past n_out
-                                     // (clamped loads) are computed and not stored.
-            float part[RW][16];
-            if constexpr (FM == 1) tiles_q4<RW>(wc, cur, lane, u, part);
-            else tiles_q6<RW>(wc, cur, lane, part);
-#pragma unroll
-            for (int r = 0; r < RW; r++)
-#pragma unroll
-                for (int i = 0; i < 16; i++) {
-                    const float4 t4 = ts4[i >> 2];
-                    const float tsc = (i & 3) == 0 ? t4.x : ((i & 3) == 1 ? t4.y : ((i & 3) == 2 ? t4.z : t4.w));
-                    y[r][i] = fmaf(tsc, part[r][i], y[r][i]);
+                for (int e = 0; e < 2; e++) {
+                    const v2h q = q2[e] - splat(1056.f), v = q * cc;
+                    b[2 * k + e] = u2(v);
+                    r[2 * k + e] = u2(__builtin_elementwise_fma(q, cc, -v));
                 }
+            }
+            B = pack8(b[0], b[1], b[2], b[3]);
+            R = pack8(r[0], r[1], r[2], r[3]);
+        };
+        v16f P = {}, Q = {};
+        v8h B, R, Bn, Rn;
+        bfrag(0, B, R);
+        Bn = B;
+        Rn = R;
+#pragma unroll
+        for (int s = 0; s < 16; s++) {
+            __builtin_amdgcn_sched_barrier(0);
+            if (s < 15) bfrag(s + 1, Bn, Rn);
+            P = mfma16(hi[s], B, P);
+            Q = mfma16(lo[s], B, Q);
+            Q = mfma16(hi[s], R, Q);
+            if ((s & 7) == 6) nx.quants(f, 2 * (s >> 3));
+#pragma unroll
+            for (int g = 0; g < 3; g++) {
+                __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x2, 8, 0);
+            }
+            B = Bn;
+            R = Rn;
         }
 #pragma unroll
-        for (int r = 0; r < RW; r++) wc[r] = wn[r];
-        if (b + 1 < b1) stage_store(nxt, stg, tid);
-        __syncthreads();
-    }
-    float* out = gridDim.z > 1 ? a.part + (size_t)blockIdx.z * a.T * a.ldy : a.Y;
+        for (int i = 0; i < 16; i++) o[i] = fmaf(dd, P[i], dd * Q[i]);
+    } else {
+        // K-steps 2k, 2k + 1 are the row's block k: its scale multiplies the
+        // block's dot (MFMAs from a zero accumulator), so d*q needs no
+        // rounding.  Blocks past the row's end read the next row's quants
+        // against activations that are zero, with a zero scale.
+        uint32_t dk[4];
+        const int lv = f.live;
 #pragma unroll
-    for (int r = 0; r < RW; r++) {
-        const int row = 32 * (rt0 + r) + n;
-        if (row >= a.L.n_out) continue;
+        for (int k = 0; k < 4; k++) dk[k] = f.d[2 * k] | (f.d[2 * k + 1] << 16);
 #pragma unroll
-        for (int i = 0; i < 16; i++) {
-            const int t = 32 * tt + 8 * (i >> 2) + 4 * u + (i & 3);
-            if (t < a.T) out[(size_t)t * a.ldy + row] = y[r][i];
+        for (int i = 0; i < 16; i++) o[i] = 0.f;
+#pragma unroll
+        for (int k = 0; k < 8; k++) {
+            __builtin_amdgcn_sched_barrier(0);
+            v16f S = {};
+            const uint4 q = f.q[k];
+#pragma unroll
+            for (int bh = 0; bh < 2; bh++) {
+                const int s = 2 * k + bh;
+                uint32_t p[4];
+#pragma unroll
+                for (int e = 0; e < 2; e++) {
+                    v2h a, b;  // bytes XOR 0x80 read 128 + q
+                    pairs((e ? (bh ? q.w : q.y) : (bh ? q.z : q.x)) ^ 0x80808080u, mk, a, b);
+                    p[2 * e] = u2(a - splat(1152.f));
+                    p[2 * e + 1] = u2(b - splat(1152.f));
+                }
+                const v8h B = pack8(p[0], p[1], p[2], p[3]);
+                S = mfma16(lo[s], B, S);
+                S = mfma16(hi[s], B, S);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            const float d = k < lv ? h2f((uint16_t)(dk[k >> 1] >> (16 * (k & 1)))) : 0.f;
+#pragma unroll
+            for (int i = 0; i < 16; i++) o[i] = fmaf(d, S[i], o[i]);
+            if (k & 1) nx.quants(f, k >> 1);
+            if (k == 3) nx.hdr(f);  // (not from the start: its 8 registers are not there)
         }
     }
 }
 
-// Y[t][row] = sum_z part[z][t][row] (z in order)
-__global__ __launch_bounds__(256) void k_gemmh_reduce(const float* __restrict__ part, float* __restrict__ Y, int T,
-                                                      int n_out, int ldy, int nz) {
-    const size_t n = (size_t)T * n_out;
-    for (size_t i = blockIdx.x * (size_t)256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256) {
-        const int t = (int)(i / n_out), row = (int)(i % n_out);
-        float s = 0.f;
-        for (int z = 0; z < nz; z++) s += part[((size_t)z * T + t) * ldy + row];
-        Y[(size_t)t * ldy + row] = s;
+constexpr int GR_NR = 2;  // row tiles (or gate / up pairs' halves) per reduction step
+
+// The steps of one block on one matrix (PAIR: on two of the same shape and
+// format, tile r of both, with the SwiGLU of the pair as the result).
+template <int FM, int NSB, bool PAIR>
+__device__ __forceinline__ void gemmr_body(const GemmHArgs& a, const GemmHSeg& sg, const uint8_t* W1, const uint8_t* W0,
+                                           int tt, int t_live, int r0, uint8_t* sm) {
+    constexpr int RS = 8 / NSB;
+    const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int n = lane & 31, u = lane >> 5;
+    const int slot = w % NSB, rs = w / NSB;
+    const DracoLayout& L = sg.L;
+    const int nb = (a.n_in + 255) >> 8, rts = (L.n_out + 31) >> 5;
+    const int tiles = min(a.rpb, (rts - r0 + RS - 1) / RS);  // row tiles of the longest stream
+    const int units = PAIR ? 2 * tiles : tiles;
+    float* red = reinterpret_cast<float*>(sm);                     // [2][8][GR_NR][1024]
+    uint8_t* mm = sm + 2 * 8 * GR_NR * 4096 + w * (2048 + 128);    // per wave: min operands, token scales
+    v8h hi[16], lo[16];
+    auto load_a = [&](int b) {
+        const __amdgpu_buffer_rsrc_t r = rsrc(a.xh + ((size_t)tt * nb + b) * XH_SB, XH_SB);
+        const v4u32 m0 = __builtin_amdgcn_raw_buffer_load_b128(r, lane * 16, XH_A, 0);
+        const v4u32 m1 = __builtin_amdgcn_raw_buffer_load_b128(r, lane * 16, XH_A + 1024, 0);
+        const uint32_t ts = __builtin_amdgcn_raw_buffer_load_b32(r, 4 * (lane & 31), XH_A + XH_M, 0);
+#pragma unroll
+        for (int s = 0; s < 16; s++) {
+            hi[s] = __builtin_bit_cast(v8h, __builtin_amdgcn_raw_buffer_load_b128(r, lane * 16, (2 * s) * 1024, 0));
+            lo[s] = __builtin_bit_cast(v8h, __builtin_amdgcn_raw_buffer_load_b128(r, lane * 16, (2 * s + 1) * 1024, 0));
+        }
+        *reinterpret_cast<v4u32*>(mm + lane * 16) = m0;
+        *reinterpret_cast<v4u32*>(mm + 1024 + lane * 16) = m1;
+        if (lane < 32) reinterpret_cast<uint32_t*>(mm + 2048)[lane] = ts;
+    };
+    const int passes = (nb + NSB - 1) / NSB;
+    const int vo = wlane<FM>(L, n, u);
+    // unit i of the block: row tile r0 + (i or i / 2) * RS + rs of matrix 0 (or 1 for the odd units of a pair)
+    auto ptr = [&](int i, int b) {
+        i = min(i, units - 1);
+        return WPtr<FM>(PAIR && (i & 1) ? W1 : W0, L, r0 + (PAIR ? i >> 1 : i) * RS + rs, min(b, nb - 1), vo, n, u);
+    };
+    load_a(min(slot, nb - 1));
+    WFrag<FM> f;
+    {
+        const WPtr<FM> q = ptr(0, slot);
+        q.hdr(f);
+#pragma unroll
+        for (int v = 0; v < 4; v++) q.quants(f, v);
+    }
+    for (int st = 0; st < units; st += GR_NR) {
+        float* rd = red + (size_t)((st / GR_NR) & 1) * 8 * GR_NR * 1024;
+        float* own = rd + (size_t)w * GR_NR * 1024 + lane;
+        const int nr = min(GR_NR, units - st);
+        for (int ps = 0; ps < passes; ps++) {
+            const int b = slot + ps * NSB;
+            if (b >= nb) {  // a slot past the row's end (uniform per wave)
+                if (ps == 0)
+                    for (int e = 0; e < 16 * nr; e++) own[e * 64] = 0.f;
+                continue;
+            }
+            if (passes > 1 && (st | ps)) load_a(b);
+            // the pass whose weights follow this one's (this slot's last pass may be short)
+            const int nps = ps + 1 < passes && b + NSB < nb ? ps + 1 : 0;
+            for (int r = 0; r < nr; r++) {
+                const WPtr<FM> nx = r + 1 < nr ? ptr(st + r + 1, b) : ptr(nps ? st : st + GR_NR, slot + nps * NSB);
+                float o[16];
+                tile_mma<FM>(f, nx, hi, lo, mm, lane, o);
+                float* y = own + r * 1024;
+                const float* ts = reinterpret_cast<const float*>(mm + 2048) + 4 * u;
+                if (ps) {  // uniform; a pass at a time, so that no sum is held across tiles
+#pragma unroll
+                    for (int i = 0; i < 16; i++) {
+                        const int e = 8 * (i >> 2) + (i & 3);
+                        y[i * 64] = fmaf(o[i], ts[e], y[i * 64]);
+                    }
+                } else {
+#pragma unroll
+                    for (int i = 0; i < 16; i++) y[i * 64] = o[i] * ts[8 * (i >> 2) + (i & 3)];
+                }
+            }
+        }
+        lds_barrier();
+        // the slots' sums, pairwise: stream rs's elements over its NSB waves
+        auto total = [&](int r, int i) {
+            float v[NSB];
+#pragma unroll
+            for (int k = 0; k < NSB; k++) v[k] = rd[(size_t)((rs * NSB + k) * GR_NR + r) * 1024 + i * 64 + lane];
+#pragma unroll
+            for (int h = NSB / 2; h; h >>= 1)
+#pragma unroll
+                for (int k = 0; k < h; k++) v[k] += v[k + h];
+            return v[0];
+        };
+        for (int e = slot; e < 16 * (PAIR ? 1 : nr); e += NSB) {
+            const int i = e & 15, r = e >> 4;
+            float s = total(r, i);
+            if (PAIR) s = (s / (1.f + expf(-s))) * total(1, i);
+            const int row = 32 * (r0 + (PAIR ? st >> 1 : st + r) * RS + rs) + n;
+            const int tl = 8 * (i >> 2) + 4 * u + (i & 3);
+            if (row < L.n_out && tl < t_live) sg.Y[(size_t)(32 * tt + tl) * sg.ldy + row] = s;
+        }
     }
 }
 
-template <int FM, int RW>
-void launch_h(const GemmHArgs& a, dim3 grid, hipStream_t st) {
+// XCD x runs blocks x, x + 8, ...: an XCD's consecutive blocks are the token
+// tiles of one row group, so a group's weights come from HBM once per XCD.
+// F0 / F1: the formats that the launch's matrices have.
+template <int F0, int F1, int NSB, bool PAIR>
+__global__ __launch_bounds__(512) void k_gemmr(const GemmHArgs a) {
+    extern __shared__ __align__(16) uint8_t sm[];
+    const int ntt = a.groups ? a.max_tiles : (a.T + 31) >> 5;
+    const int loc = blockIdx.x >> 3;
+    int tt = loc % ntt, rg = (loc / ntt) * 8 + (blockIdx.x & 7);
+    if (rg >= a.n_rg) return;
+    const int s = a.nseg > 1 && rg >= a.seg[1].rg0 ? (a.nseg > 2 && rg >= a.seg[2].rg0 ? 2 : 1) : 0;
+    const GemmHSeg& sg = a.seg[s];
+    const uint8_t *W0 = sg.W, *W1 = PAIR ? a.seg[1].W : nullptr;
+    int live = a.T - 32 * tt;
+    if (a.groups) {  // token tile tt belongs to one expert (negative: past the last tile)
+        const int e = a.groups[tt];
+        if (e < 0) return;
+        W0 = sg.bases[e];
+        if (PAIR) W1 = a.seg[1].bases[e];
+        live = 32;
+    }
+    const int r0 = (rg - sg.rg0) * a.rpb * (8 / NSB);
+    if (F0 == F1 || sg.fm == F0) gemmr_body<F0, NSB, PAIR>(a, sg, W1, W0, tt, live, r0, sm);
+    else gemmr_body<F1, NSB, PAIR>(a, sg, W1, W0, tt, live, r0, sm);
+}
+
+constexpr size_t GR_LDS = 2 * 8 * GR_NR * 4096 + 8 * (2048 + 128);
+
+int fm_of(int code) {
+    switch (code) {
+    case DRACO_Q4_K: return 1;
+    case DRACO_Q6_K: return 2;
+    case DRACO_Q8_0: return 3;
+    case DRACO_Q5_K: return 4;
+    default: return 0;
+    }
+}
+
+template <int F0, int F1, int NSB, bool PAIR>
+void launch_r(const GemmHArgs& a, unsigned grid, hipStream_t st) {
     static bool attr = false;
     if (!attr) {
-        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&k_gemmh<FM, RW>),
-                                  hipFuncAttributeMaxDynamicSharedMemorySize, 2 * XH_SB);
+        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&k_gemmr<F0, F1, NSB, PAIR>),
+                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)GR_LDS);
         attr = true;
     }
-    hipLaunchKernelGGL((k_gemmh<FM, RW>), grid, dim3(256), 2 * XH_SB, st, a);
+    hipLaunchKernelGGL((k_gemmr<F0, F1, NSB, PAIR>), dim3(grid), dim3(512), GR_LDS, st, a);
+}
+
+template <int NSB>
+int pick(const GemmHArgs& a, int f0, int f1, unsigned grid, hipStream_t st) {
+    if (a.pair) {
+        switch (f0) {
+        case 1: launch_r<1, 1, NSB, true>(a, grid, st); return 0;
+        case 2: launch_r<2, 2, NSB, true>(a, grid, st); return 0;
+        case 3: launch_r<3, 3, NSB, true>(a, grid, st); return 0;
+        default: launch_r<4, 4, NSB, true>(a, grid, st); return 0;
+        }
+    }
+    if (f0 == f1) {
+        switch (f0) {
+        case 1: launch_r<1, 1, NSB, false>(a, grid, st); return 0;
+        case 2: launch_r<2, 2, NSB, false>(a, grid, st); return 0;
+        case 3: launch_r<3, 3, NSB, false>(a, grid, st); return 0;
+        default: launch_r<4, 4, NSB, false>(a, grid, st); return 0;
+        }
+    }
+    if (f0 == 1) launch_r<1, 2, NSB, false>(a, grid, st);
+    else launch_r<4, 2, NSB, false>(a, grid, st);
+    return 0;
 }
 
 }  // namespace
 
-size_t draco_gemmh_x_bytes(int T, int n_in) { return (size_t)((T + 31) / 32) * (n_in / 256) * XH_SB + 256; }
+size_t draco_gemmh_x_bytes(int T, int n_in) { return (size_t)((T + 31) / 32) * ((n_in + 255) / 256) * XH_SB + 256; }
 
-int draco_gemmh_x_launch(const float* X, int T, int n_in, uint8_t* buf, hipStream_t st) {
-    if (T < 1 || n_in % 256) return -1;
-    hipLaunchKernelGGL(k_gemmh_x, dim3(n_in / 256, (T + 31) / 32), dim3(256), 0, st, X, T, n_in, buf);
+bool draco_gemmh_serves(int code) { return fm_of(code) != 0; }
+
+// The formats one launch can mix: Q4_K or Q5_K with Q6_K (a Q4_K_M / Q5_K_M layer's q, k and v).
+bool draco_gemmh_mixes(int c0, int c1) {
+    return c0 == c1 || ((c0 == DRACO_Q4_K || c0 == DRACO_Q5_K) && c1 == DRACO_Q6_K) ||
+           ((c1 == DRACO_Q4_K || c1 == DRACO_Q5_K) && c0 == DRACO_Q6_K);
+}
+
+int draco_gemmh_x_launch(const float* X, int T, int n_in, uint8_t* buf, hipStream_t st, const int* rows) {
+    if (T < 1 || n_in < 32 || n_in % 32) return -1;
+    hipLaunchKernelGGL(k_gemmh_x, dim3((n_in + 255) / 256, (T + 31) / 32), dim3(256), 0, st, X, T, n_in, rows, buf);
     return 0;
 }
 
-// Row blocks of 256 rows (two tiles per wave, sharing each A read) for
-// products of at least 64 row tiles over at least 4 token tiles, else 128
-// rows; K split so that about 256 blocks run, each over at least 2
-// super-blocks.  Measured on the configs[2] chunk (256 tokens): q / o 17.0 ->
-// 15.4 us, down 55.5 -> 51 us with two tiles per wave; k / v (16 row tiles)
-// slower with them, and so was the configs[4] prefill's 64-token chunk
-// (9610 -> 9385 tok/s).  part: kspl * T * ldy floats (draco_gemmh_part_floats).
-static void plan(const DracoLayout& L, int T, int& rw, int& kspl) {
-    const int nb = L.n_in / 256, tiles32 = (L.n_out + 31) / 32, ntt = (T + 31) / 32;
-    rw = tiles32 >= 64 && ntt >= 4 ? 2 : 1;
-    const int blocks = ((tiles32 + 4 * rw - 1) / (4 * rw)) * ntt;
-    kspl = 1;
-    while (blocks * kspl * 2 <= 256 && nb / (kspl * 2) >= 2) kspl *= 2;
-}
-
-size_t draco_gemmh_part_floats(const DracoLayout& L, int T, int ldy) {
-    int rw, kspl;
-    plan(L, T, rw, kspl);
-    return kspl > 1 ? (size_t)kspl * T * ldy : 0;
-}
-
+// Row tiles per block: as few as leave at most one block per CU (256).
+// Measured at T=256: 2048x2048 256 blocks 8.8 us, 512
+// 11.5; 12288 rows at T=64 11.6 / 15.9.  Four super-block slots (two row
+// streams) where rows have at most four super-blocks and there are row tiles
+// enough for both streams (960-wide rows of 30 tiles: 6.4 us with eight slots,
+// half of them idle, 8.0 with four).
 int draco_gemmh_launch(GemmHArgs& a, hipStream_t st) {
-    if (a.L.code != DRACO_Q4_K && a.L.code != DRACO_Q6_K) return -1;
-    if (a.n_in != a.L.n_in || a.T < 1 || a.n_in % 256) return -1;
-    int rw, kspl;
-    plan(a.L, a.T, rw, kspl);
-    if (kspl > 1 && !a.part) return -1;
-    const int tiles32 = (a.L.n_out + 31) / 32;
-    const dim3 grid((tiles32 + 4 * rw - 1) / (4 * rw), (a.T + 31) / 32, kspl);
-    if (a.L.code == DRACO_Q4_K) {
-        if (rw == 2) launch_h<1, 2>(a, grid, st);
-        else launch_h<1, 1>(a, grid, st);
-    } else {
-        if (rw == 2) launch_h<2, 2>(a, grid, st);
-        else launch_h<2, 1>(a, grid, st);
+    if (a.nseg < 1 || a.nseg > 3 || a.T < 1 || a.n_in < 32 || a.n_in % 32 || !a.xh) return -1;
+    if (a.groups && (a.max_tiles < 1 || a.nseg != (a.pair ? 2 : 1))) return -1;
+    int f0 = 0, f1 = 0;
+    for (int s = 0; s < a.nseg; s++) {
+        GemmHSeg& g = a.seg[s];
+        g.fm = fm_of(g.L.code);
+        if (!g.fm || g.L.n_in != a.n_in || (a.groups ? !g.bases : !g.W) || (!g.Y && !(a.pair && s))) return -1;
+        if (s && !draco_gemmh_mixes(a.seg[0].L.code, g.L.code)) return -1;
+        // F0 is the Q4_K / Q5_K one of a mix
+        if (s == 0) f0 = f1 = g.fm;
+        else if (g.fm != f0 && g.fm != f1) (g.fm == 2 ? f1 : f0) = g.fm;
     }
-    if (kspl > 1) {
-        const size_t n = (size_t)a.T * a.L.n_out;
-        const unsigned blocks = (unsigned)std::min<size_t>((n + 255) / 256, 4096);
-        hipLaunchKernelGGL(k_gemmh_reduce, dim3(blocks), dim3(256), 0, st, a.part, a.Y, a.T, a.L.n_out, a.ldy, kspl);
+    if (a.pair && (a.nseg != 2 || f0 != f1 || a.seg[0].L.n_out != a.seg[1].L.n_out)) return -1;
+    const int ntt = a.groups ? a.max_tiles : (a.T + 31) / 32, nb = (a.n_in + 255) / 256;
+    const int walk = a.pair ? 1 : a.nseg;  // matrices whose rows the blocks walk
+    int rts = 0;
+    for (int s = 0; s < walk; s++) rts += (a.seg[s].L.n_out + 31) / 32;
+    const int NSB = nb <= 4 && rts * ntt >= 1024 ? 4 : 8, RS = 8 / NSB;
+    int rpb = 1;
+    auto groups_of = [&](int s) { return ((a.seg[s].L.n_out + 31) / 32 + rpb * RS - 1) / (rpb * RS); };
+    for (;; rpb++) {
+        int rg = 0;
+        for (int s = 0; s < walk; s++) rg += groups_of(s);
+        if ((long long)rg * ntt <= 256 || rpb >= rts) break;
     }
-    return 0;
+    a.rpb = rpb;
+    a.n_rg = 0;
+    for (int s = 0; s < walk; s++) {
+        a.seg[s].rg0 = a.n_rg;
+        a.n_rg += groups_of(s);
+    }
+    if (a.pair) a.nseg = 1;  // (the second matrix is read through its base)
+    const unsigned grid = (unsigned)((a.n_rg + 7) / 8 * 8 * ntt);
+    return NSB == 4 ? pick<4>(a, f0, f1, grid, st) : pick<8>(a, f0, f1, grid, st);
 }

@@ -84,3 +84,54 @@ def test_fused_entries_not_carried_leave_nan(hip, fname):
     getattr(hip, f"m5_gemm_{fname}")(lib.pf(X), lib.pu8(W), 2, 4, 256, lib.pf(Y))
     assert np.isnan(Y).all()
 
+
+
+@pytest.mark.parametrize("T,n_out,n_in", [(1, 1, 32), (2, 33, 288), (31, 960, 960), (33, 17, 1056), (64, 320, 2528),
+                                          (5, 16, 2080), (65, 2560, 736), (32, 31, 4064)])
+def test_gemm_q8_ragged_rows_vs_oracle(hip, oracle, T, n_out, n_in):
+    """Q8_0 rows that end inside a 256-value super-block (the last one padded
+    with zero activations and zero scales), row counts off the 32-row tile.
+    Bound: 1e-5 of the row dots' scale sum|w||x| (one-row and one-block
+    products cancel)."""
+    from dracohip import lib
+    W, X = _case(0, T, n_out, n_in, T + n_out + n_in)
+    Y = np.full((T, n_out), np.nan, np.float32)
+    hip.m5_gemm_q80(lib.pf(X), lib.pu8(W), T, n_out, n_in, lib.pf(Y))
+    ref = np.zeros_like(Y)
+    assert oracle.lib.or_gemm(0, lib.pf(X), lib.pu8(W), T, n_out, n_in, lib.pf(ref)) == 0
+    blk = W.reshape(n_out, n_in // 32, 34)
+    w = np.abs(blk[:, :, 2:].view(np.int8).astype(np.float64)) * np.abs(blk[:, :, :2].copy().view(np.float16).astype(np.float64))
+    scale = np.abs(X.astype(np.float64)) @ w.reshape(n_out, n_in).T
+    assert np.all(np.abs(Y.astype(np.float64) - ref) <= 1e-5 * scale + 1e-30)
+
+
+def test_gemm_q8_nonfinite_tokens_stay_apart(hip, oracle):
+    """An infinite or NaN activation makes its own token non-finite where the
+    reference's fp32 dots are, and leaves every other token as it was."""
+    from dracohip import lib
+    T, n_out, n_in = 40, 70, 960
+    W, X = _case(0, T, n_out, n_in, 9)
+    X[3, 500], X[3, 17], X[36, 959] = np.inf, -np.inf, np.nan
+    X[7, 11] = -np.inf
+    Y = np.zeros((T, n_out), np.float32)
+    hip.m5_gemm_q80(lib.pf(X), lib.pu8(W), T, n_out, n_in, lib.pf(Y))
+    ref = np.zeros_like(Y)
+    assert oracle.lib.or_gemm(0, lib.pf(X), lib.pu8(W), T, n_out, n_in, lib.pf(ref)) == 0
+    assert np.array_equal(np.isnan(Y), np.isnan(ref))
+    assert np.array_equal(Y[np.isinf(ref)], ref[np.isinf(ref)])
+    ok = np.isfinite(ref)
+    assert ok.sum() >= (T - 3) * n_out and rel_err(Y[ok], ref[ok]) <= TOL
+
+
+@pytest.mark.parametrize("code", [5, 4, 0, 3])
+@pytest.mark.parametrize("T,n_out,n_in", [(33, 16, 256), (65, 100, 1024), (1, 33, 2304), (256, 4112, 1024)])
+def test_gemm_slots_and_streams_vs_oracle(hip, oracle, code, T, n_out, n_in):
+    """One, four and nine super-blocks a row (idle slots, a short second pass)
+    and the two-stream form (short rows, many row tiles, an odd last tile)."""
+    from dracohip import lib
+    W, X = _case(code, T, n_out, n_in, 3 * T + n_out + code)
+    Y = np.full((T, n_out), np.nan, np.float32)
+    assert hip.m5_gemm_auto(code, lib.pf(X), lib.pu8(W), T, n_out, n_in, lib.pf(Y)) == 0
+    ref = np.zeros_like(Y)
+    assert oracle.lib.or_gemm(code, lib.pf(X), lib.pu8(W), T, n_out, n_in, lib.pf(ref)) == 0
+    assert rel_err(Y, ref) <= TOL
