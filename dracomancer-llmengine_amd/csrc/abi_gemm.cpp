@@ -3,8 +3,7 @@
 // m5_gemm_auto: src/m5/m5_gemm_fused.c:231-241 (0 = done, -1 = code not served,
 // the caller falls back); m5_gemm: src/m5/m5_gemm.c:249-272 (Y[T x n_out] =
 // X[T x n_in] . W^T).  Host pointers.  Q4_K, Q5_K, Q6_K and Q8_0 run on the
-// f16-MFMA GEMM (gemmh.hip).  The int8-MFMA kernels
-// of gemm.hip serve the grouped expert GEMMs of m6_moe_tok only.
+// f16-MFMA GEMM (gemmh.hip).
 // m5_dequant_row: src/m5/m5_gemm.c:55-235, the GEMM library's row decoder.
 #include <stdio.h>
 #include <string.h>
@@ -93,7 +92,7 @@ int gemm_host(int code, const float* X, const uint8_t* W, int T, int n_out, int 
     hipStream_t st = stream();
     float* dx = (float*)scratch(0, sizeof(float) * (size_t)T * n_in);
     float* dy = (float*)scratch(1, sizeof(float) * (size_t)T * n_out);
-    uint8_t* dd = (uint8_t*)scratch(7, draco_gemm_digit_bytes(T, n_in));
+    uint8_t* dd = (uint8_t*)scratch(7, draco_gemmh_x_bytes(T, n_in));
     if (!dx || !dy || !dd) return -2;
     DRACO_HIP(hipMemcpyAsync(dx, X, sizeof(float) * (size_t)T * n_in, hipMemcpyHostToDevice, st));
     if (int rc = enqueue_gemm(*m, dx, T, dy, dd, st)) return rc;
@@ -224,7 +223,7 @@ int draco_bench_gemm(int code, const uint8_t* W, int n_out, int n_in, int T, int
     uint8_t* dd;
     DRACO_HIP(hipMalloc(&dx, sizeof(float) * xh.size()));
     DRACO_HIP(hipMalloc(&dy, sizeof(float) * (size_t)T * n_out));
-    DRACO_HIP(hipMalloc(&dd, draco_gemm_digit_bytes(T, n_in)));
+    DRACO_HIP(hipMalloc(&dd, draco_gemmh_x_bytes(T, n_in)));
     DRACO_HIP(hipMemcpy(dx, xh.data(), sizeof(float) * xh.size(), hipMemcpyHostToDevice));
     hipStream_t st = stream();
     // one eager product first: it writes the activation operands

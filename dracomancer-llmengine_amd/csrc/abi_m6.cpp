@@ -775,19 +775,14 @@ int enqueue_layer(DevModel* m, int l, float eps, hipStream_t st, const float* xi
     return 0;
 }
 
-bool has_moe(const DevModel* m) {
-    for (const MoeLayer* p : m->moe)
-        if (p) return true;
-    return false;
-}
-
 // Whether the model's tokens can go through the batched (chunked) prefill:
-// dense FFNs and attention shapes its kernel serves; other models feed
-// their prompts through token-serial decode steps.
+// attention shapes its kernel serves and FFNs that run over token rows; other
+// models feed their prompts through token-serial decode steps.
 bool chunk_ok(const DevModel* m) {
-    if (has_moe(m)) return false;
-    for (int l = 0; l < m->n_layer; l++)
+    for (int l = 0; l < m->n_layer; l++) {
         if (!pf_attention_ok(m->attn[l]->NH, m->attn[l]->NKV, m->attn[l]->HD)) return false;
+        if (m->moe[l] && !draco_moe_layer_rows_ok(m->moe[l])) return false;
+    }
     return true;
 }
 
@@ -798,7 +793,7 @@ int g_prefill_chunk = 256;  // tokens per chunk; 0 = token-serial prefill
 
 int ensure_pf(DevModel* m, int cap) {
     PfBufs& b = m->pf;
-    int QD = 0, KD = 0, FF = 0, NH = 0, HD = 0, max_t = 0;
+    int QD = 0, KD = 0, FF = 1, NH = 0, HD = 0, max_t = 0;
     for (int l = 0; l < m->n_layer; l++) {
         const DevAttn* a = m->attn[l];
         QD = std::max(QD, a->NH * a->HD);
@@ -810,7 +805,7 @@ int ensure_pf(DevModel* m, int cap) {
     }
     const size_t part_n = pf_part_floats(NH, cap, HD, pf_attn_nsplit(max_t, cap));
     const int win = std::max(std::max(m->h, QD), FF);
-    const size_t dig_n = draco_gemm_digit_bytes(cap, ((win + 255) / 256) * 256);
+    const size_t dig_n = draco_gemmh_x_bytes(cap, ((win + 255) / 256) * 256);
     if (b.cap >= cap && b.H == m->h && b.QD >= QD && b.KD >= KD && b.FF >= FF && b.part_n >= part_n && b.dig_n >= dig_n)
         return 0;
     DRACO_HIP(hipStreamSynchronize(stream()));
@@ -864,11 +859,16 @@ int enqueue_prefill_layer(DevModel* m, int l, int T, int pos0, int row0, float e
         return fail(-1, "prefill: rope rejected");
     if (pf_attention(b.Q, a->kc, a->vc, b.part, b.O, row0, T, a->NH, a->NKV, a->HD, a->scale, st))
         return fail(-1, "prefill: attention shape NH=%d NKV=%d HD=%d not served", a->NH, a->NKV, a->HD);
-    const GemmTo o = {a->wo, b.Y}, dn = {f->d, b.Y};
+    const GemmTo o = {a->wo, b.Y};
     if (draco_enqueue_gemms(&o, 1, b.O, T, b.dig, st)) return -1;
     if (pf_add_rms(b.X, b.Y, m->fnorm[l], b.Xn, T, H, eps, st)) return fail(-1, "prefill: rms rejected");
-    if (draco_enqueue_swiglu(*f->g, *f->u, b.Xn, T, b.G, b.U, b.dig, st)) return -1;
-    if (draco_enqueue_gemms(&dn, 1, b.G, T, b.dig, st)) return -1;
+    if (m->moe[l]) {
+        if (int rc = draco_moe_layer_rows(m->moe[l], b.Xn, T, b.Y, st)) return rc;
+    } else {
+        const GemmTo dn = {f->d, b.Y};
+        if (draco_enqueue_swiglu(*f->g, *f->u, b.Xn, T, b.G, b.U, b.dig, st)) return -1;
+        if (draco_enqueue_gemms(&dn, 1, b.G, T, b.dig, st)) return -1;
+    }
     // the residual; fused with the next layer's input RMSNorm when there is one
     if (l + 1 < m->n_layer) {
         if (pf_add_rms(b.X, b.Y, m->anorm[l + 1], b.Xn, T, H, eps, st)) return fail(-1, "prefill: rms rejected");
@@ -884,7 +884,7 @@ int enqueue_prefill_layer(DevModel* m, int l, int T, int pos0, int row0, float e
 // is left in pf.X row (last chunk's T - 1); returns that T (0 on error).
 int enqueue_prefill(DevModel* m, const DracoMat* em, const int* ids, int n, int pos0, float eps, hipStream_t st) {
     if (!chunk_ok(m)) {
-        fail(-1, "chunked prefill: MoE layers and attention shapes outside the batched kernel go token by token");
+        fail(-1, "chunked prefill: this model's layers go token by token");
         return 0;
     }
     const int C = g_prefill_chunk;
@@ -1301,8 +1301,7 @@ int draco_llama_generate(const void* layers_v, int n_layer, int h, float eps, co
     // prompt[0 .. n_prompt - 1) goes through the chunked prefill when enabled
     // (the last prompt token goes through the first decode step, which also
     // runs the head); the token cursor then starts past those tokens
-    // (MoE models and attention shapes outside the batched prefill kernel
-    // feed the prompt through token-serial decode steps)
+    // (models outside chunk_ok feed the prompt through token-serial decode steps)
     const int n_chunked = (g_prefill_chunk > 0 && n_prompt - 1 >= 2 && chunk_ok(m)) ? n_prompt - 1 : 0;
     if (n_chunked && ensure_pf(m, g_prefill_chunk)) return report(-2, "draco_llama_generate (prefill buffers)");
     ht[ntok + 8] = n_chunked;

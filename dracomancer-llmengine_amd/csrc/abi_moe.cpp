@@ -8,6 +8,7 @@
 #include <stdio.h>
 #include <string.h>
 
+#include <algorithm>
 #include <map>
 #include <vector>
 
@@ -229,26 +230,83 @@ int gemvn(int code, const float* x, long x_stride, const uint8_t* W, const int* 
 }
 
 // ---- token-batched MoE (prefill), src/m6_moe_tok.c:44-161 -----------------
+
+// 32-row tiles that T tokens of n_used experts each can fill at most: every
+// expert's last tile may be short
+int tiles_max(int T, int n_used, int n_exp) {
+    const long long n = (long long)T * n_used;
+    return (int)std::min<long long>(n, n / 32 + n_exp);
+}
+
+// Y[t] = sum over k (in k order) of wt[t][k] * expert order[t][k] applied to
+// X[t] (device pointers; gate/up -> silu*up -> down).  bases: device table
+// [3][n_exp] of gate, up and down; a role's experts share one format.  Every
+// product is one grouped launch over the experts' tiles.
+int moe_rows(const float* X, const int* order, const float* wt, const uint8_t* const* bases, int cg, int cu, int cd,
+             int T, int n_used, int n_exp, int inter, int n_in, int n_out, int max_tiles, float* Y, hipStream_t st) {
+    const size_t R = 32 * (size_t)max_tiles;
+    DracoLayout Lg, Lu, Ld;
+    if (draco_layout(cg, inter, n_in, &Lg) || draco_layout(cu, inter, n_in, &Lu) || draco_layout(cd, n_out, inter, &Ld))
+        return fail(-1, "moe tokens: no layout");
+    int* rows = (int*)scratch(9, sizeof(int) * (R + (size_t)max_tiles + (size_t)T * n_used));
+    float* dG = (float*)scratch(10, sizeof(float) * R * inter);
+    float* dU = cg == cu ? nullptr : (float*)scratch(11, sizeof(float) * R * inter);
+    float* dY = (float*)scratch(12, sizeof(float) * R * n_out);
+    uint8_t* xh = (uint8_t*)scratch(14, draco_gemmh_x_bytes((int)R, n_in > inter ? n_in : inter));
+    if (!rows || !dG || (cg != cu && !dU) || !dY || !xh) return -2;
+    int* tile_exp = rows + R;
+    int* pos = tile_exp + max_tiles;
+    if (draco_moe_plan_launch(order, T, n_used, n_exp, max_tiles, tile_exp, rows, pos, st))
+        return fail(-1, "moe tokens: grouping rejected");
+    GemmHArgs base = {};
+    base.T = (int)R;
+    base.xh = xh;
+    base.groups = tile_exp;
+    base.max_tiles = max_tiles;
+    if (draco_gemmh_x_launch(X, (int)R, n_in, xh, st, rows)) return fail(-1, "moe tokens: activations rejected");
+    GemmHArgs a = base;
+    a.n_in = n_in;
+    a.seg[0] = {nullptr, bases, Lg, dG, inter, 0, 0};
+    if (cg == cu) {
+        a.seg[1] = {nullptr, bases + n_exp, Lu, nullptr, inter, 0, 0};
+        a.nseg = 2;
+        a.pair = 1;
+        if (draco_gemmh_launch(a, st)) return fail(-1, "moe tokens: gate/up rejected");
+    } else {
+        a.nseg = 1;
+        if (draco_gemmh_launch(a, st)) return fail(-1, "moe tokens: gate rejected");
+        a = base;
+        a.n_in = n_in;
+        a.nseg = 1;
+        a.seg[0] = {nullptr, bases + n_exp, Lu, dU, inter, 0, 0};
+        if (draco_gemmh_launch(a, st)) return fail(-1, "moe tokens: up rejected");
+        dk_swiglu(dG, dU, (int)(R * inter), st);
+    }
+    // (a tile's padding rows hold zeros: silu(0) * 0)
+    if (draco_gemmh_x_launch(dG, (int)R, inter, xh, st)) return fail(-1, "moe tokens: activations rejected");
+    a = base;
+    a.n_in = inter;
+    a.nseg = 1;
+    a.seg[0] = {nullptr, bases + 2 * (size_t)n_exp, Ld, dY, n_out, 0, 0};
+    if (draco_gemmh_launch(a, st)) return fail(-1, "moe tokens: down rejected");
+    if (draco_moe_scatter_launch(dY, n_out, pos, wt, n_used, T, Y, st)) return fail(-1, "moe tokens: combine rejected");
+    return 0;
+}
+
 int moe_tok(const float* X, const int* order, const float* wtop, const uint64_t* ep, const int* ec, int T,
             int n_used, int inter, int n_in, int n_out, int n_exp, float* out) {
     if (T < 1 || n_used < 1 || n_exp < 1 || n_exp > MOE_EXP_MAX)
         return fail(-1, "m6_moe_tok: T %d n_used %d n_exp %d not served", T, n_used, n_exp);
     if (inter % 256 || n_in % 256 || n_out % 16)
         return fail(-1, "m6_moe_tok: shape inter %d n_in %d n_out %d not served", inter, n_in, n_out);
-    // expert grouping (the reference's off/ilist/slot, segments padded to 8 tokens)
+    const size_t n = (size_t)T * n_used;
     std::vector<int> cnt(n_exp, 0);
-    for (int i = 0; i < T * n_used; i++)
+    for (size_t i = 0; i < n; i++)
         if (order[i] >= 0 && order[i] < n_exp) cnt[order[i]]++;
-    std::vector<int> oct0(n_exp, 0), active;
-    int n_oct = 0, max_oct = 0;
-    int cg = -1, cu = -1, cd = -1;
+    int tiles = 0, cg = -1, cu = -1, cd = -1;
     for (int e = 0; e < n_exp; e++) {
         if (!cnt[e]) continue;
-        active.push_back(e);
-        oct0[e] = n_oct;
-        const int o = (cnt[e] + 7) / 8;
-        n_oct += o;
-        max_oct = o > max_oct ? o : max_oct;
+        tiles += (cnt[e] + 31) / 32;
         if (cg < 0) {
             cg = ec[3 * e];
             cu = ec[3 * e + 1];
@@ -257,107 +315,43 @@ int moe_tok(const float* X, const int* order, const float* wtop, const uint64_t*
         if (ec[3 * e] != cg || ec[3 * e + 1] != cu || ec[3 * e + 2] != cd)
             return fail(-1, "m6_moe_tok: mixed expert formats");
     }
-    if (active.empty()) {
+    if (!tiles) {
         memset(out, 0, sizeof(float) * (size_t)T * n_out);
         return 0;
     }
-    // gate and up may differ in format: the up product reuses the gate's
-    // activation digits, which do not depend on the weight format
+    // gate and up may differ in format: they are two launches then
     if (!fm_of(cg) || !fm_of(cu) || !fm_of(cd))
         return fail(-1, "m6_moe_tok: expert formats %d/%d/%d not served", cg, cu, cd);
-    const int R = 8 * n_oct;
-    std::vector<int> src(R, -1), pos((size_t)T * n_used, -1), fill(n_exp, 0);
-    for (int i = 0; i < T * n_used; i++) {
-        const int e = order[i];
-        if (e < 0 || e >= n_exp) continue;
-        const int row = 8 * oct0[e] + fill[e]++;
-        src[row] = i / n_used;
-        pos[i] = row;
-    }
     if (int rc = ensure_init()) return rc;
     hipStream_t st = stream();
-    const int na = (int)active.size();
-    std::vector<GemmGroup> gg(na), gu(na), gd(na);
-    for (int k = 0; k < na; k++) {
-        const int e = active[k];
+    // one upload of the tables: the experts' bases, the pairs' experts and weights
+    const size_t tb = sizeof(void*) * 3 * (size_t)n_exp, all = tb + (sizeof(int) + sizeof(float)) * n;
+    char* h = (char*)pinned(7, all);
+    char* d = (char*)scratch(15, all);
+    float* dX = (float*)scratch(8, sizeof(float) * (size_t)T * n_in);
+    float* dO = (float*)scratch(13, sizeof(float) * (size_t)T * n_out);
+    if (!h || !d || !dX || !dO) return -2;
+    const uint8_t** tab = (const uint8_t**)h;
+    memset(h, 0, tb);
+    for (int e = 0; e < n_exp; e++) {
+        if (!cnt[e]) continue;
         const DracoMat* g = get_mat((const void*)(uintptr_t)ep[3 * e], cg, inter, n_in);
         const DracoMat* u = get_mat((const void*)(uintptr_t)ep[3 * e + 1], cu, inter, n_in);
-        const DracoMat* d = get_mat((const void*)(uintptr_t)ep[3 * e + 2], cd, n_out, inter);
-        if (!g || !u || !d) return -2;
-        const int o = (cnt[e] + 7) / 8;
-        gg[k] = {g->dev, oct0[e], o};
-        gu[k] = {u->dev, oct0[e], o};
-        gd[k] = {d->dev, oct0[e], o};
+        const DracoMat* dn = get_mat((const void*)(uintptr_t)ep[3 * e + 2], cd, n_out, inter);
+        if (!g || !u || !dn) return -2;
+        tab[e] = g->dev;
+        tab[n_exp + e] = u->dev;
+        tab[2 * (size_t)n_exp + e] = dn->dev;
     }
-    // device buffers (scratch slots 8..): inputs, gathered rows, digits, intermediates, tables
-    const size_t fX = (size_t)T * n_in, fXg = (size_t)R * n_in, fI = (size_t)R * inter, fY = (size_t)R * n_out,
-                 fO = (size_t)T * n_out;
-    float* dX = (float*)scratch(8, sizeof(float) * fX);
-    float* dXg = (float*)scratch(9, sizeof(float) * fXg);
-    float* dG = (float*)scratch(10, sizeof(float) * fI);
-    float* dU = (float*)scratch(11, sizeof(float) * fI);
-    float* dY = (float*)scratch(12, sizeof(float) * fY);
-    float* dO = (float*)scratch(13, sizeof(float) * fO);
-    const size_t dbytes = draco_gemm_digit_bytes(R, n_in > inter ? n_in : inter);
-    uint8_t* dD = (uint8_t*)scratch(14, dbytes);
-    const size_t tb = sizeof(int) * ((size_t)R + (size_t)T * n_used) + sizeof(float) * (size_t)T * n_used +
-                      sizeof(GemmGroup) * 3 * (size_t)na + 64;
-    char* dT = (char*)scratch(15, tb);
-    if (!dX || !dXg || !dG || !dU || !dY || !dO || !dD || !dT) return -2;
-    int* dsrc = (int*)dT;
-    int* dpos = dsrc + R;
-    float* dwt = (float*)(dpos + (size_t)T * n_used);
-    GemmGroup* dgr = (GemmGroup*)(((uintptr_t)(dwt + (size_t)T * n_used) + 15) & ~(uintptr_t)15);
-    std::vector<GemmGroup> allg;
-    allg.insert(allg.end(), gg.begin(), gg.end());
-    allg.insert(allg.end(), gu.begin(), gu.end());
-    allg.insert(allg.end(), gd.begin(), gd.end());
-    DRACO_HIP(hipMemcpyAsync(dX, X, sizeof(float) * fX, hipMemcpyHostToDevice, st));
-    DRACO_HIP(hipMemcpyAsync(dsrc, src.data(), sizeof(int) * R, hipMemcpyHostToDevice, st));
-    DRACO_HIP(hipMemcpyAsync(dpos, pos.data(), sizeof(int) * pos.size(), hipMemcpyHostToDevice, st));
-    DRACO_HIP(hipMemcpyAsync(dwt, wtop, sizeof(float) * (size_t)T * n_used, hipMemcpyHostToDevice, st));
-    DRACO_HIP(hipMemcpyAsync(dgr, allg.data(), sizeof(GemmGroup) * allg.size(), hipMemcpyHostToDevice, st));
-    if (draco_moe_gather_launch(dX, n_in, dsrc, R, dXg, st)) return fail(-1, "moe_tok gather rejected");
-    auto grouped = [&](const float* Xin, int k_in, int code, const GemmGroup* groups, int rows, float* Y) -> int {
-        DracoLayout L;
-        if (draco_layout(code, rows, k_in, &L)) return fail(-1, "moe_tok layout");
-        GemmArgs a = {};
-        if (draco_gemm_digits_launch(Xin, R, k_in, dD, a, st)) return fail(-1, "moe_tok digits rejected");
-        a.L = L;
-        a.Y = Y;
-        a.ldy = rows;
-        a.groups = groups;
-        a.n_groups = na;
-        a.max_oct = max_oct;
-        if (draco_gemm_grouped_launch(a, st)) return fail(-1, "moe_tok gemm rejected");
-        return 0;
-    };
-    if (int rc = grouped(dXg, n_in, cg, dgr, inter, dG)) return rc;
-    {
-        // the gate and up GEMMs share the digits of Xg: reuse them for up
-        DracoLayout L;
-        draco_layout(cu, inter, n_in, &L);
-        GemmArgs a = {};
-        const size_t oct = (size_t)R / 8;
-        a.xdig = reinterpret_cast<const int8_t*>(dD);
-        a.xsc = reinterpret_cast<const float*>(dD + oct * ((size_t)n_in / 32) * 1024);
-        a.xs32 = a.xsc + oct * ((size_t)n_in / 256) * 8;
-        a.xs16 = a.xs32 + oct * ((size_t)n_in / 32) * 8;
-        a.T = R;
-        a.n_in = n_in;
-        a.L = L;
-        a.Y = dU;
-        a.ldy = inter;
-        a.groups = dgr + na;
-        a.n_groups = na;
-        a.max_oct = max_oct;
-        if (draco_gemm_grouped_launch(a, st)) return fail(-1, "moe_tok up gemm rejected");
-    }
-    dk_swiglu(dG, dU, R * inter, st);
-    if (int rc = grouped(dG, inter, cd, dgr + 2 * na, n_out, dY)) return rc;
-    if (draco_moe_scatter_launch(dY, n_out, dpos, dwt, n_used, T, dO, st)) return fail(-1, "moe_tok scatter rejected");
+    memcpy(h + tb, order, sizeof(int) * n);
+    memcpy(h + tb + sizeof(int) * n, wtop, sizeof(float) * n);
+    DRACO_HIP(hipMemcpyAsync(d, h, all, hipMemcpyHostToDevice, st));
+    DRACO_HIP(hipMemcpyAsync(dX, X, sizeof(float) * (size_t)T * n_in, hipMemcpyHostToDevice, st));
+    if (int rc = moe_rows(dX, (const int*)(d + tb), (const float*)(d + tb + sizeof(int) * n), (const uint8_t* const*)d, cg,
+                          cu, cd, T, n_used, n_exp, inter, n_in, n_out, tiles, dO, st))
+        return rc;
     DRACO_HIP(hipGetLastError());
-    DRACO_HIP(hipMemcpyAsync(out, dO, sizeof(float) * fO, hipMemcpyDeviceToHost, st));
+    DRACO_HIP(hipMemcpyAsync(out, dO, sizeof(float) * (size_t)T * n_out, hipMemcpyDeviceToHost, st));
     DRACO_HIP(hipStreamSynchronize(st));
     return 0;
 }
@@ -499,6 +493,34 @@ int draco_moe_layer_enqueue(MoeLayer* m, const float* x, const float* norm_w, fl
     if (split_out && !draco_moe_layer_split_ok(m)) return fail(-1, "moe layer: %d experts cannot split", p.n_used);
     return enqueue_moe(m->set, x, out, resid, m->w, p.n_exp, p.n_used, p.inter, p.n_in, p.n_out, st, norm_w, eps,
                        m->xn, pend, xs, pend_fx, split_out);
+}
+
+// Whether the layer's FFN runs over token rows: formats and widths that the
+// grouped products and the chunk's router serve.
+bool draco_moe_layer_rows_ok(const MoeLayer* m) {
+    const DracoMoeP& p = m->snap;
+    return draco_moe_route_ok(p.n_in, p.n_exp, p.n_used) && p.n_in % 256 == 0 && p.inter % 256 == 0;
+}
+
+int draco_moe_layer_rows(MoeLayer* m, const float* Xn, int T, float* Y, hipStream_t st) {
+    const DracoMoeP& p = m->snap;
+    constexpr int SLICE = 256;  // tokens at a time: bounds the gathered rows' buffers
+    const int cap = T < SLICE ? T : SLICE;
+    int* order = (int*)scratch(15, (sizeof(int) + sizeof(float)) * (size_t)cap * p.n_used);
+    if (!order) return -2;
+    float* wt = (float*)(order + (size_t)cap * p.n_used);
+    for (int t0 = 0; t0 < T; t0 += SLICE) {
+        const int n = T - t0 < SLICE ? T - t0 : SLICE;
+        const float* X = Xn + (size_t)t0 * p.n_in;
+        if (draco_moe_route_launch(X, (const float*)m->set->router->dev, n, p.n_in, p.n_exp, p.n_used, order, wt, st))
+            return fail(-1, "moe layer: chunk router rejected");
+        if (int rc = moe_rows(X, order, wt, (const uint8_t* const*)m->set->dev, m->set->host_codes[0],
+                              m->set->host_codes[1], m->set->host_codes[2], n,
+                              p.n_used, p.n_exp, p.inter, p.n_in, p.n_out, tiles_max(n, p.n_used, p.n_exp),
+                              Y + (size_t)t0 * p.n_out, st))
+            return rc;
+    }
+    return 0;
 }
 
 int draco_moe_layer_enqueue_xn(MoeLayer* m, const float* xn, float* out, const float* resid, hipStream_t st) {

@@ -910,7 +910,7 @@ int qstack_pf(QStack* s, int cap) {
         qstack_alloc(k, &s->PG, c * std::max(s->max_ff, 1)) || qstack_alloc(k, &s->PU, c * std::max(s->max_ff, 1)) ||
         qstack_alloc(k, &s->PPSS, c * std::max(s->max_vh, 1) * GDN_PSS_STRIDE))
         return -2;
-    if (hipMalloc(&s->dig, draco_gemm_digit_bytes(cap, ((win + 255) / 256) * 256)) != hipSuccess ||
+    if (hipMalloc(&s->dig, draco_gemmh_x_bytes(cap, ((win + 255) / 256) * 256)) != hipSuccess ||
         hipMalloc(&s->ids, sizeof(int) * c) != hipSuccess)
         return fail(-2, "qwen stack: prefill allocation failed");
     k.push_back(s->dig);

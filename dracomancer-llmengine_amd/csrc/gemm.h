@@ -1,39 +1,9 @@
-// gemm.h -- internal interface of the prefill GEMM kernels (gemm.hip).
+// gemm.h -- internal interface of the prefill GEMM (gemmh.hip).
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
 #include "formats.h"
-
-// One group of a grouped GEMM (e.g. one expert): its weights and its tokens,
-// octets [oct0, oct0 + n_oct) of the digit buffer.
-struct GemmGroup {
-    const uint8_t* W;
-    int oct0, n_oct;
-};
-
-struct GemmArgs {
-    const uint8_t* W;   // weights, Q4_K / Q6_K tile layout
-    DracoLayout L;
-    int n_in, T;
-    // digitized activations (draco_gemm_digits_launch)
-    const int8_t* xdig;
-    const float* xsc;
-    const float* xs32;
-    const float* xs16;
-    float* Y;           // Y[t * ldy + row]
-    int ldy;
-    // grouped launch (nullptr: one group = W, all tokens)
-    const GemmGroup* groups;  // device array [n_groups]
-    int n_groups;
-    int max_oct;              // largest n_oct of any group
-};
-
-// device bytes of the digit buffer for T tokens of length n_in
-size_t draco_gemm_digit_bytes(int T, int n_in);
-// digitize X[T][n_in] (device) into buf; fills a.xdig/xsc/xs32/xs16, a.T, a.n_in
-int draco_gemm_digits_launch(const float* X, int T, int n_in, uint8_t* buf, GemmArgs& a, hipStream_t st);
-int draco_gemm_launch(GemmArgs& a, hipStream_t st);
 
 // ---- f16-MFMA GEMM (gemmh.hip) ----
 // One matrix of a launch: Y[t * ldy + row] = x_t . W[row].
@@ -69,7 +39,7 @@ int draco_gemmh_launch(GemmHArgs& a, hipStream_t st);
 struct DracoMat;
 // Y_i[t][row] = X[t] . W_i[row] for T token rows and n matrices on the same
 // rows (X, Y device, token-major).  The block formats (draco_gemmh_serves): X's
-// activation operands (f16 hi/lo) into `digits` (draco_gemm_digit_bytes(T,
+// activation operands (f16 hi/lo) into `digits` (draco_gemmh_x_bytes(T,
 // n_in) bytes), then f16-MFMA launches of up to three matrices each; F32 and
 // F16: one GEMV per token.
 struct GemmTo {
@@ -80,5 +50,3 @@ int draco_enqueue_gemms(const GemmTo* to, int n, const float* X, int T, uint8_t*
 // silu(gate . x) * (up . x) of T rows into G; U is scratch for formats whose pair is not one launch
 int draco_enqueue_swiglu(const DracoMat& gate, const DracoMat& up, const float* X, int T, float* G, float* U,
                          uint8_t* digits, hipStream_t st);
-// Y[t] for the tokens of every group against that group's W (same shape for all groups)
-int draco_gemm_grouped_launch(GemmArgs& a, hipStream_t st);

@@ -1,18 +1,18 @@
 // gemmh.hip -- chunked-prefill GEMM on f16 MFMA (gfx950): Y[t][n] = x_t . W_n
 // for Q4_K, Q5_K, Q6_K and Q8_0 weights in their device layouts (formats.h).
 //
-// Exactness.  The weights enter the MFMA as f16 integers: Q4_K sc*q (at most
-// 63*15), Q5_K sc*(q-16) (63*16), Q8_0 q, all exact; Q6_K sc*(q-32) (|.| <= 4096)
+// Exactness.  The weights enter the MFMA as f16 integers: Q4_K sc*(q-8) (at
+// most 63*8), Q5_K sc*(q-16) (63*16), Q8_0 q, all exact; Q6_K sc*(q-32) (|.| <= 4096)
 // as its f16 rounding plus the rest (-1, 0 or 1).  Per (token, 256-value
 // super-block) the activations are scaled by 2^-e (e = ilogb(max|x|) - 14, so
 // |x'| < 2^15) and split into two f16 (hi = f16(x'), lo = f16(x' - hi));
 // x' - hi - lo is below 2^-22 |x'|, and so is the one product left out (Q6_K's
 // lo * rest).  f16 x f16 products are exact in the MFMA's fp32 accumulation.
 // Per super-block and row, with 2^e the token's scale:
-//   Q4_K: y += 2^e * (d * sum_k (sc*q)_k x'_k - 32 * dmin * sum_sb m_sb S'_sb)
-//         with S'_sb = 2^-5 * (sum of the sub-block's x'), itself on the MFMA
-//         (K = 8 sub-blocks, hi/lo);
-//   Q5_K: the same with q - 16 and 512 * d * sum_sb sc_sb S'_sb added;
+//   Q4_K, Q5_K: y += 2^e * (d * (sum_k (sc*(q-z))_k x'_k + 32 * z * sum_sb sc_sb S'_sb)
+//                           - 32 * dmin * sum_sb m_sb S'_sb), z = 8 or 16,
+//         with S'_sb = 2^-5 * (sum of the sub-block's x'), the sums over
+//         sub-blocks themselves on the MFMA (K = 8 sub-blocks, hi/lo);
 //   Q6_K: y += 2^e * d * sum (sc*(q-32)) x';
 //   Q8_0: y += 2^e * sum_blocks d_block * (sum q x').
 // The hi and the lo products accumulate apart: the lo sums are 2^-11 of the
@@ -83,6 +83,7 @@ __global__ __launch_bounds__(256) void k_gemmh_x(const float* __restrict__ X, in
     const int b = blockIdx.x, tt = blockIdx.y, tid = threadIdx.x;
     const int m = tid >> 3, sb = tid & 7, t = 32 * tt + m, nb = (n_in + 255) >> 8;
     float v[32];
+    if (rows && rows[32 * tt] < 0) return;  // a tile without tokens (they fill tiles from the front)
     const int row = t < T ? (rows ? rows[t] : t) : -1;
     const bool live = row >= 0 && b * 256 + 32 * sb < n_in;  // whole 32-value blocks (n_in % 32 == 0)
     const float* src = X + (size_t)max(row, 0) * n_in + (size_t)b * 256 + 32 * sb;
@@ -151,7 +152,8 @@ __device__ __forceinline__ v16f mfma16(v8h a, v8h b, v16f c) {
 // of w & m.  The constant is held in a VGPR (magic_k): v_and_or_b32 takes one scalar operand, and with two constants the
 // compiler uses two instructions (445 -> 365 VALU a tile).
 __device__ __forceinline__ uint32_t magic(uint32_t w, uint32_t m, uint32_t k) { return (w & m) | k; }
-__device__ __forceinline__ uint32_t magic_k(uint32_t k) {
+__device__ __forceinline__ uint32_t magic_k() {
+    uint32_t k = 0x64006400u;
     asm volatile("" : "+v"(k));
     return k;
 }
@@ -266,53 +268,49 @@ struct WPtr {
 template <int FM>
 __device__ __forceinline__ void tile_mma(WFrag<FM>& f, const WPtr<FM>& nx, const v8h (&hi)[16], const v8h (&lo)[16],
                                          const uint8_t* mm, int lane, float (&o)[16]) {
-    const uint32_t mk = magic_k(0x64006400u);
+    const uint32_t mk = magic_k();
     if constexpr (FM == 1 || FM == 4) {
-        const uint32_t mk5 = FM == 4 ? magic_k(0x50005000u) : 0u;
         // 6-bit scales and mins (src/m5_kern_scalar.c:39-46), bytes of sub-blocks 0..3 and 4..7.
-        // Q4_K, low nibbles: (1024 + q) c - 1024 c; high nibbles stay in place: (1024 + 16 q) (c / 16) - 64 c.
-        // Q5_K: (32 + q) c - 48 c = (q - 16) c, with 16 sum_sb sc_sb S_sb beside the min term: centred, the
-        // weights' sum is not twice the size of what the min term leaves of it
+        // The quant sits at bits 4.. of its half: (1024 + 16 q) (c / 16) - (64 + z) c = (q - z) c with z = 8
+        // (Q4_K) or 16 (Q5_K), and z sum_sb sc_sb S_sb joins beside the min term: centred, the weights' sum
+        // is not twice the size of what the min term leaves of it
+        constexpr float Z = FM == 4 ? 16.f : 8.f;
         const uint4 h = f.h;
         uint4 qh = {};
         if constexpr (FM == 4) qh = f.qh;
         const uint32_t sb[2] = {h.y & 0x3F3F3F3Fu, (h.w & 0x0F0F0F0Fu) | ((h.y >> 2) & 0x30303030u)};
         const uint32_t mb[2] = {h.z & 0x3F3F3F3Fu, ((h.w >> 4) & 0x0F0F0F0Fu) | ((h.z >> 2) & 0x30303030u)};
         const float dd = h2f((uint16_t)(h.x & 0xFFFF)), dm = -32.f * h2f((uint16_t)(h.x >> 16));
-        v2h cl[2], ol[2], ch[2], oh[2];
+        v2h cc[4], oo[4];  // of sub-blocks (0, 2), (1, 3), (4, 6), (5, 7)
 #pragma unroll
         for (int q = 0; q < 2; q++) {
             v2h a, b;
             pairs(sb[q], mk, a, b);
-            cl[q] = a - splat(1024.f);
+            a = a - splat(1024.f);
             b = b - splat(1024.f);
-            ch[q] = FM == 4 ? b : b * splat(0.0625f);
-            ol[q] = cl[q] * splat(FM == 4 ? -48.f : -1024.f);
-            oh[q] = b * splat(FM == 4 ? -48.f : -64.f);
+            cc[2 * q] = a * splat(0.0625f);
+            oo[2 * q] = a * splat(-64.f - Z);
+            cc[2 * q + 1] = b * splat(0.0625f);
+            oo[2 * q + 1] = b * splat(-64.f - Z);
         }
         nx.hdr(f);
         auto bfrag = [&](int s) {  // the weights of K-step s
             const int k = s >> 1, bh = s & 1, nib = k & 1;
             const uint4 qv = f.qv[s >> 2];
-            const v2h cp = nib ? ch[k >> 2] : cl[k >> 2], op = nib ? oh[k >> 2] : ol[k >> 2];
+            const v2h cp = cc[2 * (k >> 2) + nib], op = oo[2 * (k >> 2) + nib];
             const v2h c = (k & 2) ? (v2h){cp.y, cp.y} : (v2h){cp.x, cp.x};
             const v2h of = (k & 2) ? (v2h){op.y, op.y} : (v2h){op.x, op.x};
             uint32_t p[4];
 #pragma unroll
             for (int q = 0; q < 2; q++) {
                 uint32_t w = q ? (bh ? qv.w : qv.y) : (bh ? qv.z : qv.x);
-                uint32_t a, b;
-                if constexpr (FM == 1) {
-                    w ^= 0x80808080u;  // stored XOR 0x80
-                    const uint32_t m = nib ? 0x00F000F0u : 0x000F000Fu;
-                    a = magic(w, m, mk);
-                    b = magic(w >> 8, m, mk);
-                } else {  // 32 + q: the nibble at bits 5..8, the fifth bit (value 32k + i: bit k of qh[i]) at bit 9
+                if constexpr (FM == 1) w ^= 0x80808080u;  // stored XOR 0x80
+                uint32_t a = magic(nib ? w : w << 4, 0x00F000F0u, mk);
+                uint32_t b = magic(nib ? w >> 8 : w >> 4, 0x00F000F0u, mk);
+                if constexpr (FM == 4) {  // the fifth bit (value 32k + i: bit k of qh[i]) at bit 8
                     const uint32_t H = q ? (bh ? qh.w : qh.y) : (bh ? qh.z : qh.x);
-                    a = magic(nib ? w << 1 : w << 5, 0x01E001E0u, mk5);
-                    b = magic(nib ? w >> 7 : w >> 3, 0x01E001E0u, mk5);
-                    a = magic(H << (9 - k), 0x02000200u, a);
-                    b = magic(k ? H >> (k - 1) : H << 1, 0x02000200u, b);
+                    a = magic(H << (8 - k), 0x01000100u, a);
+                    b = magic(H >> k, 0x01000100u, b);
                 }
                 p[2 * q] = u2(__builtin_elementwise_fma(h2(a), c, of));
                 p[2 * q + 1] = u2(__builtin_elementwise_fma(h2(b), c, of));
@@ -348,18 +346,14 @@ __device__ __forceinline__ void tile_mma(WFrag<FM>& f, const WPtr<FM>& nx, const
         const v8h Bm = pack8(bm[0], bm[1], bm[2], bm[3]);
         const v8h mh = lds8(mm + lane * 16), ml = lds8(mm + 1024 + lane * 16);
         const v16f M = mfma16(mh, Bm, mfma16(ml, Bm, (v16f){}));
+        // 32 z sum_sb sc_sb S'_sb onto the small lo sums (cc holds sc / 16)
+        uint32_t bs[4];
 #pragma unroll
-        for (int i = 0; i < 16; i++) o[i] = fmaf(dd, P[i], dd * Q[i]);
-        if constexpr (FM == 4) {
-            const v8h Bs = pack8(u2(cl[0]) & keep, u2(ch[0]) & keep, u2(cl[1]) & keep, u2(ch[1]) & keep);
-            const v16f C = mfma16(mh, Bs, mfma16(ml, Bs, (v16f){}));
-            // the two large terms meet first
+        for (int q = 0; q < 4; q++) bs[q] = u2(cc[q] * splat(512.f * Z)) & keep;
+        const v8h Bs = pack8(bs[0], bs[1], bs[2], bs[3]);
+        Q = mfma16(mh, Bs, mfma16(ml, Bs, Q));
 #pragma unroll
-            for (int i = 0; i < 16; i++) o[i] += fmaf(dm, M[i], 512.f * dd * C[i]);
-        } else {
-#pragma unroll
-            for (int i = 0; i < 16; i++) o[i] = fmaf(dm, M[i], o[i]);
-        }
+        for (int i = 0; i < 16; i++) o[i] = fmaf(dd, P[i], fmaf(dm, M[i], dd * Q[i]));
     } else if constexpr (FM == 2) {
         const float dd = h2f((uint16_t)f.d);
         v2h c[2][2];
@@ -565,15 +559,19 @@ __device__ __forceinline__ void gemmr_body(const GemmHArgs& a, const GemmHSeg& s
 }
 
 // XCD x runs blocks x, x + 8, ...: an XCD's consecutive blocks are the token
-// tiles of one row group, so a group's weights come from HBM once per XCD.
+// tiles of one row group, so a group's weights come from HBM once per XCD; in
+// grouped launches they are the row groups of one tile, whose activations stay
+// in that XCD's L2 (the experts' weights are read once anyway).
 // F0 / F1: the formats that the launch's matrices have.
 template <int F0, int F1, int NSB, bool PAIR>
 __global__ __launch_bounds__(512) void k_gemmr(const GemmHArgs a) {
     extern __shared__ __align__(16) uint8_t sm[];
     const int ntt = a.groups ? a.max_tiles : (a.T + 31) >> 5;
     const int loc = blockIdx.x >> 3;
-    int tt = loc % ntt, rg = (loc / ntt) * 8 + (blockIdx.x & 7);
-    if (rg >= a.n_rg) return;
+    const int x = blockIdx.x & 7;
+    const int tt = a.groups ? (loc / a.n_rg) * 8 + x : loc % ntt;
+    const int rg = a.groups ? loc % a.n_rg : (loc / ntt) * 8 + x;
+    if (rg >= a.n_rg || tt >= ntt) return;
     const int s = a.nseg > 1 && rg >= a.seg[1].rg0 ? (a.nseg > 2 && rg >= a.seg[2].rg0 ? 2 : 1) : 0;
     const GemmHSeg& sg = a.seg[s];
     const uint8_t *W0 = sg.W, *W1 = PAIR ? a.seg[1].W : nullptr;
@@ -693,6 +691,6 @@ int draco_gemmh_launch(GemmHArgs& a, hipStream_t st) {
         a.n_rg += groups_of(s);
     }
     if (a.pair) a.nseg = 1;  // (the second matrix is read through its base)
-    const unsigned grid = (unsigned)((a.n_rg + 7) / 8 * 8 * ntt);
+    const unsigned grid = (unsigned)(a.groups ? (ntt + 7) / 8 * 8 * a.n_rg : (a.n_rg + 7) / 8 * 8 * ntt);
     return NSB == 4 ? pick<4>(a, f0, f1, grid, st) : pick<8>(a, f0, f1, grid, st);
 }

@@ -90,7 +90,17 @@ bool draco_moe_layer_pend_ok(const MoeLayer* m, const float* norm_w);
 // FFN input x2n, src/qwen35_engine.py:325)
 int draco_moe_layer_enqueue_xn(MoeLayer* m, const float* xn, float* out, const float* resid, hipStream_t st);
 
-// token-batched MoE helpers
-int draco_moe_gather_launch(const float* X, int n_in, const int* src, int rows, float* Xg, hipStream_t st);
+// ---- token-batched MoE (prefill) ----
+// order / wt [T][n_used]: the experts and weights of every token's FFN input row
+bool draco_moe_route_ok(int n_in, int n_exp, int n_used);
+int draco_moe_route_launch(const float* X, const float* gate_inp, int T, int n_in, int n_exp, int n_used, int* order,
+                           float* wt, hipStream_t st);
+// the pairs of order grouped by expert into 32-row tiles (k_moe_plan)
+int draco_moe_plan_launch(const int* order, int T, int n_used, int n_exp, int max_tiles, int* tile_exp, int* rows,
+                          int* pos, hipStream_t st);
 int draco_moe_scatter_launch(const float* Yd, int n_out, const int* pos, const float* wt, int n_used, int T, float* out,
                              hipStream_t st);
+// Y[t] = MoE(Xn[t]) of T FFN input rows of a decoder layer (device pointers),
+// routed, multiplied expert by expert and combined on the device.
+bool draco_moe_layer_rows_ok(const MoeLayer* m);
+int draco_moe_layer_rows(MoeLayer* m, const float* Xn, int T, float* Y, hipStream_t st);

@@ -578,30 +578,152 @@ __global__ __launch_bounds__(64 * NW) void k_moe_down(const uint8_t* const* __re
     }
 }
 
-// Token-batched MoE (prefill): gather the token rows of every expert segment
-// (src[row] = token or -1 for padding), and the deterministic scatter
-// out[t] = sum_k w[t,k] * Yd[pos[t,k]] in k order (src/m6_moe_tok.c:148-159).
-__global__ __launch_bounds__(256) void k_moe_gather(const float* __restrict__ X, int n_in, const int* __restrict__ src,
-                                                    float* __restrict__ Xg) {
-    const int row = blockIdx.x, t = src[row];
-    for (int i = threadIdx.x * 4; i < n_in; i += 1024) {
-        const float4 v = t >= 0 ? ld4(X + (size_t)t * n_in + i) : make_float4(0.f, 0.f, 0.f, 0.f);
-        *reinterpret_cast<float4*>(Xg + (size_t)row * n_in + i) = v;
+// ---- token-batched MoE (prefill) ----
+
+// Router logits, softmax and top-k of RT tokens per block, as the one-token
+// launches form them: probabilities by softmax_wave, slots by rank, weights
+// divided by their slot-order sum (at least 2^-14).  The tokens' rows are
+// staged in LDS, each wave dots them with every eighth expert row (lane sums
+// in four chains, then the wave tree).
+constexpr int RT = 4;
+__global__ __launch_bounds__(512) void k_moe_route(const float* __restrict__ X, const float* __restrict__ gi, int T,
+                                                   int n_in, int n_exp, int n_used, int* __restrict__ order,
+                                                   float* __restrict__ wt) {
+    extern __shared__ __align__(16) uint8_t smem[];
+    float* xs = reinterpret_cast<float*>(smem);                       // [RT][n_in]
+    float* lg = xs + (size_t)RT * n_in;                               // [RT][MOE_EXP_MAX]
+    float* sp = lg + RT * MOE_EXP_MAX;                                // [RT][MOE_EXP_MAX]
+    float* sw = sp + RT * MOE_EXP_MAX;                                // [RT][MOE_USED_MAX]
+    int* si = reinterpret_cast<int*>(sw + RT * MOE_USED_MAX);         // [RT][MOE_USED_MAX]
+    const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int t0 = blockIdx.x * RT, nt = min(RT, T - t0);
+    for (int i = tid * 4; i < RT * n_in; i += 2048) {
+        const int t = i / n_in;
+        *reinterpret_cast<float4*>(xs + i) = ld4(X + (size_t)(t0 + min(t, nt - 1)) * n_in + (i - t * n_in));
+    }
+    // slots default to expert 0 with weight 0 (probabilities that hold a NaN rank no expert there)
+    for (int i = tid; i < RT * MOE_USED_MAX; i += 512) {
+        si[i] = 0;
+        sw[i] = 0.f;
+    }
+    __syncthreads();
+    for (int e = w; e < n_exp; e += 8) {
+        float4 acc[RT] = {};
+        for (int i = lane * 4; i < n_in; i += 256) {
+            const float4 g = ld4(gi + (size_t)e * n_in + i);
+#pragma unroll
+            for (int t = 0; t < RT; t++) {
+                const float4 x = ld4(xs + (size_t)t * n_in + i);
+                acc[t].x = fmaf(x.x, g.x, acc[t].x);
+                acc[t].y = fmaf(x.y, g.y, acc[t].y);
+                acc[t].z = fmaf(x.z, g.z, acc[t].z);
+                acc[t].w = fmaf(x.w, g.w, acc[t].w);
+            }
+        }
+#pragma unroll
+        for (int t = 0; t < RT; t++) {
+            const float v = wave_sum((acc[t].x + acc[t].y) + (acc[t].z + acc[t].w));
+            if (lane == 0) lg[t * MOE_EXP_MAX + e] = v;
+        }
+    }
+    __syncthreads();
+    if (w < RT) softmax_wave(lg + w * MOE_EXP_MAX, n_exp, sp + w * MOE_EXP_MAX);
+    __syncthreads();
+    const int part = tid & 3, span = ((n_exp + 15) >> 4) << 2;
+    for (int t = 0; t < nt; t++)
+        for (int e0 = 0; e0 < n_exp; e0 += 128) {  // uniform
+            const int e = e0 + (tid >> 2);
+            int r = e < n_exp ? rank_part(sp + t * MOE_EXP_MAX, e, part * span, span) : 0;
+            r = group_reduce<4>(r, OpAdd{});
+            if (part == 0 && e < n_exp && r < n_used) {
+                si[t * MOE_USED_MAX + r] = e;
+                sw[t * MOE_USED_MAX + r] = sp[t * MOE_EXP_MAX + e];
+            }
+        }
+    __syncthreads();
+    for (int i = tid; i < nt * n_used; i += 512) {
+        const int t = i / n_used, j = i - t * n_used;
+        float ws = 0.f;
+        for (int k = 0; k < n_used; k++) ws += sw[t * MOE_USED_MAX + k];
+        if (ws < 6.103515625e-5f) ws = 6.103515625e-5f;
+        order[(size_t)(t0 + t) * n_used + j] = si[t * MOE_USED_MAX + j];
+        wt[(size_t)(t0 + t) * n_used + j] = sw[t * MOE_USED_MAX + j] / ws;
     }
 }
 
+// Groups the n = T * n_used (token, slot) pairs by expert into 32-row tiles:
+// tile_exp[tile] = its expert (-1 past the last tile), rows[row] = token (-1:
+// padding), pos[pair] = row (-1: an expert out of range).  Tiles fill from the
+// front.  One block; the order of a group's rows does not matter (each row's
+// result is its own).
+__global__ __launch_bounds__(1024) void k_moe_plan(const int* __restrict__ order, int n, int n_used, int n_exp,
+                                                   int max_tiles, int* __restrict__ tile_exp, int* __restrict__ rows,
+                                                   int* __restrict__ pos) {
+    __shared__ int cnt[MOE_EXP_MAX], t0[MOE_EXP_MAX], fill[MOE_EXP_MAX];
+    const int tid = threadIdx.x;
+    if (tid < MOE_EXP_MAX) cnt[tid] = fill[tid] = 0;
+    for (int i = tid; i < max_tiles; i += 1024) tile_exp[i] = -1;
+    for (int i = tid; i < 32 * max_tiles; i += 1024) rows[i] = -1;
+    __syncthreads();
+    for (int i = tid; i < n; i += 1024) {
+        const int e = order[i];
+        if (e >= 0 && e < n_exp) atomicAdd(&cnt[e], 1);
+    }
+    __syncthreads();
+    const int tiles = tid < MOE_EXP_MAX ? (cnt[tid] + 31) >> 5 : 0;
+    if (tid < MOE_EXP_MAX) t0[tid] = tiles;
+    __syncthreads();
+    for (int d = 1; d < MOE_EXP_MAX; d <<= 1) {  // inclusive scan
+        const int v = tid < MOE_EXP_MAX && tid >= d ? t0[tid - d] : 0;
+        __syncthreads();
+        if (tid < MOE_EXP_MAX) t0[tid] += v;
+        __syncthreads();
+    }
+    if (tid < MOE_EXP_MAX) {
+        const int first = t0[tid] - tiles;
+        for (int k = 0; k < tiles && first + k < max_tiles; k++) tile_exp[first + k] = tid;
+    }
+    __syncthreads();  // (also orders the -1 fills of rows before the writes below)
+    for (int i = tid; i < n; i += 1024) {
+        const int e = order[i];
+        int p = -1;
+        if (e >= 0 && e < n_exp) {
+            p = 32 * (t0[e] - ((cnt[e] + 31) >> 5)) + atomicAdd(&fill[e], 1);
+            rows[p] = i / n_used;
+        }
+        pos[i] = p;
+    }
+}
+
+// out[t] = sum_k w[t,k] * Yd[pos[t,k]] in k order (src/m6_moe_tok.c:148-159).
+// Eight slots' values are requested before the first is added (T = 128, 8
+// slots of 2048: one dependent load a slot and one float a thread took 22 us).
 __global__ __launch_bounds__(256) void k_moe_scatter(const float* __restrict__ Yd, int n_out, const int* __restrict__ pos,
                                                      const float* __restrict__ wt, int n_used, float* __restrict__ out) {
-    const int t = blockIdx.x;
-    for (int r = threadIdx.x; r < n_out; r += 256) {
-        float o = 0.f;
-        for (int k = 0; k < n_used; k++) {
-            const int p = pos[t * n_used + k];
-            if (p < 0) continue;
-            o += wt[t * n_used + k] * Yd[(size_t)p * n_out + r];
+    const int t = blockIdx.x, r = 4 * (blockIdx.y * 256 + threadIdx.x);
+    if (r >= n_out) return;
+    float4 o = make_float4(0.f, 0.f, 0.f, 0.f);
+    for (int k0 = 0; k0 < n_used; k0 += 8) {
+        float4 v[8];
+        float wk[8];
+        int p[8];
+#pragma unroll
+        for (int k = 0; k < 8; k++) {
+            const int i = t * n_used + min(k0 + k, n_used - 1);
+            p[k] = k0 + k < n_used ? pos[i] : -1;
+            wk[k] = wt[i];
+            v[k] = ld4(Yd + (size_t)max(p[k], 0) * n_out + r);
         }
-        out[(size_t)t * n_out + r] = o;
+#pragma unroll
+        for (int k = 0; k < 8; k++) {
+            if (p[k] < 0) continue;
+            o.x += wk[k] * v[k].x;
+            o.y += wk[k] * v[k].y;
+            o.z += wk[k] * v[k].z;
+            o.w += wk[k] * v[k].w;
+        }
     }
+    *reinterpret_cast<float4*>(out + (size_t)t * n_out + r) = o;
 }
 
 int cu_count() {
@@ -782,15 +904,32 @@ int draco_moe_down_launch(MoeArgs& a, int fm, hipStream_t st) {
     return 0;
 }
 
-int draco_moe_gather_launch(const float* X, int n_in, const int* src, int rows, float* Xg, hipStream_t st) {
-    if (n_in % 4 || rows < 1) return -1;
-    hipLaunchKernelGGL(k_moe_gather, dim3(rows), dim3(256), 0, st, X, n_in, src, Xg);
+static size_t route_lds(int n_in) {
+    return sizeof(float) * RT * ((size_t)n_in + 2 * MOE_EXP_MAX + 2 * MOE_USED_MAX);
+}
+bool draco_moe_route_ok(int n_in, int n_exp, int n_used) {
+    return n_in % 4 == 0 && n_exp >= 1 && n_exp <= MOE_EXP_MAX && n_used >= 1 && n_used <= MOE_USED_MAX &&
+           n_used <= n_exp && route_lds(n_in) <= 160 * 1024;
+}
+int draco_moe_route_launch(const float* X, const float* gate_inp, int T, int n_in, int n_exp, int n_used, int* order,
+                           float* wt, hipStream_t st) {
+    if (T < 1 || !draco_moe_route_ok(n_in, n_exp, n_used)) return -1;
+    static std::once_flag once;
+    std::call_once(once, [] { allow_big_lds(&k_moe_route); });
+    hipLaunchKernelGGL(k_moe_route, dim3((T + RT - 1) / RT), dim3(512), route_lds(n_in), st, X, gate_inp, T, n_in, n_exp,
+                       n_used, order, wt);
     return 0;
 }
-
+int draco_moe_plan_launch(const int* order, int T, int n_used, int n_exp, int max_tiles, int* tile_exp, int* rows,
+                          int* pos, hipStream_t st) {
+    if (T < 1 || n_used < 1 || n_exp < 1 || n_exp > MOE_EXP_MAX || max_tiles < 1) return -1;
+    hipLaunchKernelGGL(k_moe_plan, dim3(1), dim3(1024), 0, st, order, T * n_used, n_used, n_exp, max_tiles, tile_exp,
+                       rows, pos);
+    return 0;
+}
 int draco_moe_scatter_launch(const float* Yd, int n_out, const int* pos, const float* wt, int n_used, int T, float* out,
                              hipStream_t st) {
-    if (T < 1) return -1;
-    hipLaunchKernelGGL(k_moe_scatter, dim3(T), dim3(256), 0, st, Yd, n_out, pos, wt, n_used, out);
+    if (T < 1 || n_out % 4) return -1;
+    hipLaunchKernelGGL(k_moe_scatter, dim3(T, (n_out + 1023) / 1024), dim3(256), 0, st, Yd, n_out, pos, wt, n_used, out);
     return 0;
 }
