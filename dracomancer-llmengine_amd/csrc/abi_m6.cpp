@@ -1347,12 +1347,14 @@ int draco_llama_generate(const void* layers_v, int n_layer, int h, float eps, co
         dk_advance(m->state, n_layer, cursor, st);
         return 0;
     };
-    constexpr int GEN_STEPS = 16;
+    // tokens per decode graph: a graph of 16 steps decodes 0.2% faster than one
+    // of 4 but takes 2 ms more to capture, 400 tokens' worth
+    constexpr int GEN_STEPS = 4;
     // events and graphs are released on every return path (the guard's
     // destructor waits for the stream first, so no replay is still running)
     struct Guard {
         hipStream_t st;
-        hipEvent_t ev[3] = {nullptr, nullptr, nullptr};
+        hipEvent_t ev[4] = {nullptr, nullptr, nullptr, nullptr};
         hipGraphExec_t gx[3] = {nullptr, nullptr, nullptr};
         hipGraph_t gg[3] = {nullptr, nullptr, nullptr};
         ~Guard() {
@@ -1366,43 +1368,42 @@ int draco_llama_generate(const void* layers_v, int n_layer, int h, float eps, co
         }
     } G{st};
     for (hipEvent_t& e : G.ev) DRACO_HIP(hipEventCreate(&e));
-    hipEvent_t e0 = G.ev[0], e1 = G.ev[1], e2 = G.ev[2];
+    hipEvent_t e0 = G.ev[0], e1 = G.ev[1], e2 = G.ev[2], ep = G.ev[3];
     hipGraphExec_t* gx = G.gx;
+    // The chunked prompt is enqueued first, so that it runs while the host
+    // captures the decode graphs.
+    if (n_chunked) {
+        DRACO_HIP(hipEventRecord(e0, st));
+        if (enqueue_prefill(m, em, dtok, n_chunked, pos0, eps, st) <= 0)
+            return report(-1, "draco_llama_generate (chunked prefill)");
+        DRACO_HIP(hipEventRecord(ep, st));
+    }
+    if (int rc = upload_state(m, pos0 + n_chunked, st, n_chunked)) return report(rc, "draco_llama_generate");
     if (use_graph) {
-        for (int k = 0; k < 2; k++) {
-            DRACO_HIP(hipStreamBeginCapture(st, hipStreamCaptureModeRelaxed));
-            int rc = step(k == 1);
-            hipGraph_t gr = nullptr;
-            hipError_t ce = hipStreamEndCapture(st, &gr);
-            G.gg[k] = gr;
-            if (rc) return report(rc, "draco_llama_generate");
-            if (ce != hipSuccess) return report(fail(-2, "graph capture: %s", hipGetErrorString(ce)), "draco_llama_generate");
-            DRACO_HIP(hipGraphInstantiate(&gx[k], gr, nullptr, nullptr, 0));
-        }
-        // GEN_STEPS generated tokens in one graph (the state advances on the
-        // device, so consecutive steps capture as they run): one graph launch
-        // per GEN_STEPS tokens instead of per token (configs[2], 98 kernels a
-        // step: 2,219 -> 2,243 tok/s same-box).  Steps of more kernels keep one
-        // graph per token: configs[0] (194 a step) and configs[3] were 0.1-0.2%
-        // slower with 16-step graphs.
-        size_t step_nodes = 0;
-        DRACO_HIP(hipGraphGetNodes(G.gg[1], nullptr, &step_nodes));
-        if (n_gen >= GEN_STEPS && step_nodes * GEN_STEPS <= 2048) {
+        auto capture = [&](int k, int n, bool decode) -> int {
             DRACO_HIP(hipStreamBeginCapture(st, hipStreamCaptureModeRelaxed));
             int rc = 0;
-            for (int k = 0; k < GEN_STEPS && !rc; k++) rc = step(true);
-            hipGraph_t gr = nullptr;
-            hipError_t ce = hipStreamEndCapture(st, &gr);
-            G.gg[2] = gr;
-            if (rc) return report(rc, "draco_llama_generate");
-            if (ce != hipSuccess) return report(fail(-2, "graph capture: %s", hipGetErrorString(ce)), "draco_llama_generate");
-            DRACO_HIP(hipGraphInstantiate(&gx[2], gr, nullptr, nullptr, 0));
-        }
+            for (int i = 0; i < n && !rc; i++) rc = step(decode);
+            hipError_t ce = hipStreamEndCapture(st, &G.gg[k]);
+            if (rc) return rc;
+            if (ce != hipSuccess) return fail(-2, "graph capture: %s", hipGetErrorString(ce));
+            DRACO_HIP(hipGraphInstantiate(&gx[k], G.gg[k], nullptr, nullptr, 0));
+            return 0;
+        };
+        if (n_chunked < n_prompt - 1)  // token-serial prompt steps
+            if (int rc = capture(0, 1, false)) return report(rc, "draco_llama_generate");
+        if (int rc = capture(1, 1, true)) return report(rc, "draco_llama_generate");
+        // GEN_STEPS generated tokens in one graph (the state advances on the
+        // device, so consecutive steps capture as they run): one graph launch
+        // per GEN_STEPS tokens instead of per token.  Steps of more than 128
+        // kernels keep one graph per token (SmolLM2-360M's 130 and the 48-layer
+        // MoE stack were 0.1-0.2% slower with several).
+        size_t step_nodes = 0;
+        DRACO_HIP(hipGraphGetNodes(G.gg[1], nullptr, &step_nodes));
+        if (n_gen >= GEN_STEPS && step_nodes <= 128)
+            if (int rc = capture(2, GEN_STEPS, true)) return report(rc, "draco_llama_generate");
     }
-    DRACO_HIP(hipEventRecord(e0, st));
-    if (n_chunked && enqueue_prefill(m, em, dtok, n_chunked, pos0, eps, st) <= 0)
-        return report(-1, "draco_llama_generate (chunked prefill)");
-    if (int rc = upload_state(m, pos0 + n_chunked, st, n_chunked)) return report(rc, "draco_llama_generate");
+    if (!n_chunked) DRACO_HIP(hipEventRecord(e0, st));  // (the stats leave the capture out)
     for (int i = n_chunked; i < n_prompt - 1; i++) {
         if (use_graph) DRACO_HIP(hipGraphLaunch(gx[0], st));
         else if (int rc = step(false)) return report(rc, "draco_llama_generate");
@@ -1423,7 +1424,7 @@ int draco_llama_generate(const void* layers_v, int n_layer, int h, float eps, co
     if (out_hidden) DRACO_HIP(hipMemcpyAsync(out_hidden, m->w.x, sizeof(float) * h, hipMemcpyDeviceToHost, st));
     DRACO_HIP(hipStreamSynchronize(st));
     float ms_pre = 0, ms_dec = 0;
-    hipEventElapsedTime(&ms_pre, e0, e1);
+    hipEventElapsedTime(&ms_pre, e0, n_chunked ? ep : e1);
     hipEventElapsedTime(&ms_dec, e1, e2);
     if (stats) {
         stats[0] = ms_dec;

@@ -1369,7 +1369,7 @@ int draco_qwen_generate(const void* layers, int n_layer, int h, float eps, const
     };
     struct Guard {
         hipStream_t st;
-        hipEvent_t ev[3] = {nullptr, nullptr, nullptr};
+        hipEvent_t ev[4] = {nullptr, nullptr, nullptr, nullptr};
         hipGraphExec_t gx[2] = {nullptr, nullptr};
         hipGraph_t gg[2] = {nullptr, nullptr};
         ~Guard() {
@@ -1383,6 +1383,16 @@ int draco_qwen_generate(const void* layers, int n_layer, int h, float eps, const
         }
     } G{st};
     for (hipEvent_t& e : G.ev) DRACO_HIP(hipEventCreate(&e));
+    // the chunked prompt first: it runs while the host captures
+    if (n_chunked) {
+        DRACO_HIP(hipEventRecord(G.ev[0], st));
+        if (enqueue_qprefill(s, em, dtok, n_chunked, pos0, st) <= 0)
+            return report(-1, "draco_qwen_generate (chunked prefill)");
+        DRACO_HIP(hipEventRecord(G.ev[3], st));
+    }
+    s->hstate[0] = pos0 + n_chunked;
+    s->hstate[1] = pos0 + n_chunked;
+    DRACO_HIP(hipMemcpyAsync(s->state, s->hstate, sizeof(int) * 2, hipMemcpyHostToDevice, st));
     if (use_graph) {
         for (int k = 0; k < 2; k++) {
             if (k == 0 && n_chunked == n_prompt - 1) continue;  // no token-serial prompt step to capture
@@ -1396,12 +1406,7 @@ int draco_qwen_generate(const void* layers, int n_layer, int h, float eps, const
             DRACO_HIP(hipGraphInstantiate(&G.gx[k], gr, nullptr, nullptr, 0));
         }
     }
-    DRACO_HIP(hipEventRecord(G.ev[0], st));
-    if (n_chunked && enqueue_qprefill(s, em, dtok, n_chunked, pos0, st) <= 0)
-        return report(-1, "draco_qwen_generate (chunked prefill)");
-    s->hstate[0] = pos0 + n_chunked;
-    s->hstate[1] = pos0 + n_chunked;
-    DRACO_HIP(hipMemcpyAsync(s->state, s->hstate, sizeof(int) * 2, hipMemcpyHostToDevice, st));
+    if (!n_chunked) DRACO_HIP(hipEventRecord(G.ev[0], st));  // (the stats leave the capture out)
     for (int i = n_chunked; i < n_prompt - 1; i++) {
         if (use_graph) DRACO_HIP(hipGraphLaunch(G.gx[0], st));
         else if (int rc = step(false)) return report(rc, "draco_qwen_generate");
@@ -1417,7 +1422,7 @@ int draco_qwen_generate(const void* layers, int n_layer, int h, float eps, const
     if (out_hidden) DRACO_HIP(hipMemcpyAsync(out_hidden, s->x, sizeof(float) * h, hipMemcpyDeviceToHost, st));
     DRACO_HIP(hipStreamSynchronize(st));
     float ms_pre = 0.f, ms_dec = 0.f;
-    hipEventElapsedTime(&ms_pre, G.ev[0], G.ev[1]);
+    hipEventElapsedTime(&ms_pre, G.ev[0], n_chunked ? G.ev[3] : G.ev[1]);
     hipEventElapsedTime(&ms_dec, G.ev[1], G.ev[2]);
     if (stats) {
         stats[0] = ms_dec;
