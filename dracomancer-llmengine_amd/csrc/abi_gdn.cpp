@@ -22,21 +22,20 @@ int gdn_host(const float* QKV, const float* Z, const float* B, const float* G, c
     hipStream_t st = stream();
     const size_t nq = (size_t)T * n_qkv, nz = (size_t)T * n_vh * 128, nbg = (size_t)T * n_vh,
                  ns = (size_t)n_vh * 128 * 128, nt = (size_t)n_qkv * 3, nc = (size_t)n_qkv * 4;
-    const size_t npss = (size_t)T * n_vh * GDN_PSS_STRIDE;
-    float* d = (float*)scratch(6, sizeof(float) * (nq + 2 * nz + 2 * nbg + ns + nt + nc + 128 + npss));
+    float* d = (float*)scratch(6, sizeof(float) * (nq + 2 * nz + 2 * nbg + ns + nt + nc + 128 + nq));
     if (!d) return -2;
     GdnArgs a = {};
     float* p = d;
     float* dq = p; p += nq;
     float* dz = p; p += nz;
-    float* db = p; p += nbg;
-    float* dg = p; p += nbg;
     float* dc = p; p += nc;
     float* dn = p; p += 128;
     float* dt = p; p += nt;
     float* ds = p; p += ns;
-    float* dpss = p; p += npss;
-    float* don = p;
+    float* dcv = p; p += nq;
+    float* don = p; p += nz;
+    float* db = p; p += nbg;
+    float* dg = p;
     // a state the per-layer GDN op holds on the device is scanned in place
     // there (the caller's arrays hold only its sample); any other is uploaded
     float *rs = nullptr, *rt = nullptr;
@@ -69,7 +68,7 @@ int gdn_host(const float* QKV, const float* Z, const float* B, const float* G, c
     a.n_vh = n_vh;
     a.nhq = (n_qkv - n_vh * 128) / 256;
     a.nspl = T == 1 ? 1 : draco_gdn_split(false);  // one token: nothing to take the split's rms
-    a.PSS = dpss;
+    a.CV = dcv;
     if (draco_gdn_scan_launch(a, st)) return fail(-1, "gdn scan launch rejected");
     DRACO_HIP(hipGetLastError());
     DRACO_HIP(hipMemcpyAsync(ON, don, sizeof(float) * nz, hipMemcpyDeviceToHost, st));
@@ -110,8 +109,8 @@ int draco_bench_gdn_scan(const float* QKV, const float* Z, const float* B, const
     hipStream_t st = stream();
     const size_t nq = (size_t)T * n_qkv, nz = (size_t)T * n_vh * 128, nbg = (size_t)T * n_vh,
                  ns = (size_t)n_vh * 128 * 128, nt = (size_t)n_qkv * 3, nc = (size_t)n_qkv * 4;
-    float *dq, *dz, *db, *dg, *dc, *dn, *dt, *ds, *don, *dpss;
-    DRACO_HIP(hipMalloc(&dpss, sizeof(float) * (size_t)(chunk > 1 ? chunk : 1) * n_vh * GDN_PSS_STRIDE));
+    float *dq, *dz, *db, *dg, *dc, *dn, *dt, *ds, *don, *dcv;
+    DRACO_HIP(hipMalloc(&dcv, sizeof(float) * (size_t)chunk * n_qkv));
     DRACO_HIP(hipMalloc(&dq, sizeof(float) * nq));
     DRACO_HIP(hipMalloc(&dz, sizeof(float) * nz));
     DRACO_HIP(hipMalloc(&db, sizeof(float) * nbg));
@@ -145,7 +144,7 @@ int draco_bench_gdn_scan(const float* QKV, const float* Z, const float* B, const
         a.n_vh = n_vh;
         a.nhq = (n_qkv - n_vh * 128) / 256;
         a.nspl = n == 1 ? 1 : draco_gdn_split(false);
-        a.PSS = dpss;
+        a.CV = dcv;
         return a;
     };
     hipEvent_t e0, e1;
@@ -179,7 +178,7 @@ int draco_bench_gdn_scan(const float* QKV, const float* Z, const float* B, const
     }
     hipEventDestroy(e0);
     hipEventDestroy(e1);
-    for (float* p : {dq, dz, db, dg, dc, dn, dt, ds, don, dpss}) hipFree(p);
+    for (float* p : {dq, dz, db, dg, dc, dn, dt, ds, don, dcv}) hipFree(p);
     return 0;
 }
 

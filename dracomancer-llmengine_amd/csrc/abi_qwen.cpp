@@ -338,7 +338,7 @@ int enqueue_gdn(const GdnDev& g, const GdnBufs& b, hipStream_t st, bool post_nor
     a.PSS = b.pss;
     // split over several blocks per V head only when the ssm_out GEMV can
     // take the gated rms into its prologue (Q4_K / Q6_K): the split's extra
-    // k_gdn_gnorm launch costs more than the split saves
+    // launch of its own costs more than the split saves
     const bool kq = g.out->L.code == DRACO_Q4_K || g.out->L.code == DRACO_Q6_K;
     a.nspl = kq ? draco_gdn_split(true) : 1;
     a.defer_gnorm = a.nspl > 1;
@@ -691,7 +691,7 @@ struct QStack {
     int pf_cap = 0;
     float *X = nullptr, *Xn = nullptr, *QKV = nullptr, *Z = nullptr, *B = nullptr, *G = nullptr, *ON = nullptr,
           *Y = nullptr, *PQG = nullptr, *PQr = nullptr, *PK = nullptr, *PV = nullptr, *AO = nullptr, *Ppart = nullptr,
-          *PG = nullptr, *PU = nullptr, *PPSS = nullptr;
+          *PG = nullptr, *PU = nullptr, *PCV = nullptr;
     uint8_t* dig = nullptr;
     int* ids = nullptr;
     std::vector<void*> allocs, pf_allocs;
@@ -908,7 +908,7 @@ int qstack_pf(QStack* s, int cap) {
         qstack_alloc(k, &s->PK, c * FNKV * FHD) || qstack_alloc(k, &s->PV, c * FNKV * FHD) ||
         qstack_alloc(k, &s->AO, c * nh * FHD) || qstack_alloc(k, &s->Ppart, pf_part_floats(nh, cap, FHD, nspl)) ||
         qstack_alloc(k, &s->PG, c * std::max(s->max_ff, 1)) || qstack_alloc(k, &s->PU, c * std::max(s->max_ff, 1)) ||
-        qstack_alloc(k, &s->PPSS, c * std::max(s->max_vh, 1) * GDN_PSS_STRIDE))
+        qstack_alloc(k, &s->PCV, c * std::max(s->max_qkv, 1)))
         return -2;
     if (hipMalloc(&s->dig, draco_gemmh_x_bytes(cap, ((win + 255) / 256) * 256)) != hipSuccess ||
         hipMalloc(&s->ids, sizeof(int) * c) != hipSuccess)
@@ -1057,7 +1057,7 @@ int enqueue_qchunk(QStack* s, int T, int pos0, hipStream_t st) {
             a.n_vh = g.n_vh;
             a.nhq = QNKH;
             a.nspl = T == 1 ? 1 : draco_gdn_split(false);
-            a.PSS = s->PPSS;
+            a.CV = s->PCV;
             if (draco_gdn_scan_launch(a, st)) return fail(-1, "qwen prefill: scan rejected");
             if (gemm(g.out, s->ON, s->Y)) return -1;
             if (pf_add_rms(s->X, s->Y, g.post_norm, s->Xn, T, QH, QEPS, st)) return fail(-1, "qwen prefill: rms");

@@ -2,8 +2,8 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
-// floats per (token, V head) in GdnArgs::PSS (one per wave of the head's
-// blocks); a split decode step fills 16
+// floats per V head in GdnArgs::PSS; a split decode step fills 16 (one per
+// wave of the head's blocks)
 constexpr int GDN_PSS_STRIDE = 64;
 
 struct GdnArgs {
@@ -30,14 +30,16 @@ struct GdnArgs {
     // then [n_vh] xn.alpha_wt rows, by the in-projection launch); the kernel
     // then reads them instead of dotting h1 with bw / aw itself
     const float* glog;
-    // column split: nspl blocks per V head (1, 2, 4 or 8; 0 = 1).  Above 1
-    // the gated rms runs in a second launch (or in the consumer) and needs
-    // PSS [T][n_vh][GDN_PSS_STRIDE] floats (the waves' partial sums).
+    // column split: nspl blocks per V head (1, 2, 4 or 8; 0 = 1).
     int nspl;
+    // a split scan of several tokens: [T][n_qkv] for its conv outputs (q and
+    // k l2-normalised)
+    float* CV;
+    // a split decode step: [n_vh][GDN_PSS_STRIDE], the waves' partial sums of
+    // squares.  It leaves ON = (o / sqrt(128)) * ssm_norm * silu(z) and the
+    // consumer scales each head by its rms itself (the ssm_out GEMV's GNORM
+    // prologue); defer_gnorm must be set.
     float* PSS;
-    // split only: leave ON = (o / sqrt(128)) * ssm_norm * silu(z) and PSS
-    // for the consumer, which scales each head by its rms itself (the
-    // ssm_out GEMV's GNORM prologue) instead of a k_gdn_gnorm launch
     bool defer_gnorm;
 };
 

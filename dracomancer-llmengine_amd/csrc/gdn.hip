@@ -9,7 +9,10 @@
 //   on = (o/sqrt(128)) * rsqrt(mean(o^2)+1e-6) * ssm_norm * silu(z)
 // S is [k][v] (row k), 128 x 128 fp32 per V head.
 //
-// Mapping: the 128 columns of a V head's state are split over NSPL blocks
+// Scans of several tokens run in three launches (k_gdn_conv, k_gdn_chain,
+// k_gdn_rms below), one token (and a split setting of 1) in one:
+//
+// k_gdn_scan: the 128 columns of a V head's state are split over NSPL blocks
 // of NW waves (grid n_vh x NSPL); every block keeps its columns of the state
 // in registers for the whole scan.  Wave w of split sp owns CPW = 128 /
 // (NSPL NW) columns, v = CPW (sp NW + w) + v_lo; lane (v_lo = lane / KQ,
@@ -21,20 +24,17 @@
 // tid + r * threads (q and k of head j in every block: the l2 norms need
 // them whole; v only for the block's columns), the tails in registers; only
 // the block that owns a channel writes its tail back (q/k channels: the last
-// block of the head's readers to count itself in g_qk_cnt).  The l2 norms reduce across the block's waves
-// through LDS.  The gated rms needs all 128 columns of a head: with one
-// block per head (NW = 8) it is finished in the block; split across blocks,
-// each wave writes its columns' o / sqrt(128) to ON and the sum of their
-// squares to a partial buffer, and k_gdn_gnorm applies the rms, the norm
-// weight and the gate in place.  Results agree with the reference to fp32
-// rounding: the per-column sums are split in KQ chunks and the l2 / rms
-// sums use a tree.
-//
-// The split spreads each head's 64 KB of state over NSPL CUs (the state load
-// and store at the ends of a launch run NSPL-wide) and gives a long scan one
-// in-block barrier per token fewer with fewer waves behind each (the rms
-// needs none when split); the defaults below are the measured best.
+// block of the head's readers to count itself in g_qk_cnt).  The l2 norms
+// reduce across the block's waves through LDS.  The gated rms needs all 128
+// columns of a head: with one block per head (NW = 8) it is finished in the
+// block; split across blocks (the decode step), each wave writes its columns'
+// o / sqrt(128) * ssm_norm * silu(z) and the sum of their squares, and the
+// consumer applies the rms.  Results agree with the reference to fp32
+// rounding: the per-column sums are split in KQ chunks and the l2 / rms sums
+// use a tree.
 #include <hip/hip_runtime.h>
+
+#include <type_traits>
 
 #include "dev_common.h"
 #include "gdn.h"
@@ -309,9 +309,9 @@ __global__ __launch_bounds__(64 * NW) void k_gdn_scan(const GdnArgs a) {
             const float inv2 = 1.f / sqrtf(ms2 / SV + EPS);
             if (kq == 0) a.ON[(size_t)t * n_vh * SV + (size_t)h * SV + v] = o * inv2 * nw * silu(z);
         } else {
-            // o / sqrt(128) and this wave's sum of squares; k_gdn_gnorm finishes
-            // (deferred: o * ssm_norm * silu(z), and the consumer applies the rms)
-            if (kq == 0) a.ON[(size_t)t * n_vh * SV + (size_t)h * SV + v] = a.defer_gnorm ? o * nw * silu(z) : o;
+            // o / sqrt(128) * ssm_norm * silu(z) and this wave's sum of squares;
+            // the consumer applies the rms
+            if (kq == 0) a.ON[(size_t)t * n_vh * SV + (size_t)h * SV + v] = o * nw * silu(z);
             if (lane == 0) a.PSS[((size_t)t * n_vh + h) * GDN_PSS_STRIDE + sp * NW + w] = o2;
         }
         lds_barrier();  // cq/ck/cv/red/ored are rewritten by the next token
@@ -461,20 +461,208 @@ __global__ __launch_bounds__(64 * NW) void k_gdn_dec(float* __restrict__ pS, con
         }
 }
 
-// The gated rms of split scans, in place: for token t and V head h,
-// ON[t][h][v] = o * rsqrt(sum of the NP wave partials / 128 + eps) *
-// ssm_norm[v] * silu(Z[t][h][v]), the reference's order (src/m6_layer.c:
-// 320-331).  Block (t, h), 128 threads.
-template <int NP>
-__global__ __launch_bounds__(128) void k_gdn_gnorm(const GdnArgs a) {
-    const int t = blockIdx.x, h = blockIdx.y, v = threadIdx.x;
-    const float* ps = a.PSS + ((size_t)t * a.n_vh + h) * GDN_PSS_STRIDE;
-    float ms2 = 0.f;
+// Scans of several tokens.  A token's recurrence (delta rule) is a chain
+// through the state; everything else is not: k_gdn_conv forms the conv + silu
+// of all tokens and the l2-normalised q and k first, k_gdn_chain then runs
+// the chain alone, and k_gdn_rms the gated rms of all tokens after it.  The
+// chain of one token is bound by its latency (one wave per SIMD): 8 rows a
+// lane instead of 16 halve the dependent multiply-adds, the waves never wait
+// for each other inside a 16-token tile, and the next tile's q, k and v come
+// into LDS meanwhile.  64 tokens of 32 V heads: 22.5 us in three launches
+// (4.7 + 14.4 + 4.4 under the profiler; 0.155 us a token in the chain, half
+// of it VALU issue), 256 tokens 63 us; with conv, norms and rms inside the
+// token loop (three block barriers a token) 71 and 269 us.
+
+// conv + silu of CONV_T tokens' channels of one 128-channel head per wave
+// (q heads, k heads, V heads in channel order); q and k rows l2-normalised.
+// Lane l: channels 2 l, 2 l + 1.
+constexpr int CONV_T = 4;
+__global__ __launch_bounds__(256) void k_gdn_conv(const GdnArgs a) {
+    const int lane = threadIdx.x & 63, hd = blockIdx.y * 4 + (threadIdx.x >> 6);
+    if (hd >= 2 * a.nhq + a.n_vh) return;
+    const int c = hd * SV + 2 * lane, t0 = blockIdx.x * CONV_T, T = a.T;
+    const float4 wa = ld4(a.conv + (size_t)c * 4), wb = ld4(a.conv + (size_t)c * 4 + 4);
+    float2 x[CONV_T + 3];
 #pragma unroll
-    for (int q = 0; q < NP; q++) ms2 += ps[q];
-    const float inv2 = 1.f / sqrtf(ms2 / SV + EPS);
-    const size_t i = (size_t)t * a.n_vh * SV + (size_t)h * SV + v;
-    a.ON[i] = a.ON[i] * inv2 * a.ssm_norm[v] * silu(a.Z[i]);
+    for (int i = 0; i < CONV_T + 3; i++) {
+        const int t = t0 + i - 3;
+        if (t < 0) {  // the history before this call
+            x[i].x = a.tail[(size_t)c * 3 + 3 + t];
+            x[i].y = a.tail[(size_t)c * 3 + 6 + t];
+        } else {
+            x[i] = *reinterpret_cast<const float2*>(a.QKV + (size_t)(t < T ? t : T - 1) * a.n_qkv + c);
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < CONV_T; i++) {
+        if (t0 + i >= T) break;
+        float2 y;
+        y.x = silu(wa.x * x[i].x + wa.y * x[i + 1].x + wa.z * x[i + 2].x + wa.w * x[i + 3].x);
+        y.y = silu(wb.x * x[i].y + wb.y * x[i + 1].y + wb.z * x[i + 2].y + wb.w * x[i + 3].y);
+        if (hd < 2 * a.nhq) {
+            const float n = sqrtf(wave_sum(y.x * y.x + y.y * y.y));
+            const float in = 1.f / (n > EPS ? n : EPS);
+            y.x *= in;
+            y.y *= in;
+        }
+        *reinterpret_cast<float2*>(a.CV + (size_t)(t0 + i) * a.n_qkv + c) = y;
+    }
+}
+
+// The delta rule over T tokens.  Block (V head, sp) of NW waves owns 4 NW
+// columns: lane (vl = lane / 16, kq = lane % 16) of wave w holds rows 4 kq ..
+// 4 kq + 3 and 64 + 4 kq .. of column 4 NW sp + 4 w + vl, so a wave's reads of
+// a token's k and q are 16 consecutive float4.  Tiles of CH_T tokens, two in
+// LDS; the o of a tile are reduced over the lanes and stored together.  Also shifts the conv history (k_gdn_conv has read it).
+constexpr int CH_T = 16;
+template <int NW>
+__global__ __launch_bounds__(64 * NW) void k_gdn_chain(const GdnArgs a) {
+    constexpr int NT = 64 * NW, NC = 4 * NW, QK4 = CH_T * 2 * SV / 4 / NT;  // float4 of q and k per thread and tile
+    constexpr int V4 = CH_T * NC / 4;                                        // float4 of v per tile
+    static_assert(V4 <= NT && 2 * CH_T <= NT, "tile loads");
+    __shared__ float4 lqk[2][CH_T * 2 * SV / 4];  // per token: k (32 float4), q
+    __shared__ float4 lv[2][V4];
+    __shared__ float lgb[2][2 * CH_T];  // g, b of a token
+    const int h = blockIdx.x, sp = blockIdx.y, tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    const int n_qkv = a.n_qkv, n_vh = a.n_vh, T = a.T, nhq = a.nhq, j = h % nhq;
+    const int vl = lane >> 4, kq = lane & 15, vloc = 4 * w + vl, v = NC * sp + vloc;
+    float4 rqk[QK4], rv;
+    float rgb;
+    auto fetch = [&](int t0) {
+#pragma unroll
+        for (int i = 0; i < QK4; i++) {
+            const int e = tid + i * NT, t = t0 + (e >> 6), q = (e >> 5) & 1, c = e & 31;
+            rqk[i] = ld4(a.CV + (size_t)(t < T ? t : T - 1) * n_qkv + (q ? j : nhq + j) * SV + 4 * c);
+        }
+        {
+            const int e = tid < V4 ? tid : V4 - 1, t = t0 + e / NW, c = e % NW;
+            rv = ld4(a.CV + (size_t)(t < T ? t : T - 1) * n_qkv + (2 * nhq + h) * SV + NC * sp + 4 * c);
+        }
+        {
+            const int e = tid < 2 * CH_T ? tid : 0, t = t0 + (e >> 1);
+            rgb = (e & 1 ? a.B : a.G)[(size_t)(t < T ? t : T - 1) * n_vh + h];
+        }
+    };
+    auto stash = [&](int b) {
+#pragma unroll
+        for (int i = 0; i < QK4; i++) lqk[b][tid + i * NT] = rqk[i];
+        if (tid < V4) lv[b][tid] = rv;
+        if (tid < 2 * CH_T) lgb[b][tid] = rgb;
+    };
+    fetch(0);
+    float* Sh = a.S + (size_t)h * SV * SV + v;
+    float s[8];
+#pragma unroll
+    for (int i = 0; i < 8; i++) s[i] = Sh[(size_t)((i >> 2) * 64 + 4 * kq + (i & 3)) * SV];
+    // the conv history of this thread's channels
+    for (int c = (sp * n_vh + h) * NT + tid; c < n_qkv; c += gridDim.x * gridDim.y * NT) {
+        float n[3];
+#pragma unroll
+        for (int i = 0; i < 3; i++)
+            n[i] = T - 3 + i >= 0 ? a.QKV[(size_t)(T - 3 + i) * n_qkv + c] : a.tail[(size_t)c * 3 + T + i];
+#pragma unroll
+        for (int i = 0; i < 3; i++) a.tail[(size_t)c * 3 + i] = n[i];
+    }
+    const float scale = 1.f / sqrtf((float)SV);
+    stash(0);
+    // the state has arrived before the loop (a wait for it inside would also
+    // wait for the next tile's loads)
+#pragma unroll
+    for (int i = 0; i < 8; i++) asm volatile("" : "+v"(s[i]));
+    lds_barrier();
+    for (int t0 = 0, b = 0; t0 < T; t0 += CH_T, b ^= 1) {
+        const bool more = t0 + CH_T < T;
+        if (more) fetch(t0 + CH_T);
+        const int nt = T - t0 < CH_T ? T - t0 : CH_T;
+        const float4* const qk = lqk[b] + kq;
+        const float* vv = reinterpret_cast<const float*>(lv[b]) + vloc;
+        const float2* gb = reinterpret_cast<const float2*>(lgb[b]);
+        float op[CH_T];  // this lane's part of every token's o
+        auto token = [&](const float4& k0, const float4& k1, const float4& q0, const float4& q1, float vt, float2 gbt) {
+            const float kk[8] = {k0.x, k0.y, k0.z, k0.w, k1.x, k1.y, k1.z, k1.w};
+            const float qq[8] = {q0.x, q0.y, q0.z, q0.w, q1.x, q1.y, q1.z, q1.w};
+#pragma unroll
+            for (int i = 0; i < 8; i++) s[i] *= gbt.x;
+            float sa = s[0] * kk[0], sb = s[4] * kk[4];
+#pragma unroll
+            for (int i = 1; i < 4; i++) {
+                sa = __builtin_fmaf(s[i], kk[i], sa);
+                sb = __builtin_fmaf(s[4 + i], kk[4 + i], sb);
+            }
+            const float d = (vt - group_sum<16>(sa + sb)) * gbt.y;
+#pragma unroll
+            for (int i = 0; i < 8; i++) s[i] = __builtin_fmaf(kk[i], d, s[i]);
+            float oa = s[0] * qq[0], ob = s[4] * qq[4];
+#pragma unroll
+            for (int i = 1; i < 4; i++) {
+                oa = __builtin_fmaf(s[i], qq[i], oa);
+                ob = __builtin_fmaf(s[4 + i], qq[4 + i], ob);
+            }
+            return oa + ob;
+        };
+        if (nt == CH_T) {
+            // a token's operands leave LDS while the token before runs
+            float4 n0 = qk[0], n1 = qk[16], n2 = qk[32], n3 = qk[48];
+            float nv = vv[0];
+            float2 ngb = gb[0];
+#pragma unroll
+            for (int t = 0; t < CH_T; t++) {
+                const float4 k0 = n0, k1 = n1, q0 = n2, q1 = n3;
+                const float vt = nv;
+                const float2 gbt = ngb;
+                if (t + 1 < CH_T) {
+                    n0 = qk[64 * t + 64], n1 = qk[64 * t + 80], n2 = qk[64 * t + 96], n3 = qk[64 * t + 112];
+                    nv = vv[NC * (t + 1)];
+                    ngb = gb[t + 1];
+                }
+                __builtin_amdgcn_sched_barrier(0);
+                op[t] = token(k0, k1, q0, q1, vt, gbt);
+            }
+        } else {
+#pragma unroll
+            for (int t = 0; t < CH_T; t++)
+                op[t] = t < nt ? token(qk[64 * t], qk[64 * t + 16], qk[64 * t + 32], qk[64 * t + 48], vv[NC * t], gb[t])
+                               : 0.f;
+        }
+        // reduce-scatter over the 16 lanes of a column: lane kq ends with
+        // token kq's o (15 exchanges for 16 tokens)
+        auto halve = [&](auto mc) {
+            constexpr int m = decltype(mc)::value;
+            const bool up = kq & m;
+#pragma unroll
+            for (int t = 0; t < m; t++) {
+                const float keep = up ? op[t + m] : op[t], give = up ? op[t] : op[t + m];
+                op[t] = keep + lane_flip(give, m);
+            }
+        };
+        halve(std::integral_constant<int, 8>{});
+        halve(std::integral_constant<int, 4>{});
+        halve(std::integral_constant<int, 2>{});
+        halve(std::integral_constant<int, 1>{});
+        if (kq < nt) a.ON[(size_t)(t0 + kq) * n_vh * SV + (size_t)h * SV + v] = op[0] * scale;
+        if (more) {
+            stash(b ^ 1);  // every wave read it last before the previous barrier
+            lds_barrier();
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < 8; i++) Sh[(size_t)((i >> 2) * 64 + 4 * kq + (i & 3)) * SV] = s[i];
+}
+
+// Gated rms of a scan's outputs: ON = ON * rsqrt(mean ON^2 + eps) * ssm_norm *
+// silu(Z), the reference's order (src/m6_layer.c:320-331).  One wave per
+// (token, V head).
+__global__ __launch_bounds__(256) void k_gdn_rms(const GdnArgs a) {
+    const int lane = threadIdx.x & 63, t = blockIdx.x, h = blockIdx.y * 4 + (threadIdx.x >> 6);
+    if (h >= a.n_vh) return;
+    const size_t i = ((size_t)t * a.n_vh + h) * SV + 2 * lane;
+    const float2 o = *reinterpret_cast<const float2*>(a.ON + i), z = *reinterpret_cast<const float2*>(a.Z + i),
+                 nw = *reinterpret_cast<const float2*>(a.ssm_norm + 2 * lane);
+    const float inv = 1.f / sqrtf(wave_sum(o.x * o.x + o.y * o.y) / SV + EPS);
+    float2 y;
+    y.x = o.x * inv * nw.x * silu(z.x);
+    y.y = o.y * inv * nw.y * silu(z.y);
+    *reinterpret_cast<float2*>(a.ON + i) = y;
 }
 
 // A split decode step leaves NSPL * NW = 16 partials (the ssm_out GEMV's
@@ -484,53 +672,53 @@ int g_dec_waves = 2;
 
 template <bool DEC>
 int launch_scan(const GdnArgs& a, int nspl, hipStream_t st) {
-    if (nspl > 1 && !a.PSS) return -1;
-    const dim3 g(a.n_vh, nspl);
-    int np = 16;
-    if (DEC && nspl == 8 && a.glog && g_dec_waves) {
-        // the barrier-free decode step: 16 waves per V head in blocks of 1 or 2
-        if (g_dec_waves == 1)
-            hipLaunchKernelGGL(k_gdn_dec<1>, dim3(a.n_vh, 16), dim3(64), 0, st, a.S, a.conv, a.tail, a.QKV, a.glog,
-                               a.nhq, a.n_vh, a.Z, a);
-        else
-            hipLaunchKernelGGL(k_gdn_dec<2>, dim3(a.n_vh, 8), dim3(128), 0, st, a.S, a.conv, a.tail, a.QKV, a.glog,
-                               a.nhq, a.n_vh, a.Z, a);
-    } else if (DEC || nspl == 1) {
-        switch (nspl) {
-        case 1: hipLaunchKernelGGL((k_gdn_scan<DEC, 8, 1>), g, dim3(512), 0, st, a); return 0;
-        case 2: hipLaunchKernelGGL((k_gdn_scan<DEC, 8, 2>), g, dim3(512), 0, st, a); break;
-        case 4: hipLaunchKernelGGL((k_gdn_scan<DEC, 4, 4>), g, dim3(256), 0, st, a); break;
-        case 8: hipLaunchKernelGGL((k_gdn_scan<DEC, 2, 8>), g, dim3(128), 0, st, a); break;
-        default: return -1;
-        }
-    } else {
-        switch (nspl) {
-        case 2: hipLaunchKernelGGL((k_gdn_scan<DEC, 8, 2>), g, dim3(512), 0, st, a); np = 16; break;
-        case 4: hipLaunchKernelGGL((k_gdn_scan<DEC, 8, 4>), g, dim3(512), 0, st, a); np = 32; break;
-        case 8: hipLaunchKernelGGL((k_gdn_scan<DEC, 8, 8>), g, dim3(512), 0, st, a); np = 64; break;
-        default: return -1;
-        }
+    // (two tokens: one launch 8.7 us, three 9.2; four: 12.1 against 10.2)
+    if (nspl == 1 || (!DEC && a.T <= 2)) {
+        hipLaunchKernelGGL((k_gdn_scan<DEC, 8, 1>), dim3(a.n_vh), dim3(512), 0, st, a);
+        return 0;
     }
-    if (a.defer_gnorm) return np == 16 ? 0 : -1;
-    const dim3 gg(a.T, a.n_vh);
-    if (np == 16) hipLaunchKernelGGL(k_gdn_gnorm<16>, gg, dim3(SV), 0, st, a);
-    else if (np == 32) hipLaunchKernelGGL(k_gdn_gnorm<32>, gg, dim3(SV), 0, st, a);
-    else hipLaunchKernelGGL(k_gdn_gnorm<64>, gg, dim3(SV), 0, st, a);
-    return 0;
+    const dim3 g(a.n_vh, nspl);
+    if constexpr (DEC) {
+        // the consumer finishes the gated rms (16 partials per head)
+        if (!a.PSS || !a.defer_gnorm) return -1;
+        if (nspl == 8 && a.glog && g_dec_waves) {
+            // the barrier-free decode step: 16 waves per V head in blocks of 1 or 2
+            if (g_dec_waves == 1)
+                hipLaunchKernelGGL(k_gdn_dec<1>, dim3(a.n_vh, 16), dim3(64), 0, st, a.S, a.conv, a.tail, a.QKV,
+                                   a.glog, a.nhq, a.n_vh, a.Z, a);
+            else
+                hipLaunchKernelGGL(k_gdn_dec<2>, dim3(a.n_vh, 8), dim3(128), 0, st, a.S, a.conv, a.tail, a.QKV,
+                                   a.glog, a.nhq, a.n_vh, a.Z, a);
+            return 0;
+        }
+        switch (nspl) {
+        case 2: hipLaunchKernelGGL((k_gdn_scan<true, 8, 2>), g, dim3(512), 0, st, a); return 0;
+        case 4: hipLaunchKernelGGL((k_gdn_scan<true, 4, 4>), g, dim3(256), 0, st, a); return 0;
+        case 8: hipLaunchKernelGGL((k_gdn_scan<true, 2, 8>), g, dim3(128), 0, st, a); return 0;
+        }
+        return -1;
+    } else {
+        if (!a.CV || a.defer_gnorm || (nspl != 2 && nspl != 4 && nspl != 8)) return -1;
+        hipLaunchKernelGGL(k_gdn_conv, dim3((a.T + CONV_T - 1) / CONV_T, (2 * a.nhq + a.n_vh + 3) / 4), dim3(256), 0,
+                           st, a);
+        if (nspl == 2) hipLaunchKernelGGL(k_gdn_chain<16>, g, dim3(1024), 0, st, a);
+        else if (nspl == 4) hipLaunchKernelGGL(k_gdn_chain<8>, g, dim3(512), 0, st, a);
+        else hipLaunchKernelGGL(k_gdn_chain<4>, g, dim3(256), 0, st, a);
+        hipLaunchKernelGGL(k_gdn_rms, dim3(a.T, (a.n_vh + 3) / 4), dim3(256), 0, st, a);
+        return 0;
+    }
 }
 
 // Measured on MI355X (configs[4] heads, 32 V heads, graph-replayed): the
 // decode step with its gates (kernel alone) takes 8.3 us in one block of 8
 // waves per head, split 4 ways 6.2 us in blocks of 2 waves, 5.8 in blocks of
 // 4 (7.3 of 8), split 8 ways 5.9 in blocks of 4; the split's gated rms then
-// costs 0.5 us in the ssm_out GEMV's prologue (a k_gdn_gnorm launch would
+// costs 0.5 us in the ssm_out GEMV's prologue (a launch of its own would
 // cost more than the split saves): the 48-layer configs[4] stack decodes at
 // 974 tok/s split 4 (2-wave blocks) against 922 unsplit, 964 split 4 in
-// 4-wave blocks and 998 split 8 in 2-wave blocks (same box, +-2%).  A 64-token scan (the kernel
-// alone) takes 1.43 us/token in 2 blocks of 4 waves per head, 1.09 in 8
-// blocks of 4 waves, 1.17 / 1.00 / 0.96 in 2 / 4 / 8 blocks of 8 waves
-// (more lanes per column: shorter per-lane chains, every wave busy on its
-// SIMD) and 1.39 / 1.27 in 2 / 4 blocks of 16 waves.
+// 4-wave blocks and 998 split 8 in 2-wave blocks (same box, +-2%).  A scan of
+// 64 tokens takes 22.5 us split 8 (blocks of 4 waves: one wave per SIMD at 32
+// V heads), 25.9 split 4 (8 waves), 114 unsplit.
 int g_split_dec = 8;
 int g_split_scan = 8;
 

@@ -412,7 +412,7 @@ __global__ __launch_bounds__(64 * NW) void k_dq(const float* __restrict__ ax, co
         }
         if constexpr (NORM == 2) {
             // GNORM (src/m6_layer.c:320-331): the group's 16 partial sums in
-            // order (as k_gdn_gnorm), x = (o * norm_w * silu(z)) * rsqrt(.)
+            // order (as k_gdn_rms), x = (o * norm_w * silu(z)) * rsqrt(.)
             const float4 p0 = pv0[q], p1 = pv1[q], p2 = pv2[q], p3 = pv3[q];
             float ms2 = 0.f;
             ms2 += p0.x; ms2 += p0.y; ms2 += p0.z; ms2 += p0.w;

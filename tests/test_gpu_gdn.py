@@ -131,3 +131,17 @@ def test_gdn_scan_column_split(hip, oracle, split, T):
     assert rel_err(ON, ONo) <= TOL
     assert rel_err(S2, So) <= TOL
     assert np.array_equal(tail2, tailo)
+
+
+@pytest.mark.parametrize("T", [3, 15, 16, 17, 33])
+def test_gdn_scan_tile_edges(hip, oracle, T):
+    """The tiled scan at a tile's edges: shorter than the conv (its history is
+    then part old, part new), one token short of a 16-token tile, whole tiles
+    and remainders, with V heads that leave a block of four part empty."""
+    n_vh, nhq = 6, 3
+    n_qkv, QKV, Z, B, G, conv, ssm_norm, tail, S = gg.gdn_inputs(T, n_vh, nhq, 60 + T)
+    ON, S2, tail2 = scan(hip, T, n_qkv, n_vh, QKV, Z, B, G, conv, ssm_norm, tail, S)
+    ONo, So, tailo = scan_oracle(oracle, T, n_qkv, n_vh, QKV, Z, B, G, conv, ssm_norm, tail, S)
+    assert rel_err(ON, ONo) <= TOL
+    assert rel_err(S2, So) <= TOL
+    assert np.array_equal(tail2, tailo)
