@@ -17,6 +17,8 @@
 // online form, exact in exact arithmetic).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include "dev_common.h"
 #include "embed_dev.h"
 #include "formats.h"
@@ -144,287 +146,232 @@ __global__ __launch_bounds__(256) void k_pf_rope_append(float* __restrict__ Q, c
     }
 }
 
-// Causal attention of a chunk, split over the key rows.  Block (g, qt, s):
-// kv head g, queries qt*64 .. qt*64+63 of the chunk (lane = query), key split
-// s of rows [0, row0 + last query of the tile].  Wave j is q head g*rep + j;
-// the rep waves share the K / V rows, staged in LDS 64 rows at a time and
-// read by every lane at the same address (broadcast).  Keys go in groups of
-// 16: scores, one online-softmax rescale, then P.V.  Writes the unnormalised
-// (o[HD], m, l) of (head, query, split) for k_pf_merge.
-constexpr int PF_QT = 64, PF_KT = 64, PF_KG = 16;
-
-// K and V rows [kb, kb + nr) of kv head g into LDS (row-major, HD wide):
-// each thread requests up to 4 float4s of each array together (clamped
-// index; the stores skip the clamped ones), so a tile costs one memory round
-// trip per 4 float4s per thread instead of one per float4.
-template <int HD>
-__device__ __forceinline__ void stage_kv(float* Ks, float* Vs, const float* __restrict__ kc,
-                                         const float* __restrict__ vc, int kb, int nr, int KD, int g) {
-    constexpr int SB = 4;
-    const int n = nr * (HD / 4), nt = blockDim.x, tid = threadIdx.x;
-    for (int b0 = 0; b0 < n; b0 += SB * nt) {
-        float4 kv[SB], vv[SB];
-#pragma unroll
-        for (int u = 0; u < SB; u++) {
-            const int i = b0 + tid + u * nt, ic = i < n ? i : n - 1;
-            const int r = ic / (HD / 4), c = 4 * (ic % (HD / 4));
-            kv[u] = ld4(kc + (size_t)(kb + r) * KD + g * HD + c);
-            vv[u] = ld4(vc + (size_t)(kb + r) * KD + g * HD + c);
-        }
-#pragma unroll
-        for (int u = 0; u < SB; u++) {
-            const int i = b0 + tid + u * nt;
-            if (i < n) {
-                const int r = i / (HD / 4), c = 4 * (i % (HD / 4));
-                *reinterpret_cast<float4*>(Ks + r * HD + c) = kv[u];
-                *reinterpret_cast<float4*>(Vs + r * HD + c) = vv[u];
-            }
-        }
-    }
-}
+// Causal attention of a chunk on the fp32 matrix instructions (16x16x4),
+// split over the key rows: products and sums stay fp32, as a VALU dot's.
+// Wave (16 queries of one q head) x tiles of 32 keys:
+//   S^T = K Q^T   A = K rows (LDS), B = the queries (registers); lane (n, u) =
+//                 (lane & 15, lane >> 4) gets keys 4u .. 4u+3 of query n
+//   O^T += V^T P^T  the lane's scores are already the B operand of the step
+//                 whose four keys are 4u + r, so P never leaves its registers;
+//                 A row n of dim tile dt is dim 64 dg + 4 n + dt: one 16-byte
+//                 LDS read feeds four products, and a lane's outputs come out
+//                 as float4
+// with the online softmax per 32 keys (a query's keys lie in four lanes: one
+// max over them a tile, the sum only at the end).  A block is `hg` q heads of
+// one kv head (a group's waves share the staged rows) x blockDim / 64 / hg
+// query tiles; blockIdx.x = kv head * head groups + group.  K and V tiles are
+// double-buffered in LDS, rows padded by 4 floats (conflict-free for both
+// reads).  Writes the unnormalised (o[HD], m, l) of (head, query, split) for
+// the merge kernels.
+//
+// Bound by the matrix instructions' issue on whole chunks (HD products of 32
+// cycles per 32 keys and wave).  Per launch, average over a prompt: 256-token
+// chunks of 32 heads of 64 up to 960 keys 51 -> 19.3 us, 75 tokens at 275
+// keys 36 -> 8.3; 191 tokens of 32 heads of 128 634 -> 16; 256-token chunks of
+// 16 heads of 256 up to 2000 keys 107 -> 60 (a VALU lane per query, whose q
+// and o of 128 dims spilled, before).
+constexpr int PF_QT = 16, PF_KT = 32;
+constexpr int PF_WAVES = 2048;  // waves a launch splits the keys for (launch_attn)
+typedef float v4f __attribute__((ext_vector_type(4)));
 
 template <int HD>
 __global__ __launch_bounds__(512) void k_pf_attn(const float* __restrict__ Q, const float* __restrict__ kc,
                                                  const float* __restrict__ vc, float* __restrict__ part, int row0,
-                                                 int T, int NH, int NKV, int nspl, float scale) {
-    extern __shared__ __align__(16) float sm[];
-    float* Ks = sm;
-    float* Vs = sm + PF_KT * HD;
-    const int g = blockIdx.x, qt = blockIdx.y, s = blockIdx.z;
-    const int tid = threadIdx.x, lane = tid & 63, j = tid >> 6;
-    const int rep = NH / NKV, h = g * rep + j, KD = NKV * HD, QD = NH * HD;
-    const int t = qt * PF_QT + lane, qrow = row0 + t;
-    const bool live = t < T;
-    const int kend = row0 + min(T, (qt + 1) * PF_QT);
-    const int chunk = (kend + nspl - 1) / nspl;
-    const int k0 = min(kend, s * chunk), k1 = min(kend, k0 + chunk);
-    float q[HD], o[HD];
-    const int tq = live ? t : 0;  // a query past the chunk reads row 0 and discards it
+                                                 int T, int NH, int NKV, int nspl, int hg, float scale) {
+    constexpr int RS = HD + 4, NL = HD / 32;  // LDS row, float4 of a tile per thread of a 256-thread block
+    extern __shared__ __align__(16) float sm[];  // [2][K 32 rows, V 32 rows][RS]
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, n = lane & 15, u = lane >> 4, NT = blockDim.x;
+    const int rep = NH / NKV, ngrp = (rep + hg - 1) / hg, qw = (NT >> 6) / hg;
+    const int g = blockIdx.x / ngrp, j = (blockIdx.x % ngrp) * hg + w % hg, qt = blockIdx.y * qw + w / hg;
+    const int h = g * rep + min(j, rep - 1), KD = NKV * HD, QD = NH * HD;
+    const int t = qt * PF_QT + n, qrow = row0 + t;
+    const bool live = t < T && j < rep;
+    const int kend = row0 + min(T, ((int)blockIdx.y + 1) * qw * PF_QT);
+    const int chunk = ((kend + nspl - 1) / nspl + PF_KT - 1) / PF_KT * PF_KT;
+    const int k0 = min(kend, (int)blockIdx.z * chunk), k1 = min(kend, k0 + chunk);
+    // this wave's queries end here (a wave without any computes nothing)
+    const int wend = j < rep && qt * PF_QT < T ? row0 + min(T, (qt + 1) * PF_QT) : 0;
+    float4 q[HD / 16];
+    const int tq = min(t, T - 1);  // a query past the chunk reads the last row and is discarded
 #pragma unroll
-    for (int d = 0; d < HD; d += 4) {
-        const float4 v = ld4(Q + (size_t)tq * QD + h * HD + d);
-        q[d] = live ? v.x : 0.f; q[d + 1] = live ? v.y : 0.f; q[d + 2] = live ? v.z : 0.f; q[d + 3] = live ? v.w : 0.f;
-        o[d] = o[d + 1] = o[d + 2] = o[d + 3] = 0.f;
-    }
+    for (int i = 0; i < HD / 16; i++) q[i] = ld4(Q + (size_t)tq * QD + h * HD + 16 * i + 4 * u);
+    float4 rg[NL];
+    auto fetch = [&](const float* __restrict__ src, int kb) {  // rows past the split repeat its last one (masked)
+#pragma unroll
+        for (int i = 0; i < NL; i++) {
+            const int e = min(tid + i * NT, PF_KT * HD / 4 - 1), r = e / (HD / 4), c = 4 * (e % (HD / 4));
+            rg[i] = ld4(src + (size_t)min(kb + r, k1 - 1) * KD + g * HD + c);
+        }
+    };
+    auto stash = [&](float* dst) {
+#pragma unroll
+        for (int i = 0; i < NL; i++) {
+            const int e = tid + i * NT, r = e / (HD / 4), c = 4 * (e % (HD / 4));
+            if (e < PF_KT * HD / 4) *reinterpret_cast<float4*>(dst + r * RS + c) = rg[i];
+        }
+    };
+    v4f o[HD / 16];
+#pragma unroll
+    for (int i = 0; i < HD / 16; i++) o[i] = (v4f){0.f, 0.f, 0.f, 0.f};
     float m = -INFINITY, l = 0.f;
-    for (int kb = k0; kb < k1; kb += PF_KT) {
-        const int nr = min(PF_KT, k1 - kb);
-        stage_kv<HD>(Ks, Vs, kc, vc, kb, nr, KD, g);
-        __syncthreads();
-        for (int c0 = 0; c0 < nr; c0 += PF_KG) {
-            const int ng = min(PF_KG, nr - c0);
-            float sc[PF_KG];
+    if (k0 < k1) {
+        fetch(kc, k0);
+        stash(sm);
+        fetch(vc, k0);
+        stash(sm + PF_KT * RS);
+    }
+    // the queries have arrived before the loop (a wait for them inside would
+    // also wait for the next tile)
+#pragma unroll
+    for (int i = 0; i < HD / 16; i++) asm volatile("" : "+v"(q[i].x), "+v"(q[i].y), "+v"(q[i].z), "+v"(q[i].w));
+    lds_barrier();
+    int b = 0;
+    for (int kb = k0; kb < k1; kb += PF_KT, b ^= 1) {
+        const bool more = kb + PF_KT < k1;
+        // the next tile's K arrives during the scores, its V during P V (one
+        // set of registers); the other buffer was last read before the barrier
+        if (more) fetch(kc, kb + PF_KT);
+        const float* Ks = sm + b * 2 * PF_KT * RS;
+        const float* Vs = Ks + PF_KT * RS;
+        float* const next = sm + (b ^ 1) * 2 * PF_KT * RS;
+        v4f sc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+        if (kb < wend) {
+#pragma unroll
+            for (int i = 0; i < HD / 16; i++) {
+                const float4 ka = ld4(Ks + n * RS + 16 * i + 4 * u), kz = ld4(Ks + (16 + n) * RS + 16 * i + 4 * u);
+                sc[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(ka.x, q[i].x, sc[0], 0, 0, 0);
+                sc[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(kz.x, q[i].x, sc[1], 0, 0, 0);
+                sc[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(ka.y, q[i].y, sc[0], 0, 0, 0);
+                sc[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(kz.y, q[i].y, sc[1], 0, 0, 0);
+                sc[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(ka.z, q[i].z, sc[0], 0, 0, 0);
+                sc[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(kz.z, q[i].z, sc[1], 0, 0, 0);
+                sc[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(ka.w, q[i].w, sc[0], 0, 0, 0);
+                sc[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(kz.w, q[i].w, sc[1], 0, 0, 0);
+            }
+        }
+        if (more) {
+            stash(next);
+            fetch(vc, kb + PF_KT);
+        }
+        if (kb < wend) {
             float cm = -INFINITY;
 #pragma unroll
-            for (int jj = 0; jj < PF_KG; jj++) {
-                sc[jj] = -INFINITY;
-                if (jj < ng) {
-                    const float* kr = Ks + (c0 + jj) * HD;
-                    float acc = 0.f;
+            for (int kt = 0; kt < 2; kt++)
 #pragma unroll
-                    for (int d = 0; d < HD; d += 4) {
-                        const float4 kv = *reinterpret_cast<const float4*>(kr + d);
-                        acc = fmaf(q[d], kv.x, acc);
-                        acc = fmaf(q[d + 1], kv.y, acc);
-                        acc = fmaf(q[d + 2], kv.z, acc);
-                        acc = fmaf(q[d + 3], kv.w, acc);
-                    }
-                    if (live && kb + c0 + jj <= qrow) sc[jj] = acc * scale;
-                    cm = fmaxf(cm, sc[jj]);
+                for (int r = 0; r < 4; r++) {
+                    const int key = kb + 16 * kt + 4 * u + r;
+                    sc[kt][r] = live && key <= qrow && key < k1 ? sc[kt][r] * scale : -INFINITY;
+                    cm = fmaxf(cm, sc[kt][r]);
                 }
-            }
-            const float mn = fmaxf(m, cm);
-            if (mn > -INFINITY) {
-                const float corr = m > -INFINITY ? expf(m - mn) : 0.f;
-                l *= corr;
+            const float mn = fmaxf(m, rows_reduce(cm, OpMax{}));
+            const float corr = m > -INFINITY ? expf(m - mn) : 0.f;
+            l *= corr;
 #pragma unroll
-                for (int d = 0; d < HD; d++) o[d] *= corr;
+            for (int i = 0; i < HD / 16; i++) o[i] *= corr;
 #pragma unroll
-                for (int jj = 0; jj < PF_KG; jj++) {
-                    if (jj < ng) {
-                        const float p = sc[jj] > -INFINITY ? expf(sc[jj] - mn) : 0.f;
-                        l += p;
-                        const float* vr = Vs + (c0 + jj) * HD;
+            for (int kt = 0; kt < 2; kt++)
 #pragma unroll
-                        for (int d = 0; d < HD; d += 4) {
-                            const float4 vv = *reinterpret_cast<const float4*>(vr + d);
-                            o[d] = fmaf(p, vv.x, o[d]);
-                            o[d + 1] = fmaf(p, vv.y, o[d + 1]);
-                            o[d + 2] = fmaf(p, vv.z, o[d + 2]);
-                            o[d + 3] = fmaf(p, vv.w, o[d + 3]);
-                        }
+                for (int r = 0; r < 4; r++) {
+                    const float p = sc[kt][r] > -INFINITY ? expf(sc[kt][r] - mn) : 0.f;
+                    l += p;
+                    const float* vr = Vs + (16 * kt + 4 * u + r) * RS + 4 * n;
+#pragma unroll
+                    for (int dg = 0; dg < HD / 64; dg++) {
+                        const float4 v = ld4(vr + 64 * dg);
+                        o[4 * dg] = __builtin_amdgcn_mfma_f32_16x16x4f32(v.x, p, o[4 * dg], 0, 0, 0);
+                        o[4 * dg + 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(v.y, p, o[4 * dg + 1], 0, 0, 0);
+                        o[4 * dg + 2] = __builtin_amdgcn_mfma_f32_16x16x4f32(v.z, p, o[4 * dg + 2], 0, 0, 0);
+                        o[4 * dg + 3] = __builtin_amdgcn_mfma_f32_16x16x4f32(v.w, p, o[4 * dg + 3], 0, 0, 0);
                     }
                 }
-                m = mn;
-            }
+            m = mn;
         }
-        __syncthreads();
+        if (more) {
+            stash(next + PF_KT * RS);
+            lds_barrier();
+        }
     }
+    l = rows_sum(l);
     if (!live) return;
-    float* pp = part + (((size_t)h * T + t) * nspl + s) * (HD + 2);
+    float* pp = part + (((size_t)h * T + t) * nspl + blockIdx.z) * (HD + 2);
 #pragma unroll
-    for (int d = 0; d < HD; d++) pp[d] = o[d];
-    pp[HD] = m;
-    pp[HD + 1] = l;
-}
-
-// The split merge of one (query, head, dim): M = max_s m_s, then num / den
-// with den = sum_s l_s e^(m_s - M), num = sum_s o_s[d] e^(m_s - M) in split
-// order.  Loads go in batches of 16 splits, all of a batch requested together
-// (clamped split index; the merge skips the clamped ones), instead of one
-// dependent round trip per split.
-__device__ __forceinline__ float pf_merge_one(const float* __restrict__ pp, int HD, int nspl, int d) {
-    constexpr int MB = 16;
-    float M = -INFINITY;
-    for (int s0 = 0; s0 < nspl; s0 += MB) {
-        float mv[MB];
+    for (int dg = 0; dg < HD / 64; dg++)
 #pragma unroll
-        for (int k = 0; k < MB; k++) mv[k] = pp[(size_t)min(s0 + k, nspl - 1) * (HD + 2) + HD];
-#pragma unroll
-        for (int k = 0; k < MB; k++)
-            if (s0 + k < nspl) M = fmaxf(M, mv[k]);
-    }
-    float num = 0.f, den = 0.f;
-    for (int s0 = 0; s0 < nspl; s0 += MB) {
-        float mv[MB], lv[MB], ov[MB];
-#pragma unroll
-        for (int k = 0; k < MB; k++) {
-            const float* q = pp + (size_t)min(s0 + k, nspl - 1) * (HD + 2);
-            mv[k] = q[HD];
-            lv[k] = q[HD + 1];
-            ov[k] = q[d];
-        }
-#pragma unroll
-        for (int k = 0; k < MB; k++) {
-            if (s0 + k >= nspl || mv[k] == -INFINITY) continue;
-            const float e = expf(mv[k] - M);
-            den = fmaf(lv[k], e, den);
-            num = fmaf(ov[k], e, num);
-        }
-    }
-    return num / den;
-}
-
-// out[t][h*HD + d] = sum_s o_s[d] e^(m_s - M) / sum_s l_s e^(m_s - M)
-__global__ __launch_bounds__(256) void k_pf_merge(const float* __restrict__ part, float* __restrict__ O, int T,
-                                                  int NH, int HD, int nspl) {
-    const int t = blockIdx.x, h = blockIdx.y, d = threadIdx.x;
-    if (d >= HD) return;
-    const float* pp = part + ((size_t)h * T + t) * nspl * (HD + 2);
-    O[(size_t)t * NH * HD + h * HD + d] = pf_merge_one(pp, HD, nspl, d);
-}
-
-// Causal chunk attention at head dim 256 (qwen35 full attention, the chunked
-// form of src/m6_layer.c:455-500 that src/qwen35_prefill.py:137-168 runs).
-// Block (g, qt, s): kv head g, queries qt*8 .. qt*8+7 of the chunk, key split
-// s; wave j = q head g*rep + j.  Eight lanes share a query: lane = 8*query +
-// k holds the dims 4*(k + 8*i) .. +3 (i < 8) of q and of the output, so the
-// eight lanes of a query read one 128-byte run of a staged K / V row
-// (conflict-free) and a score is the sum over those eight lanes.  K / V rows
-// are staged in LDS 32 at a time; keys go in groups of 16 (scores, one
-// online-softmax rescale, P.V).  Writes (o[256], m, l) per (head, query,
-// split) for k_pf_merge256.
-constexpr int PF256_QT = 8, PF256_KT = 32;
-
-__global__ __launch_bounds__(1024) void k_pf_attn256(const float* __restrict__ Q, const float* __restrict__ kc,
-                                                     const float* __restrict__ vc, float* __restrict__ part,
-                                                     int row0, int T, int NH, int NKV, int nspl, float scale) {
-    constexpr int HD = 256;
-    __shared__ __align__(16) float Ks[PF256_KT * HD];
-    __shared__ __align__(16) float Vs[PF256_KT * HD];
-    const int g = blockIdx.x, qt = blockIdx.y, s = blockIdx.z;
-    const int tid = threadIdx.x, lane = tid & 63, j = tid >> 6, k = lane & 7;
-    const int rep = NH / NKV, h = g * rep + j, KD = NKV * HD, QD = NH * HD;
-    const int t = qt * PF256_QT + (lane >> 3), qrow = row0 + t;
-    const bool live = t < T;
-    const int kend = row0 + min(T, (qt + 1) * PF256_QT);
-    const int chunk = (kend + nspl - 1) / nspl;
-    const int k0 = min(kend, s * chunk), k1 = min(kend, k0 + chunk);
-    float q[32], o[32];
-    const int tq = live ? t : 0;  // a query past the chunk reads row 0 and discards it
-#pragma unroll
-    for (int i = 0; i < 8; i++) {
-        const float4 v = ld4(Q + (size_t)tq * QD + h * HD + 4 * (k + 8 * i));
-        q[4 * i] = live ? v.x : 0.f; q[4 * i + 1] = live ? v.y : 0.f;
-        q[4 * i + 2] = live ? v.z : 0.f; q[4 * i + 3] = live ? v.w : 0.f;
-        o[4 * i] = o[4 * i + 1] = o[4 * i + 2] = o[4 * i + 3] = 0.f;
-    }
-    float m = -INFINITY, l = 0.f;
-    for (int kb = k0; kb < k1; kb += PF256_KT) {
-        const int nr = min(PF256_KT, k1 - kb);
-        stage_kv<HD>(Ks, Vs, kc, vc, kb, nr, KD, g);
-        __syncthreads();
-        for (int c0 = 0; c0 < nr; c0 += 16) {
-            const int ng = min(16, nr - c0);
-            float sc[16];
-            float cm = -INFINITY;
-#pragma unroll
-            for (int jj = 0; jj < 16; jj++) {
-                float acc = 0.f;
-                if (jj < ng) {
-                    const float* kr = Ks + (c0 + jj) * HD;
-#pragma unroll
-                    for (int i = 0; i < 8; i++) {
-                        const float4 kv = *reinterpret_cast<const float4*>(kr + 4 * (k + 8 * i));
-                        acc = fmaf(q[4 * i], kv.x, acc);
-                        acc = fmaf(q[4 * i + 1], kv.y, acc);
-                        acc = fmaf(q[4 * i + 2], kv.z, acc);
-                        acc = fmaf(q[4 * i + 3], kv.w, acc);
-                    }
-                }
-                acc = group_sum<8>(acc);
-                sc[jj] = (jj < ng && live && kb + c0 + jj <= qrow) ? acc * scale : -INFINITY;
-                cm = fmaxf(cm, sc[jj]);
-            }
-            const float mn = fmaxf(m, cm);
-            if (mn > -INFINITY) {
-                const float corr = m > -INFINITY ? expf(m - mn) : 0.f;
-                l *= corr;
-#pragma unroll
-                for (int d = 0; d < 32; d++) o[d] *= corr;
-#pragma unroll
-                for (int jj = 0; jj < 16; jj++) {
-                    if (jj < ng) {
-                        const float p = sc[jj] > -INFINITY ? expf(sc[jj] - mn) : 0.f;
-                        l += p;
-                        const float* vr = Vs + (c0 + jj) * HD;
-#pragma unroll
-                        for (int i = 0; i < 8; i++) {
-                            const float4 vv = *reinterpret_cast<const float4*>(vr + 4 * (k + 8 * i));
-                            o[4 * i] = fmaf(p, vv.x, o[4 * i]);
-                            o[4 * i + 1] = fmaf(p, vv.y, o[4 * i + 1]);
-                            o[4 * i + 2] = fmaf(p, vv.z, o[4 * i + 2]);
-                            o[4 * i + 3] = fmaf(p, vv.w, o[4 * i + 3]);
-                        }
-                    }
-                }
-                m = mn;
-            }
-        }
-        __syncthreads();
-    }
-    if (!live) return;
-    float* pp = part + (((size_t)h * T + t) * nspl + s) * (HD + 2);
-#pragma unroll
-    for (int i = 0; i < 8; i++)
-        *reinterpret_cast<float4*>(pp + 4 * (k + 8 * i)) = make_float4(o[4 * i], o[4 * i + 1], o[4 * i + 2], o[4 * i + 3]);
-    if (k == 0) {
+        for (int r = 0; r < 4; r++)
+            *reinterpret_cast<float4*>(pp + 64 * dg + 16 * u + 4 * r) =
+                make_float4(o[4 * dg][r], o[4 * dg + 1][r], o[4 * dg + 2][r], o[4 * dg + 3][r]);
+    if (u == 0) {
         pp[HD] = m;
         pp[HD + 1] = l;
     }
 }
 
-// k_pf_merge with the qwen35 output gate: O[t][h*HD + d] *= sigmoid(gate
-// row t, h*gstride_h + d) (the reference's attn * sigmoid(q gate half),
-// src/qwen35_prefill.py:164-166 / src/m6_layer.c:497).
-__global__ __launch_bounds__(256) void k_pf_merge_gate(const float* __restrict__ part, float* __restrict__ O, int T,
-                                                       int NH, int HD, int nspl, const float* __restrict__ gate,
-                                                       int g_row, int g_head) {
-    const int t = blockIdx.x, h = blockIdx.y, d = threadIdx.x;
-    if (d >= HD) return;
+// The split merge of four dims of one (query, head): M = max_s m_s, then
+// num / den with den = sum_s l_s e^(m_s - M), num = sum_s o_s e^(m_s - M) in
+// split order.  Loads go in batches of 8 splits, all of a batch requested
+// together (clamped split index; the merge skips the clamped ones), instead of
+// one dependent round trip per split.
+__device__ __forceinline__ float4 pf_merge4(const float* __restrict__ pp, int HD, int nspl, int d) {
+    constexpr int MB = 8;
+    float M = -INFINITY;
+    float4 num = make_float4(0.f, 0.f, 0.f, 0.f);
+    float den = 0.f;
+    float2 ml[MB];
+    float4 ov[MB];
+    auto load = [&](int s0) {
+#pragma unroll
+        for (int k = 0; k < MB; k++) {
+            const float* q = pp + (size_t)min(s0 + k, nspl - 1) * (HD + 2);
+            ml[k] = *reinterpret_cast<const float2*>(q + HD);
+            ov[k] = ld4(q + d);
+        }
+    };
+    auto add = [&](int s0) {
+#pragma unroll
+        for (int k = 0; k < MB; k++) {
+            if (s0 + k >= nspl || ml[k].x == -INFINITY) continue;
+            const float e = expf(ml[k].x - M);
+            den = fmaf(ml[k].y, e, den);
+            num.x = fmaf(ov[k].x, e, num.x);
+            num.y = fmaf(ov[k].y, e, num.y);
+            num.z = fmaf(ov[k].z, e, num.z);
+            num.w = fmaf(ov[k].w, e, num.w);
+        }
+    };
+    load(0);  // the only batch of up to 8 splits: one round trip
+#pragma unroll
+    for (int k = 0; k < MB; k++) M = fmaxf(M, ml[k].x);
+    for (int s = MB; s < nspl; s++) M = fmaxf(M, pp[(size_t)s * (HD + 2) + HD]);
+    add(0);
+    for (int s0 = MB; s0 < nspl; s0 += MB) {
+        load(s0);
+        add(s0);
+    }
+    return make_float4(num.x / den, num.y / den, num.z / den, num.w / den);
+}
+
+// out[t][h*HD + d] = sum_s o_s[d] e^(m_s - M) / sum_s l_s e^(m_s - M); a
+// thread per four dims (a block per (token, head) of HD threads made
+// 8192 one-wave blocks of a chunk: 9.7 us, now 5.2).  gate (nullable): the qwen35 output
+// gate, O *= sigmoid(gate row t, h*g_head + d) (the reference's attn *
+// sigmoid(q gate half), src/qwen35_prefill.py:164-166 / src/m6_layer.c:497).
+__global__ __launch_bounds__(256) void k_pf_merge(const float* __restrict__ part, float* __restrict__ O, int T,
+                                                  int NH, int HD, int nspl, const float* __restrict__ gate,
+                                                  int g_row, int g_head) {
+    const int i = blockIdx.x * 256 + threadIdx.x, nd = HD / 4;
+    if (i >= T * NH * nd) return;
+    const int d = 4 * (i % nd), h = i / nd % NH, t = i / nd / NH;
     const float* pp = part + ((size_t)h * T + t) * nspl * (HD + 2);
-    const float gv = gate[(size_t)t * g_row + (size_t)h * g_head + d];
-    O[(size_t)t * NH * HD + h * HD + d] = pf_merge_one(pp, HD, nspl, d) * (1.f / (1.f + expf(-gv)));
+    float4 gv;
+    if (gate) gv = ld4(gate + (size_t)t * g_row + (size_t)h * g_head + d);
+    float4 v = pf_merge4(pp, HD, nspl, d);
+    if (gate) {
+        v.x *= 1.f / (1.f + expf(-gv.x));
+        v.y *= 1.f / (1.f + expf(-gv.y));
+        v.z *= 1.f / (1.f + expf(-gv.z));
+        v.w *= 1.f / (1.f + expf(-gv.w));
+    }
+    *reinterpret_cast<float4*>(O + (size_t)t * NH * HD + h * HD + d) = v;
 }
 
 // GDN gates of a chunk (src/qwen35_prefill.py:118-123): for token t and V
@@ -471,7 +418,11 @@ int pf_attn_nsplit(int row0, int T) {
     return n < 1 ? 1 : (n > 64 ? 64 : n);
 }
 
-size_t pf_part_floats(int NH, int T, int HD, int nspl) { return (size_t)NH * T * nspl * (HD + 2); }
+// Enough for every chunk of up to T tokens: launch_attn's splits are at most
+// nspl, and at most PF_WAVES / waves rounded up, with at least NH * T / 16 waves.
+size_t pf_part_floats(int NH, int T, int HD, int nspl) {
+    return std::min((size_t)NH * T * nspl, (size_t)PF_QT * PF_WAVES + (size_t)NH * T) * (HD + 2);
+}
 
 int pf_embed(const uint8_t* base, const DracoLayout& L, const int* ids, int T, float* X, hipStream_t st) {
     if (T < 1) return -1;
@@ -500,34 +451,51 @@ int pf_rope_append(float* Q, const float* K, const float* V, float* kc, float* v
     return 0;
 }
 
+namespace {
+
+// The attention launch of a chunk.  Blocks of 4 to 8 waves: a kv head's q
+// heads (up to 8), and two or four query tiles where the group has fewer than
+// four.  The key rows are split until about PF_WAVES waves run (never finer
+// than pf_attn_nsplit): a split costs a row of partials per query that the
+// merge reads again.  1024 / 2048 / 4096 waves: 22.3 / 19.3 / 18.9 us at head
+// dim 64 (chunks of a 960-token prompt), 92 / 60 / 76 at 256 (2000 tokens).
+template <int HD>
+int launch_attn(const float* Q, const float* kc, const float* vc, float* part, int row0, int T, int NH, int NKV,
+                float scale, hipStream_t st, int* nsplit) {
+    const int rep = NH / NKV, hg = rep < 8 ? rep : 8, qw = hg >= 4 ? 1 : (hg == 1 ? 4 : 2), ngrp = (rep + hg - 1) / hg;
+    const int qb = (T + PF_QT * qw - 1) / (PF_QT * qw), waves = NKV * ngrp * qb * hg * qw;
+    const int nspl = std::min(pf_attn_nsplit(row0, T), (PF_WAVES + waves - 1) / waves);
+    constexpr int lds = sizeof(float) * 2 * 2 * PF_KT * (HD + 4);
+    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_pf_attn<HD>),
+                                                       hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    if (attr != hipSuccess) return -1;
+    hipLaunchKernelGGL(k_pf_attn<HD>, dim3(NKV * ngrp, qb, nspl), dim3(64 * hg * qw), lds, st, Q, kc, vc, part, row0,
+                       T, NH, NKV, nspl, hg, scale);
+    *nsplit = nspl;
+    return 0;
+}
+
+}  // namespace
+
 int pf_attention(const float* Q, const float* kc, const float* vc, float* part, float* O, int row0, int T, int NH,
                  int NKV, int HD, float scale, hipStream_t st) {
     if (T < 1 || !pf_attention_ok(NH, NKV, HD)) return -1;
-    const int nspl = pf_attn_nsplit(row0, T);
-    const dim3 grid(NKV, (T + PF_QT - 1) / PF_QT, nspl), block(64 * (NH / NKV));
-    const size_t lds = sizeof(float) * 2 * PF_KT * HD;
-    if (HD == 64) {
-        hipLaunchKernelGGL(k_pf_attn<64>, grid, block, lds, st, Q, kc, vc, part, row0, T, NH, NKV, nspl, scale);
-    } else {
-        static bool attr = false;
-        if (!attr) {
-            (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&k_pf_attn<128>),
-                                      hipFuncAttributeMaxDynamicSharedMemorySize, 64 * 1024);
-            attr = true;
-        }
-        hipLaunchKernelGGL(k_pf_attn<128>, grid, block, lds, st, Q, kc, vc, part, row0, T, NH, NKV, nspl, scale);
-    }
-    hipLaunchKernelGGL(k_pf_merge, dim3(T, NH), dim3(HD), 0, st, part, O, T, NH, HD, nspl);
+    int nspl = 1;
+    const int rc = HD == 64 ? launch_attn<64>(Q, kc, vc, part, row0, T, NH, NKV, scale, st, &nspl)
+                            : launch_attn<128>(Q, kc, vc, part, row0, T, NH, NKV, scale, st, &nspl);
+    if (rc) return rc;
+    hipLaunchKernelGGL(k_pf_merge, dim3((T * NH * (HD / 4) + 255) / 256), dim3(256), 0, st, part, O, T, NH, HD, nspl,
+                       (const float*)nullptr, 0, 0);
     return 0;
 }
 
 int pf_attention256(const float* Q, const float* kc, const float* vc, float* part, float* O, int row0, int T, int NH,
                     int NKV, float scale, const float* gate, int g_row, int g_head, hipStream_t st) {
     if (T < 1 || NKV < 1 || NH % NKV || NH / NKV > 16 || !gate) return -1;
-    const int nspl = pf_attn_nsplit(row0, T);
-    const dim3 grid(NKV, (T + PF256_QT - 1) / PF256_QT, nspl), block(64 * (NH / NKV));
-    hipLaunchKernelGGL(k_pf_attn256, grid, block, 0, st, Q, kc, vc, part, row0, T, NH, NKV, nspl, scale);
-    hipLaunchKernelGGL(k_pf_merge_gate, dim3(T, NH), dim3(256), 0, st, part, O, T, NH, 256, nspl, gate, g_row, g_head);
+    int nspl = 1;
+    if (launch_attn<256>(Q, kc, vc, part, row0, T, NH, NKV, scale, st, &nspl)) return -1;
+    hipLaunchKernelGGL(k_pf_merge, dim3((T * NH * 64 + 255) / 256), dim3(256), 0, st, part, O, T, NH, 256, nspl, gate,
+                       g_row, g_head);
     return 0;
 }
 

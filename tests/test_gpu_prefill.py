@@ -112,6 +112,39 @@ def test_prefill_head_shapes(oracle, hd, nh, nkv):
     assert rel_err(lg, lr) <= 1e-4
 
 
+@pytest.mark.parametrize("hd,nh,nkv", [(64, 2, 2), (64, 4, 2), (64, 6, 2), (128, 7, 1)])
+def test_prefill_attention_tile_edges(oracle, hd, nh, nkv):
+    """The attention's 16-query and 32-key tiles at their edges: chunks of 33,
+    33 and 5 tokens, with blocks of one q head and four query tiles, two and
+    two, three and two (six waves) and seven heads (the logits depend on every
+    position's attention through the second layer's K / V rows)."""
+    cfg = dataclasses.replace(models.TINY_Q8, name=f"pfe-{hd}-{nh}-{nkv}", head_dim=hd, n_head=nh, n_kv=nkv,
+                              max_t=128)
+    model, drv, ref = _pair(cfg, oracle)
+    lib.load().draco_set_prefill_chunk(33)
+    ids = np.random.default_rng(17).integers(0, cfg.vocab, 71).astype(np.int32)
+    lg = drv.prefill_chunk(ids, 0).copy()
+    lr = _serial_logits(ref, ids, 0)
+    assert rel_err(lg, lr) <= 1e-4
+
+
+@pytest.mark.parametrize("chunk", [1, 4, 5, 33])
+@pytest.mark.parametrize("n_used", [1, 3])
+def test_moe_prefill_matches_oracle_serial(oracle, chunk, n_used):
+    """A MoE model's prompt in chunks (the router, top-k and expert grouping
+    of all rows on the device) against the oracle's token-serial run, at chunk
+    lengths around the router's four tokens a block and the experts' 32-token
+    tiles."""
+    cfg = dataclasses.replace(models.MOE_TINY, name=f"moe-pf-{n_used}", hidden=1024, n_head=8, n_kv=2,
+                              n_exp=16, n_used=n_used, exp_ff=512, vocab=512, max_t=64, wscale=0.05)
+    model, drv, ref = _pair(cfg, oracle)
+    lib.load().draco_set_prefill_chunk(chunk)
+    ids = np.random.default_rng(19).integers(0, cfg.vocab, 38).astype(np.int32)
+    lg = drv.prefill_chunk(ids, 0).copy()
+    lr = _serial_logits(ref, ids, 0)
+    assert rel_err(lg, lr) <= 1e-4
+
+
 @pytest.mark.parametrize("cfgname,fname", [("tiny-kquant", "llama_tiny_k.npz"), ("tiny-q8_0", "llama_tiny_q8.npz")])
 def test_generate_token_serial_prompt(cfgname, fname):
     """draco_llama_generate with the chunked prefill switched off feeds the
