@@ -609,15 +609,24 @@ __global__ __launch_bounds__(512) void k_moe_route(const float* __restrict__ X, 
     __syncthreads();
     for (int e = w; e < n_exp; e += 8) {
         float4 acc[RT] = {};
-        for (int i = lane * 4; i < n_in; i += 256) {
-            const float4 g = ld4(gi + (size_t)e * n_in + i);
+        // eight of the row's float4s requested together (one at a time the 64
+        // round trips of a wave's 16 experts took 64 us at 191 tokens)
+        for (int i0 = lane * 4; i0 < n_in; i0 += 2048) {
+            float4 g[8];
 #pragma unroll
-            for (int t = 0; t < RT; t++) {
-                const float4 x = ld4(xs + (size_t)t * n_in + i);
-                acc[t].x = fmaf(x.x, g.x, acc[t].x);
-                acc[t].y = fmaf(x.y, g.y, acc[t].y);
-                acc[t].z = fmaf(x.z, g.z, acc[t].z);
-                acc[t].w = fmaf(x.w, g.w, acc[t].w);
+            for (int q = 0; q < 8; q++) g[q] = ld4(gi + (size_t)e * n_in + min(i0 + 256 * q, n_in - 4));
+#pragma unroll
+            for (int q = 0; q < 8; q++) {
+                const int i = i0 + 256 * q;
+                if (i < n_in)
+#pragma unroll
+                    for (int t = 0; t < RT; t++) {
+                        const float4 x = ld4(xs + (size_t)t * n_in + i);
+                        acc[t].x = fmaf(x.x, g[q].x, acc[t].x);
+                        acc[t].y = fmaf(x.y, g[q].y, acc[t].y);
+                        acc[t].z = fmaf(x.z, g[q].z, acc[t].z);
+                        acc[t].w = fmaf(x.w, g[q].w, acc[t].w);
+                    }
             }
         }
 #pragma unroll
