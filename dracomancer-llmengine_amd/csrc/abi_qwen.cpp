@@ -1092,7 +1092,9 @@ bool qstack_has_moe(const QStack* s) {
     return false;
 }
 
-int g_qwen_chunk = 64;
+// 2000-token prompt and 32 tokens: 12.3 ms in chunks of 64, 9.3 of 128, 8.7 of
+// 192, 8.1 of 256 (every chunk reads every weight once)
+int g_qwen_chunk = QCHUNK_MAX;
 
 // ids (device) [0, n) at positions pos0 .. through the chunked prefill;
 // leaves the last token's hidden row in s->X row (returned T - 1)
@@ -1273,7 +1275,7 @@ int draco_qwen_prefill(const void* layers, int n_layer, int h, const uint8_t* em
 }
 
 // Tokens per chunk of draco_qwen_prefill and of draco_qwen_generate's prompt
-// (default 64, at most 256; 0 = the prompt goes token by token).  Returns the
+// (default 256, the most; 0 = the prompt goes token by token).  Returns the
 // previous value; n < 0 only queries.
 int draco_set_qwen_chunk(int n) {
     std::lock_guard<std::recursive_mutex> g(api_mutex());

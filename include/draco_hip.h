@@ -388,7 +388,7 @@ typedef struct {
 /* One token: x[2048] (host, in / out) through every layer at position pos. */
 int draco_qwen_forward(float* x, int h, int pos, const void* layers, int n_layer);
 /* forward_chunk: ids[0..n) at positions pos0 .. pos0 + n - 1 in chunks
- * (draco_set_qwen_chunk, default 64): projections as f16-MFMA GEMMs over the
+ * (draco_set_qwen_chunk, default 256): projections as f16-MFMA GEMMs over the
  * chunk, the GDN scan token-serial, causal gated attention over the cache;
  * out_x[2048] (host, nullable) = the last token's hidden row.  Layers with a
  * MoE FFN are not served here (-1; draco_qwen_generate feeds them token by
