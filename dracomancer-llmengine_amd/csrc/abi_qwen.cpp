@@ -1027,7 +1027,7 @@ int qstack_positions(QStack* s, int pos0, int n) {
 // T tokens whose hidden rows are in s->X (positions pos0 .. pos0 + T - 1)
 // through every layer: the chunked form the reference runs in
 // src/qwen35_prefill.py:209-239 (_gdn :110-135, _full :137-168), with the
-// projections as f16-MFMA GEMMs over the chunk and the scan token-serial
+// projections as f16-MFMA GEMMs over the chunk
 int enqueue_qchunk(QStack* s, int T, int pos0, hipStream_t st) {
     auto gemm = [&](const DracoMat* m, const float* X, float* Y) {
         const GemmTo to = {m, Y};

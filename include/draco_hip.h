@@ -122,8 +122,9 @@ int draco_state_push(const void* layers, int n_layer);
  * tokens by argmax (first index on ties), all on the device.
  * prompt[0..n_prompt-1) goes through the chunked prefill below (token-serial
  * decode steps when the chunk size is 0); the last prompt token goes through
- * the first decode step.  With use_graph the token-serial prefill step and
- * the decode step are captured as HIP graphs and replayed.
+ * the first decode step.  With use_graph the decode step (and the token-serial
+ * prompt step where the call uses it) is captured as a HIP graph and replayed,
+ * while the chunked prompt runs.
  * out_hidden[h] = x after the last forward (nullable); stats[0] = decode ms,
  * stats[1] = prefill ms of the n_prompt - 1 tokens (nullable). */
 int draco_llama_generate(const void* layers, int n_layer, int h, float eps,
@@ -389,7 +390,7 @@ typedef struct {
 int draco_qwen_forward(float* x, int h, int pos, const void* layers, int n_layer);
 /* forward_chunk: ids[0..n) at positions pos0 .. pos0 + n - 1 in chunks
  * (draco_set_qwen_chunk, default 256): projections as f16-MFMA GEMMs over the
- * chunk, the GDN scan token-serial, causal gated attention over the cache;
+ * chunk, the GDN scan over it, causal gated attention over the cache;
  * out_x[2048] (host, nullable) = the last token's hidden row.  Layers with a
  * MoE FFN are not served here (-1; draco_qwen_generate feeds them token by
  * token). */
