@@ -33,7 +33,7 @@ __global__ __launch_bounds__(256) void k_pf_embed(const uint8_t* __restrict__ ba
 }
 
 // one block of 256 threads per token row; x held in registers (h <= 256 * PF_RMS_PT)
-constexpr int PF_RMS_PT = 16;
+constexpr int PF_RMS_PT = PF_H_MAX / 256;
 __global__ __launch_bounds__(256) void k_pf_rms(const float* __restrict__ X, const float* __restrict__ w,
                                                 float* __restrict__ Xn, int h, float eps) {
     __shared__ float red[4];
@@ -431,13 +431,13 @@ int pf_embed(const uint8_t* base, const DracoLayout& L, const int* ids, int T, f
 }
 
 int pf_rms(const float* X, const float* w, float* Xn, int T, int h, float eps, hipStream_t st) {
-    if (T < 1 || h > 256 * PF_RMS_PT) return -1;
+    if (T < 1 || h > PF_H_MAX) return -1;
     hipLaunchKernelGGL(k_pf_rms, dim3(T), dim3(256), 0, st, X, w, Xn, h, eps);
     return 0;
 }
 
 int pf_add_rms(float* X, const float* Y, const float* w, float* Xn, int T, int h, float eps, hipStream_t st) {
-    if (T < 1 || h > 256 * PF_RMS_PT) return -1;
+    if (T < 1 || h > PF_H_MAX) return -1;
     hipLaunchKernelGGL(k_pf_add_rms, dim3(T), dim3(256), 0, st, X, Y, w, Xn, h, eps);
     return 0;
 }

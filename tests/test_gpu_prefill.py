@@ -145,6 +145,18 @@ def test_moe_prefill_matches_oracle_serial(oracle, chunk, n_used):
     assert rel_err(lg, lr) <= 1e-4
 
 
+def test_moe_prefill_wider_than_the_chunk_norms(oracle):
+    """A MoE model of hidden rows beyond the chunk's norms (4096): its prompt
+    goes token by token through the decode layers."""
+    cfg = dataclasses.replace(models.MOE_TINY, name="moe-pf-wide", hidden=4352, n_layer=1, n_head=4, n_kv=2,
+                              head_dim=64, n_exp=8, n_used=2, exp_ff=256, vocab=256, max_t=16, wscale=0.05)
+    model, drv, ref = _pair(cfg, oracle)
+    ids = np.random.default_rng(23).integers(0, cfg.vocab, 5).astype(np.int32)
+    lg = drv.prefill_chunk(ids, 0).copy()
+    lr = _serial_logits(ref, ids, 0)
+    assert rel_err(lg, lr) <= 1e-4
+
+
 @pytest.mark.parametrize("cfgname,fname", [("tiny-kquant", "llama_tiny_k.npz"), ("tiny-q8_0", "llama_tiny_q8.npz")])
 def test_generate_token_serial_prompt(cfgname, fname):
     """draco_llama_generate with the chunked prefill switched off feeds the
