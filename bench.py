@@ -387,8 +387,9 @@ def prefill_gemm_configs2(lib, T=256, n_copies=4, iters=20):
     """configs[2] chunked prefill: one 256-token chunk through a Llama-1B layer's seven projections.
 
     fp32-equivalent TFLOP/s = 2*T*n_out*n_in / time.  The f16 MFMA work issued
-    is 2x that for Q4_K (hi and lo halves of x; plus 1/8 for the min term on a
-    K-padded 16-slot MFMA) and 4x for Q6_K (hi/lo x the two scale parts);
+    is 2x that for Q4_K (hi and lo halves of x; plus 1/4 for the min and centre
+    terms on K-padded 16-slot MFMAs) and 3x for Q6_K (hi and lo of x, and the
+    rest of the rounded weight with hi);
     `mfma_util` = issued f16 MFMA flops / (time * 2.5 PFLOP/s dense f16).
     """
     shapes = [("q", 5, 2048, 2048), ("k", 5, 512, 2048), ("v", 4, 512, 2048), ("o", 5, 2048, 2048),
@@ -403,7 +404,7 @@ def prefill_gemm_configs2(lib, T=256, n_copies=4, iters=20):
             raise RuntimeError(lib.last_error())
         us = float(o[0])
         flop = 2.0 * T * n_out * n_in
-        i8 = flop * (2.0 * 34.0 / 32.0 if code == 5 else 4.0)
+        i8 = flop * (36.0 / 16.0 if code == 5 else 3.0)
         res[name] = {"us": round(us, 2), "us_kernel_only": round(float(o[1]), 2),
                      "tflops_fp32_equiv": round(flop / us / 1e6, 1)}
         tot_us += us

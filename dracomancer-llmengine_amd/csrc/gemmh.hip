@@ -41,7 +41,7 @@
 // activations are read once per block and pass instead of once per row tile,
 // no wave waits for another inside a tile, and there is no K split over
 // blocks with partials in memory.  What bounds it: issue -- about 365 VALU and
-// 34 MFMA instructions a (row tile, super-block) for Q4_K, which overlap only
+// 36 MFMA instructions a (row tile, super-block) for Q4_K, which overlap only
 // in part (measured: 5.4k cycles a step of two waves against 2.2k of MFMA and
 // 2.9k of VALU); a 32-token tile re-forms the weights that the next one forms
 // too.  Against the kernel it replaced (activations staged in LDS super-block
