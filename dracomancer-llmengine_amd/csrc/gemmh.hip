@@ -20,7 +20,7 @@
 // Relative error against 64 bits, 2048-wide rows: Q4_K 1.7e-7 (2.3e-7 in one
 // chain, the sub-block sums added in sequence), Q5_K 1.2e-7 (a GEMV with exact
 // integer dots 1.26e-7; not centred 1.8e-7), Q6_K 1.3e-7 (1.6e-7 in one chain),
-// Q8_0 1.05e-7 (its GEMV 1.25e-7).
+// Q8_0 9.7e-8 at 2560 (its GEMV 1.26e-7).
 //
 // Operand order.  v_mfma_f32_32x32x16_f16: A lane l = row (token) l%32,
 // K 8*(l/32)..+7; B lane l = column (weight row) l%32, same K; C lane l =
@@ -420,6 +420,13 @@ __device__ __forceinline__ void tile_mma(WFrag<FM>& f, const WPtr<FM>& nx, const
         // block's dot (MFMAs from a zero accumulator), so d*q needs no
         // rounding.  Blocks past the row's end read the next row's quants
         // against activations that are zero, with a zero scale.
+        // The odd blocks' quants enter negated, and their scale too: the MFMA
+        // rounds the products' low bits down, not to nearest, so every block's
+        // dot is off in the same direction.  Block sums of one sign left a mean
+        // error of 3e-8 of the result's rms at 960-wide rows (5e-8 at 2560), the
+        // same for every token: what averages over tokens (the attention)
+        // kept it while its own size fell.  With the signs alternating it is
+        // below 1e-9.
         uint32_t dk[4];
         const int lv = f.live;
 #pragma unroll
@@ -439,8 +446,8 @@ __device__ __forceinline__ void tile_mma(WFrag<FM>& f, const WPtr<FM>& nx, const
                 for (int e = 0; e < 2; e++) {
                     v2h a, b;  // bytes XOR 0x80 read 128 + q
                     pairs((e ? (bh ? q.w : q.y) : (bh ? q.z : q.x)) ^ 0x80808080u, mk, a, b);
-                    p[2 * e] = u2(a - splat(1152.f));
-                    p[2 * e + 1] = u2(b - splat(1152.f));
+                    p[2 * e] = u2(k & 1 ? splat(1152.f) - a : a - splat(1152.f));
+                    p[2 * e + 1] = u2(k & 1 ? splat(1152.f) - b : b - splat(1152.f));
                 }
                 const v8h B = pack8(p[0], p[1], p[2], p[3]);
                 S = mfma16(lo[s], B, S);
@@ -449,7 +456,7 @@ __device__ __forceinline__ void tile_mma(WFrag<FM>& f, const WPtr<FM>& nx, const
             __builtin_amdgcn_sched_barrier(0);
             const float d = k < lv ? h2f((uint16_t)(dk[k >> 1] >> (16 * (k & 1)))) : 0.f;
 #pragma unroll
-            for (int i = 0; i < 16; i++) o[i] = fmaf(d, S[i], o[i]);
+            for (int i = 0; i < 16; i++) o[i] = fmaf(k & 1 ? -d : d, S[i], o[i]);
             if (k & 1) nx.quants(f, k >> 1);
             if (k == 3) nx.hdr(f);  // (not from the start: its 8 registers are not there)
         }

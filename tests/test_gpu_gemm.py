@@ -135,3 +135,22 @@ def test_gemm_slots_and_streams_vs_oracle(hip, oracle, code, T, n_out, n_in):
     ref = np.zeros_like(Y)
     assert oracle.lib.or_gemm(code, lib.pf(X), lib.pu8(W), T, n_out, n_in, lib.pf(ref)) == 0
     assert rel_err(Y, ref) <= TOL
+
+
+@pytest.mark.parametrize("n_out,n_in", [(960, 960), (320, 2560), (64, 4064)])
+def test_gemm_q8_errors_have_no_common_sign(hip, n_out, n_in):
+    """The rounding errors of a Q8_0 product against 64 bits average out over
+    tokens and rows.  Bound: 5e-9 of the result's rms, some three times the spread of
+    the mean of 64 x 64 independent errors of 1.2e-7 (a GEMV per token: 3e-10
+    over 256 x 960; a sum rounded downwards throughout: 3e-8 to 7e-8)."""
+    from dracohip import lib
+    T = 64
+    rng = np.random.default_rng(n_out + n_in)
+    W = lib.quantize(0, rng.standard_normal((n_out, n_in), dtype=np.float32) * np.float32(0.02))
+    X = rng.standard_normal((T, n_in)).astype(np.float32)
+    Y = np.zeros((T, n_out), np.float32)
+    hip.m5_gemm_q80(lib.pf(X), lib.pu8(W), T, n_out, n_in, lib.pf(Y))
+    blk = W.reshape(n_out, n_in // 32, 34)
+    w = blk[:, :, 2:].view(np.int8).astype(np.float64) * blk[:, :, :2].copy().view(np.float16).astype(np.float64)
+    ref = X.astype(np.float64) @ w.reshape(n_out, n_in).T
+    assert abs(np.mean(Y - ref)) <= 5e-9 * np.sqrt(np.mean(ref ** 2))
