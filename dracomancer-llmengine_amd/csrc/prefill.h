@@ -7,6 +7,9 @@
 
 #include "formats.h"
 
+// A (head, query, split) row of the chunk attention's partials: o[HD], m, l and
+// two floats of padding, so that every row's o starts 16-byte aligned
+constexpr int pf_part_row(int HD) { return HD + 4; }
 // key splits of the chunk attention and the partial buffer it needs (floats)
 int pf_attn_nsplit(int row0, int T);
 size_t pf_part_floats(int NH, int T, int HD, int nspl);

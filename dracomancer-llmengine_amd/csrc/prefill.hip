@@ -162,7 +162,7 @@ __global__ __launch_bounds__(256) void k_pf_rope_append(float* __restrict__ Q, c
 // query tiles; blockIdx.x = kv head * head groups + group.  K and V tiles are
 // double-buffered in LDS, rows padded by 4 floats (conflict-free for both
 // reads).  Writes the unnormalised (o[HD], m, l) of (head, query, split) for
-// the merge kernels.
+// the merge kernel (pf_part_row).
 //
 // Bound by the matrix instructions' issue on whole chunks (HD products of 32
 // cycles per 32 keys and wave).  Per launch, average over a prompt: 256-token
@@ -178,6 +178,7 @@ template <int HD>
 __global__ __launch_bounds__(512) void k_pf_attn(const float* __restrict__ Q, const float* __restrict__ kc,
                                                  const float* __restrict__ vc, float* __restrict__ part, int row0,
                                                  int T, int NH, int NKV, int nspl, int hg, float scale) {
+    static_assert(pf_part_row(HD) % 4 == 0, "16-byte aligned rows of partials");
     constexpr int RS = HD + 4, NL = HD / 32;  // LDS row, float4 of a tile per thread of a 256-thread block
     extern __shared__ __align__(16) float sm[];  // [2][K 32 rows, V 32 rows][RS]
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, n = lane & 15, u = lane >> 4, NT = blockDim.x;
@@ -293,7 +294,7 @@ __global__ __launch_bounds__(512) void k_pf_attn(const float* __restrict__ Q, co
     }
     l = rows_sum(l);
     if (!live) return;
-    float* pp = part + (((size_t)h * T + t) * nspl + blockIdx.z) * (HD + 2);
+    float* pp = part + (((size_t)h * T + t) * nspl + blockIdx.z) * pf_part_row(HD);
 #pragma unroll
     for (int dg = 0; dg < HD / 64; dg++)
 #pragma unroll
@@ -321,7 +322,7 @@ __device__ __forceinline__ float4 pf_merge4(const float* __restrict__ pp, int HD
     auto load = [&](int s0) {
 #pragma unroll
         for (int k = 0; k < MB; k++) {
-            const float* q = pp + (size_t)min(s0 + k, nspl - 1) * (HD + 2);
+            const float* q = pp + (size_t)min(s0 + k, nspl - 1) * pf_part_row(HD);
             ml[k] = *reinterpret_cast<const float2*>(q + HD);
             ov[k] = ld4(q + d);
         }
@@ -341,7 +342,7 @@ __device__ __forceinline__ float4 pf_merge4(const float* __restrict__ pp, int HD
     load(0);  // the only batch of up to 8 splits: one round trip
 #pragma unroll
     for (int k = 0; k < MB; k++) M = fmaxf(M, ml[k].x);
-    for (int s = MB; s < nspl; s++) M = fmaxf(M, pp[(size_t)s * (HD + 2) + HD]);
+    for (int s = MB; s < nspl; s++) M = fmaxf(M, pp[(size_t)s * pf_part_row(HD) + HD]);
     add(0);
     for (int s0 = MB; s0 < nspl; s0 += MB) {
         load(s0);
@@ -361,7 +362,7 @@ __global__ __launch_bounds__(256) void k_pf_merge(const float* __restrict__ part
     const int i = blockIdx.x * 256 + threadIdx.x, nd = HD / 4;
     if (i >= T * NH * nd) return;
     const int d = 4 * (i % nd), h = i / nd % NH, t = i / nd / NH;
-    const float* pp = part + ((size_t)h * T + t) * nspl * (HD + 2);
+    const float* pp = part + ((size_t)h * T + t) * nspl * pf_part_row(HD);
     float4 gv;
     if (gate) gv = ld4(gate + (size_t)t * g_row + (size_t)h * g_head + d);
     float4 v = pf_merge4(pp, HD, nspl, d);
@@ -421,7 +422,7 @@ int pf_attn_nsplit(int row0, int T) {
 // Enough for every chunk of up to T tokens: launch_attn's splits are at most
 // nspl, and at most PF_WAVES / waves rounded up, with at least NH * T / 16 waves.
 size_t pf_part_floats(int NH, int T, int HD, int nspl) {
-    return std::min((size_t)NH * T * nspl, (size_t)PF_QT * PF_WAVES + (size_t)NH * T) * (HD + 2);
+    return std::min((size_t)NH * T * nspl, (size_t)PF_QT * PF_WAVES + (size_t)NH * T) * pf_part_row(HD);
 }
 
 int pf_embed(const uint8_t* base, const DracoLayout& L, const int* ids, int T, float* X, hipStream_t st) {
