@@ -776,13 +776,14 @@ int enqueue_layer(DevModel* m, int l, float eps, hipStream_t st, const float* xi
 }
 
 // Whether the model's tokens can go through the batched (chunked) prefill:
-// attention shapes its kernel serves and FFNs that run over token rows (MoE
-// ones of rows that the chunk's norms hold); other models feed their prompts
-// through token-serial decode steps.
+// hidden rows that the chunk's norms hold, attention shapes its kernel serves
+// and FFNs that run over token rows; other models feed their prompts through
+// token-serial decode steps.
 bool chunk_ok(const DevModel* m) {
+    if (m->h > PF_H_MAX) return false;
     for (int l = 0; l < m->n_layer; l++) {
         if (!pf_attention_ok(m->attn[l]->NH, m->attn[l]->NKV, m->attn[l]->HD)) return false;
-        if (m->moe[l] && (m->h > PF_H_MAX || !draco_moe_layer_rows_ok(m->moe[l]))) return false;
+        if (m->moe[l] && !draco_moe_layer_rows_ok(m->moe[l])) return false;
     }
     return true;
 }

@@ -157,6 +157,24 @@ def test_moe_prefill_wider_than_the_chunk_norms(oracle):
     assert rel_err(lg, lr) <= 1e-4
 
 
+@pytest.mark.parametrize("base", ["TINY_K", "TINY_Q8"])
+def test_dense_prefill_wider_than_the_chunk_norms(oracle, base):
+    """A dense model of hidden rows beyond the chunk's norms (4096) and an
+    attention shape that the chunk serves: its prompt goes token by token, also
+    inside a generate call."""
+    cfg = dataclasses.replace(getattr(models, base), name="pf-wide-" + base, hidden=4352, n_layer=1, n_head=4, n_kv=2,
+                              head_dim=64, n_ff=512, vocab=256, max_t=16)
+    model, drv, ref = _pair(cfg, oracle)
+    ids = np.random.default_rng(29).integers(0, cfg.vocab, 5).astype(np.int32)
+    lg = drv.prefill_chunk(ids, 0).copy()
+    lr = _serial_logits(ref, ids, 0)
+    assert rel_err(lg, lr) <= 1e-4
+    drv.reset()
+    lib.load().draco_reset()
+    _, hidden, _ = drv.generate_device(ids, 1)
+    assert rel_err(hidden, ref.x) <= 1e-4
+
+
 @pytest.mark.parametrize("cfgname,fname", [("tiny-kquant", "llama_tiny_k.npz"), ("tiny-q8_0", "llama_tiny_q8.npz")])
 def test_generate_token_serial_prompt(cfgname, fname):
     """draco_llama_generate with the chunked prefill switched off feeds the
