@@ -29,6 +29,26 @@ struct GemmHArgs {
     int max_tiles;
     int rpb, n_rg;                // set by the launch
 };
+// The blocks of a launch: the pairs (major, minor), major of M, minor of m.
+// Blocks of one major share operands and lie on one XCD (block id mod 8)
+// where that spreads evenly: the majors of whole eights go to an XCD each,
+// the pairs of the other M % 8 majors in equal runs to all eight.
+struct GemmHMap {
+    int full, rem;  // blocks per XCD of the whole eights, of the rest
+};
+static inline __host__ __device__ GemmHMap gemmh_map(int M, int m) {
+    return {(M >> 3) * m, ((M & 7) * m + 7) >> 3};
+}
+// block's pair as major * m + minor, or -1
+static inline __host__ __device__ int gemmh_place(int M, int m, int block) {
+    const GemmHMap g = gemmh_map(M, m);
+    const int x = block & 7, loc = block >> 3;
+    if (loc < g.full) return (loc / m * 8 + x) * m + loc % m;
+    const int r = x * g.rem + loc - g.full;
+    return loc - g.full < g.rem && r < (M & 7) * m ? (M & ~7) * m + r : -1;
+}
+unsigned draco_gemmh_blocks(int M, int m);               // grid of the map above
+int draco_gemmh_place(int M, int m, int block);          // gemmh_place, for the map's test
 bool draco_gemmh_serves(int code);  // Q4_K, Q5_K, Q6_K, Q8_0
 bool draco_gemmh_mixes(int c0, int c1);
 size_t draco_gemmh_x_bytes(int T, int n_in);

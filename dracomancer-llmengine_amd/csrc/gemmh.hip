@@ -565,20 +565,22 @@ __device__ __forceinline__ void gemmr_body(const GemmHArgs& a, const GemmHSeg& s
     }
 }
 
-// XCD x runs blocks x, x + 8, ...: an XCD's consecutive blocks are the token
-// tiles of one row group, so a group's weights come from HBM once per XCD; in
-// grouped launches they are the row groups of one tile, whose activations stay
-// in that XCD's L2 (the experts' weights are read once anyway).
+// An XCD (blocks x, x + 8, ...) runs the token tiles of one row group one
+// after the other, so a group's weights come from HBM once per XCD; in grouped
+// launches the row groups of one tile, whose activations stay in that XCD's L2
+// (the experts' weights are read once anyway).  gemmh_place spreads what does
+// not divide by eight: with every row group whole on one XCD, launches of fewer
+// than 8 groups (more than 1024 tokens) left the other XCDs idle and those of 9
+// put two rounds on one (Q4_K: T=288 8192x2048 61.6 -> 35.4 us, T=4096
+// 2048x2048 362 -> 118).
 // F0 / F1: the formats that the launch's matrices have.
 template <int F0, int F1, int NSB, bool PAIR>
 __global__ __launch_bounds__(512) void k_gemmr(const GemmHArgs a) {
     extern __shared__ __align__(16) uint8_t sm[];
     const int ntt = a.groups ? a.max_tiles : (a.T + 31) >> 5;
-    const int loc = blockIdx.x >> 3;
-    const int x = blockIdx.x & 7;
-    const int tt = a.groups ? (loc / a.n_rg) * 8 + x : loc % ntt;
-    const int rg = a.groups ? loc % a.n_rg : (loc / ntt) * 8 + x;
-    if (rg >= a.n_rg || tt >= ntt) return;
+    const int m = a.groups ? a.n_rg : ntt, at = gemmh_place(a.groups ? ntt : a.n_rg, m, blockIdx.x);
+    if (at < 0) return;
+    const int maj = at / m, mnr = at - maj * m, tt = a.groups ? maj : mnr, rg = a.groups ? mnr : maj;
     const int s = a.nseg > 1 && rg >= a.seg[1].rg0 ? (a.nseg > 2 && rg >= a.seg[2].rg0 ? 2 : 1) : 0;
     const GemmHSeg& sg = a.seg[s];
     const uint8_t *W0 = sg.W, *W1 = PAIR ? a.seg[1].W : nullptr;
@@ -647,6 +649,12 @@ size_t draco_gemmh_x_bytes(int T, int n_in) { return (size_t)((T + 31) / 32) * (
 
 bool draco_gemmh_serves(int code) { return fm_of(code) != 0; }
 
+unsigned draco_gemmh_blocks(int M, int m) {
+    const GemmHMap g = gemmh_map(M, m);
+    return 8u * (unsigned)(g.full + g.rem);
+}
+int draco_gemmh_place(int M, int m, int block) { return gemmh_place(M, m, block); }
+
 // The formats one launch can mix: Q4_K or Q5_K with Q6_K (a Q4_K_M / Q5_K_M layer's q, k and v).
 bool draco_gemmh_mixes(int c0, int c1) {
     return c0 == c1 || ((c0 == DRACO_Q4_K || c0 == DRACO_Q5_K) && c1 == DRACO_Q6_K) ||
@@ -698,6 +706,6 @@ int draco_gemmh_launch(GemmHArgs& a, hipStream_t st) {
         a.n_rg += groups_of(s);
     }
     if (a.pair) a.nseg = 1;  // (the second matrix is read through its base)
-    const unsigned grid = (unsigned)(a.groups ? (ntt + 7) / 8 * 8 * a.n_rg : (a.n_rg + 7) / 8 * 8 * ntt);
+    const unsigned grid = draco_gemmh_blocks(a.groups ? ntt : a.n_rg, a.groups ? a.n_rg : ntt);
     return NSB == 4 ? pick<4>(a, f0, f1, grid, st) : pick<8>(a, f0, f1, grid, st);
 }

@@ -154,3 +154,17 @@ def test_gemm_q8_errors_have_no_common_sign(hip, n_out, n_in):
     w = blk[:, :, 2:].view(np.int8).astype(np.float64) * blk[:, :, :2].copy().view(np.float16).astype(np.float64)
     ref = X.astype(np.float64) @ w.reshape(n_out, n_in).T
     assert abs(np.mean(Y - ref)) <= 5e-9 * np.sqrt(np.mean(ref ** 2))
+
+
+@pytest.mark.parametrize("code", [5, 4, 0, 3])
+@pytest.mark.parametrize("T,n_out,n_in", [(290, 4200, 256), (1100, 100, 512), (2050, 70, 512), (8200, 33, 256)])
+def test_gemm_long_launches_vs_oracle(hip, oracle, code, T, n_out, n_in):
+    """More than 256 tokens: row groups that do not divide by the eight XCDs,
+    fewer than eight of them, one, and more token tiles than a round of blocks."""
+    from dracohip import lib
+    W, X = _case(code, T, n_out, n_in, T + n_out + code)
+    Y = np.full((T, n_out), np.nan, np.float32)
+    assert hip.m5_gemm_auto(code, lib.pf(X), lib.pu8(W), T, n_out, n_in, lib.pf(Y)) == 0
+    ref = np.zeros_like(Y)
+    assert oracle.lib.or_gemm(code, lib.pf(X), lib.pu8(W), T, n_out, n_in, lib.pf(ref)) == 0
+    assert rel_err(Y, ref) <= TOL
