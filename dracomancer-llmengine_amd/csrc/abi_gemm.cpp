@@ -18,6 +18,8 @@ extern "C" int draco_repack(int code, const uint8_t* src, int n_out, int n_in, u
 
 using namespace draco;
 
+constexpr int GEMM_PART = 18;  // scratch slot
+
 int draco_enqueue_gemms(const GemmTo* to, int n, const float* X, int T, uint8_t* digits, hipStream_t st) {
     bool have = false;  // X's operands are in `digits`
     GemmHArgs a = {};
@@ -43,11 +45,12 @@ int draco_enqueue_gemms(const GemmTo* to, int n, const float* X, int T, uint8_t*
         bool more = a.nseg < 3 && i + 1 < n && draco_gemmh_serves(to[i + 1].m->L.code);
         for (int k = 0; more && k < a.nseg; k++) more = draco_gemmh_mixes(a.seg[k].L.code, to[i + 1].m->L.code);
         if (more) continue;
+        // partial sums of long rows (grow-only; a caller that captures enqueues
+        // once before; without the memory the rows are not split)
+        if (const size_t n = draco_gemmh_part_floats(a)) a.part = (float*)scratch(GEMM_PART, sizeof(float) * n);
         if (draco_gemmh_launch(a, st)) return fail(-1, "gemm: launch rejected");
         a = GemmHArgs{};
     }
-    // (a plain-format matrix in between leaves an unlaunched group)
-    if (a.nseg && draco_gemmh_launch(a, st)) return fail(-1, "gemm: launch rejected");
     return 0;
 }
 
@@ -246,6 +249,7 @@ int draco_bench_gemm(int code, const uint8_t* W, int n_out, int n_in, int T, int
                 b.T = T;
                 b.xh = dd;
                 b.seg[0] = {mats[i % n_copies].dev, nullptr, L, dy, n_out, 0, 0};
+                if (const size_t n = draco_gemmh_part_floats(b)) b.part = (float*)scratch(GEMM_PART, sizeof(float) * n);
                 draco_gemmh_launch(b, st);
             }
         }

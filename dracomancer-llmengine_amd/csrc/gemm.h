@@ -27,7 +27,8 @@ struct GemmHArgs {
     const uint8_t* xh;            // activations from draco_gemmh_x_launch
     const int* groups;
     int max_tiles;
-    int rpb, n_rg;                // set by the launch
+    float* part;                  // draco_gemmh_part_floats floats; null: rows are not split over blocks
+    int rpb, n_rg, ksp, pps;      // set by the launch
 };
 // The blocks of a launch: the pairs (major, minor), major of M, minor of m.
 // Blocks of one major share operands and lie on one XCD (block id mod 8)
@@ -39,21 +40,26 @@ struct GemmHMap {
 static inline __host__ __device__ GemmHMap gemmh_map(int M, int m) {
     return {(M >> 3) * m, ((M & 7) * m + 7) >> 3};
 }
-// block's pair as major * m + minor, or -1
-static inline __host__ __device__ int gemmh_place(int M, int m, int block) {
+// block's pair (false: none)
+static inline __host__ __device__ bool gemmh_place(int M, int m, int block, int& major, int& minor) {
     const GemmHMap g = gemmh_map(M, m);
     const int x = block & 7, loc = block >> 3;
-    if (loc < g.full) return (loc / m * 8 + x) * m + loc % m;
-    const int r = x * g.rem + loc - g.full;
-    return loc - g.full < g.rem && r < (M & 7) * m ? (M & ~7) * m + r : -1;
+    const bool whole = loc < g.full;
+    const int i = whole ? loc : x * g.rem + loc - g.full, q = i / m;  // (one division)
+    major = whole ? 8 * q + x : (M & ~7) + q;
+    minor = i - q * m;
+    return whole || (loc - g.full < g.rem && i < (M & 7) * m);
 }
 unsigned draco_gemmh_blocks(int M, int m);               // grid of the map above
-int draco_gemmh_place(int M, int m, int block);          // gemmh_place, for the map's test
+int draco_gemmh_place(int M, int m, int block);          // major * m + minor or -1, for the map's test
+void draco_gemmh_plan(int n_out, int n_in, int T, int* out);  // one matrix: slots, row tiles, row splits, passes a split
 bool draco_gemmh_serves(int code);  // Q4_K, Q5_K, Q6_K, Q8_0
 bool draco_gemmh_mixes(int c0, int c1);
 size_t draco_gemmh_x_bytes(int T, int n_in);
 // rows (device, nullable): token t's values are row rows[t] of X, zeros where negative
 int draco_gemmh_x_launch(const float* X, int T, int n_in, uint8_t* buf, hipStream_t st, const int* rows = nullptr);
+// floats of partial sums that the launch of these arguments would use (0: none)
+size_t draco_gemmh_part_floats(const GemmHArgs& a);
 int draco_gemmh_launch(GemmHArgs& a, hipStream_t st);
 
 struct DracoMat;

@@ -464,12 +464,13 @@ __device__ __forceinline__ void tile_mma(WFrag<FM>& f, const WPtr<FM>& nx, const
 }
 
 constexpr int GR_NR = 2;  // row tiles (or gate / up pairs' halves) per reduction step
+constexpr size_t PART_MAX = (size_t)1 << 25;  // floats of partial sums that a launch takes at most (128 MB)
 
 // The steps of one block on one matrix (PAIR: on two of the same shape and
 // format, tile r of both, with the SwiGLU of the pair as the result).
 template <int FM, int NSB, bool PAIR>
 __device__ __forceinline__ void gemmr_body(const GemmHArgs& a, const GemmHSeg& sg, const uint8_t* W1, const uint8_t* W0,
-                                           int tt, int t_live, int r0, uint8_t* sm) {
+                                           int tt, int t_live, int r0, int z, uint8_t* sm) {
     constexpr int RS = 8 / NSB;
     const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int n = lane & 31, u = lane >> 5;
@@ -495,17 +496,19 @@ __device__ __forceinline__ void gemmr_body(const GemmHArgs& a, const GemmHSeg& s
         *reinterpret_cast<v4u32*>(mm + 1024 + lane * 16) = m1;
         if (lane < 32) reinterpret_cast<uint32_t*>(mm + 2048)[lane] = ts;
     };
-    const int passes = (nb + NSB - 1) / NSB;
+    // this block's passes of the row: split z of ksp
+    const int passes = min(a.pps, (nb + NSB - 1) / NSB - z * a.pps), sb0 = slot + z * a.pps * NSB;
+    float* const out = PAIR || a.ksp == 1 ? sg.Y : a.part + (size_t)z * a.T * sg.ldy;
     const int vo = wlane<FM>(L, n, u);
     // unit i of the block: row tile r0 + (i or i / 2) * RS + rs of matrix 0 (or 1 for the odd units of a pair)
     auto ptr = [&](int i, int b) {
         i = min(i, units - 1);
         return WPtr<FM>(PAIR && (i & 1) ? W1 : W0, L, r0 + (PAIR ? i >> 1 : i) * RS + rs, min(b, nb - 1), vo, n, u);
     };
-    load_a(min(slot, nb - 1));
+    load_a(min(sb0, nb - 1));
     WFrag<FM> f;
     {
-        const WPtr<FM> q = ptr(0, slot);
+        const WPtr<FM> q = ptr(0, sb0);
         q.hdr(f);
 #pragma unroll
         for (int v = 0; v < 4; v++) q.quants(f, v);
@@ -515,7 +518,7 @@ __device__ __forceinline__ void gemmr_body(const GemmHArgs& a, const GemmHSeg& s
         float* own = rd + (size_t)w * GR_NR * 1024 + lane;
         const int nr = min(GR_NR, units - st);
         for (int ps = 0; ps < passes; ps++) {
-            const int b = slot + ps * NSB;
+            const int b = sb0 + ps * NSB;
             if (b >= nb) {  // a slot past the row's end (uniform per wave)
                 if (ps == 0)
                     for (int e = 0; e < 16 * nr; e++) own[e * 64] = 0.f;
@@ -525,7 +528,7 @@ __device__ __forceinline__ void gemmr_body(const GemmHArgs& a, const GemmHSeg& s
             // the pass whose weights follow this one's (this slot's last pass may be short)
             const int nps = ps + 1 < passes && b + NSB < nb ? ps + 1 : 0;
             for (int r = 0; r < nr; r++) {
-                const WPtr<FM> nx = r + 1 < nr ? ptr(st + r + 1, b) : ptr(nps ? st : st + GR_NR, slot + nps * NSB);
+                const WPtr<FM> nx = r + 1 < nr ? ptr(st + r + 1, b) : ptr(nps ? st : st + GR_NR, sb0 + nps * NSB);
                 float o[16];
                 tile_mma<FM>(f, nx, hi, lo, mm, lane, o);
                 float* y = own + r * 1024;
@@ -560,13 +563,13 @@ __device__ __forceinline__ void gemmr_body(const GemmHArgs& a, const GemmHSeg& s
             if (PAIR) s = (s / (1.f + expf(-s))) * total(1, i);
             const int row = 32 * (r0 + (PAIR ? st >> 1 : st + r) * RS + rs) + n;
             const int tl = 8 * (i >> 2) + 4 * u + (i & 3);
-            if (row < L.n_out && tl < t_live) sg.Y[(size_t)(32 * tt + tl) * sg.ldy + row] = s;
+            if (row < L.n_out && tl < t_live) out[(size_t)(32 * tt + tl) * sg.ldy + row] = s;
         }
     }
 }
 
-// An XCD (blocks x, x + 8, ...) runs the token tiles of one row group one
-// after the other, so a group's weights come from HBM once per XCD; in grouped
+// An XCD (blocks x, x + 8, ...) runs the token tiles of one row group (of one
+// split of its rows) one after the other, so a group's weights come from HBM once per XCD; in grouped
 // launches the row groups of one tile, whose activations stay in that XCD's L2
 // (the experts' weights are read once anyway).  gemmh_place spreads what does
 // not divide by eight: with every row group whole on one XCD, launches of fewer
@@ -578,9 +581,10 @@ template <int F0, int F1, int NSB, bool PAIR>
 __global__ __launch_bounds__(512) void k_gemmr(const GemmHArgs a) {
     extern __shared__ __align__(16) uint8_t sm[];
     const int ntt = a.groups ? a.max_tiles : (a.T + 31) >> 5;
-    const int m = a.groups ? a.n_rg : ntt, at = gemmh_place(a.groups ? ntt : a.n_rg, m, blockIdx.x);
-    if (at < 0) return;
-    const int maj = at / m, mnr = at - maj * m, tt = a.groups ? maj : mnr, rg = a.groups ? mnr : maj;
+    int maj, mnr;
+    if (!gemmh_place(a.groups ? ntt : a.ksp * a.n_rg, a.groups ? a.n_rg : ntt, blockIdx.x, maj, mnr)) return;
+    const int tt = a.groups ? maj : mnr, z = !PAIR && a.ksp > 1 ? maj / a.n_rg : 0;  // (grouped: ksp 1)
+    const int rg = a.groups ? mnr : maj - z * a.n_rg;
     const int s = a.nseg > 1 && rg >= a.seg[1].rg0 ? (a.nseg > 2 && rg >= a.seg[2].rg0 ? 2 : 1) : 0;
     const GemmHSeg& sg = a.seg[s];
     const uint8_t *W0 = sg.W, *W1 = PAIR ? a.seg[1].W : nullptr;
@@ -593,8 +597,32 @@ __global__ __launch_bounds__(512) void k_gemmr(const GemmHArgs a) {
         live = 32;
     }
     const int r0 = (rg - sg.rg0) * a.rpb * (8 / NSB);
-    if (F0 == F1 || sg.fm == F0) gemmr_body<F0, NSB, PAIR>(a, sg, W1, W0, tt, live, r0, sm);
-    else gemmr_body<F1, NSB, PAIR>(a, sg, W1, W0, tt, live, r0, sm);
+    if (F0 == F1 || sg.fm == F0) gemmr_body<F0, NSB, PAIR>(a, sg, W1, W0, tt, live, r0, z, sm);
+    else gemmr_body<F1, NSB, PAIR>(a, sg, W1, W0, tt, live, r0, z, sm);
+}
+
+// Y = the sum of the ksp partial products, in their order
+__global__ __launch_bounds__(256) void k_gemmr_sum(const float* __restrict__ part, float* __restrict__ Y, size_t n,
+                                                   int ksp) {
+    for (size_t i = blockIdx.x * (size_t)256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256) {
+        float s = part[i];
+        for (int z = 1; z < ksp; z++) s += part[z * n + i];
+        Y[i] = s;
+    }
+}
+__global__ __launch_bounds__(256) void k_gemmr_sum4(const float4* __restrict__ part, float4* __restrict__ Y, size_t n,
+                                                    int ksp) {
+    for (size_t i = blockIdx.x * (size_t)256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256) {
+        float4 s = part[i];
+        for (int z = 1; z < ksp; z++) {
+            const float4 v = part[z * n + i];
+            s.x += v.x;
+            s.y += v.y;
+            s.z += v.z;
+            s.w += v.w;
+        }
+        Y[i] = s;
+    }
 }
 
 constexpr size_t GR_LDS = 2 * 8 * GR_NR * 4096 + 8 * (2048 + 128);
@@ -621,26 +649,25 @@ void launch_r(const GemmHArgs& a, unsigned grid, hipStream_t st) {
 }
 
 template <int NSB>
-int pick(const GemmHArgs& a, int f0, int f1, unsigned grid, hipStream_t st) {
+void pick(const GemmHArgs& a, int f0, int f1, unsigned grid, hipStream_t st) {
     if (a.pair) {
         switch (f0) {
-        case 1: launch_r<1, 1, NSB, true>(a, grid, st); return 0;
-        case 2: launch_r<2, 2, NSB, true>(a, grid, st); return 0;
-        case 3: launch_r<3, 3, NSB, true>(a, grid, st); return 0;
-        default: launch_r<4, 4, NSB, true>(a, grid, st); return 0;
+        case 1: launch_r<1, 1, NSB, true>(a, grid, st); return;
+        case 2: launch_r<2, 2, NSB, true>(a, grid, st); return;
+        case 3: launch_r<3, 3, NSB, true>(a, grid, st); return;
+        default: launch_r<4, 4, NSB, true>(a, grid, st); return;
         }
     }
     if (f0 == f1) {
         switch (f0) {
-        case 1: launch_r<1, 1, NSB, false>(a, grid, st); return 0;
-        case 2: launch_r<2, 2, NSB, false>(a, grid, st); return 0;
-        case 3: launch_r<3, 3, NSB, false>(a, grid, st); return 0;
-        default: launch_r<4, 4, NSB, false>(a, grid, st); return 0;
+        case 1: launch_r<1, 1, NSB, false>(a, grid, st); return;
+        case 2: launch_r<2, 2, NSB, false>(a, grid, st); return;
+        case 3: launch_r<3, 3, NSB, false>(a, grid, st); return;
+        default: launch_r<4, 4, NSB, false>(a, grid, st); return;
         }
     }
     if (f0 == 1) launch_r<1, 2, NSB, false>(a, grid, st);
     else launch_r<4, 2, NSB, false>(a, grid, st);
-    return 0;
 }
 
 }  // namespace
@@ -653,7 +680,10 @@ unsigned draco_gemmh_blocks(int M, int m) {
     const GemmHMap g = gemmh_map(M, m);
     return 8u * (unsigned)(g.full + g.rem);
 }
-int draco_gemmh_place(int M, int m, int block) { return gemmh_place(M, m, block); }
+int draco_gemmh_place(int M, int m, int block) {
+    int maj, mnr;
+    return gemmh_place(M, m, block, maj, mnr) ? maj * m + mnr : -1;
+}
 
 // The formats one launch can mix: Q4_K or Q5_K with Q6_K (a Q4_K_M / Q5_K_M layer's q, k and v).
 bool draco_gemmh_mixes(int c0, int c1) {
@@ -667,12 +697,82 @@ int draco_gemmh_x_launch(const float* X, int T, int n_in, uint8_t* buf, hipStrea
     return 0;
 }
 
+namespace {
+
+// What a launch does per block: NSB super-block slots, rpb row tiles per
+// stream, the row's passes (of NSB super-blocks) in ksp blocks of pps each.
+struct Plan {
+    int NSB, rpb, ksp, pps;
+};
+
 // Row tiles per block: as few as leave at most one block per CU (256).
 // Measured at T=256: 2048x2048 256 blocks 8.8 us, 512
 // 11.5; 12288 rows at T=64 11.6 / 15.9.  Four super-block slots (two row
 // streams) where rows have at most four super-blocks and there are row tiles
 // enough for both streams (960-wide rows of 30 tiles: 6.4 us with eight slots,
 // half of them idle, 8.0 with four).
+//
+// Rows of several passes load a block's activations again for every two row
+// tiles and pass.  A single matrix may have its passes in ksp blocks instead,
+// whose partial sums a second launch adds: where that is less work by the
+// costs below (us), measured at 8 waves a block.
+Plan plan(const GemmHArgs& a, bool may_split) {
+    const int ntt = a.groups ? a.max_tiles : (a.T + 31) / 32, nb = (a.n_in + 255) / 256;
+    const int walk = a.pair ? 1 : a.nseg;  // matrices whose rows the blocks walk
+    int rts = 0;
+    for (int s = 0; s < walk; s++) rts += (a.seg[s].L.n_out + 31) / 32;
+    Plan p;
+    p.NSB = nb <= 4 && rts * ntt >= 1024 ? 4 : 8;
+    const int RS = 8 / p.NSB, passes = (nb + p.NSB - 1) / p.NSB;
+    auto rpb_of = [&](int ksp) {
+        for (int rpb = 1;; rpb++) {
+            int rg = 0;
+            for (int s = 0; s < walk; s++) rg += ((a.seg[s].L.n_out + 31) / 32 + rpb * RS - 1) / (rpb * RS);
+            if ((long long)rg * ntt * ksp <= 256 || rpb >= rts) return rpb;
+        }
+    };
+    p.rpb = rpb_of(1);
+    p.ksp = 1;
+    p.pps = passes;
+    if (!may_split || passes == 1) return p;
+    constexpr double STEP = 2.2, LOAD = 1.8, SUM = 3.0;  // a tile's pass, an activation load, the second launch
+    auto cost = [&](const Plan& q) {
+        const double n = (double)a.T * a.seg[0].L.n_out;
+        return q.rpb * q.pps * STEP + (q.pps > 1 ? (q.rpb + GR_NR - 1) / GR_NR * q.pps : 1) * LOAD +
+               (q.ksp > 1 ? SUM + q.ksp * n * 8 / 5e6 : 0.);
+    };
+    for (int pps = passes - 1; pps >= 1; pps--) {
+        Plan q = p;
+        q.pps = pps;
+        q.ksp = (passes + pps - 1) / pps;
+        q.rpb = rpb_of(q.ksp);
+        if (q.ksp * ntt <= 256 && (size_t)q.ksp * a.T * a.seg[0].L.n_out <= PART_MAX && cost(q) < cost(p)) p = q;
+    }
+    return p;
+}
+bool splits(const GemmHArgs& a) { return a.nseg == 1 && !a.pair && !a.groups && a.seg[0].ldy == a.seg[0].L.n_out; }
+
+}  // namespace
+
+void draco_gemmh_plan(int n_out, int n_in, int T, int* out) {
+    GemmHArgs a = {};
+    a.nseg = 1;
+    a.n_in = n_in;
+    a.T = T;
+    a.seg[0].L.n_out = a.seg[0].ldy = n_out;
+    const Plan p = plan(a, true);
+    out[0] = p.NSB;
+    out[1] = p.rpb;
+    out[2] = p.ksp;
+    out[3] = p.pps;
+}
+
+size_t draco_gemmh_part_floats(const GemmHArgs& a) {
+    if (!splits(a)) return 0;
+    const Plan p = plan(a, true);
+    return p.ksp > 1 ? (size_t)p.ksp * a.T * a.seg[0].L.n_out : 0;
+}
+
 int draco_gemmh_launch(GemmHArgs& a, hipStream_t st) {
     if (a.nseg < 1 || a.nseg > 3 || a.T < 1 || a.n_in < 32 || a.n_in % 32 || !a.xh) return -1;
     if (a.groups && (a.max_tiles < 1 || a.nseg != (a.pair ? 2 : 1))) return -1;
@@ -687,25 +787,30 @@ int draco_gemmh_launch(GemmHArgs& a, hipStream_t st) {
         else if (g.fm != f0 && g.fm != f1) (g.fm == 2 ? f1 : f0) = g.fm;
     }
     if (a.pair && (a.nseg != 2 || f0 != f1 || a.seg[0].L.n_out != a.seg[1].L.n_out)) return -1;
-    const int ntt = a.groups ? a.max_tiles : (a.T + 31) / 32, nb = (a.n_in + 255) / 256;
-    const int walk = a.pair ? 1 : a.nseg;  // matrices whose rows the blocks walk
-    int rts = 0;
-    for (int s = 0; s < walk; s++) rts += (a.seg[s].L.n_out + 31) / 32;
-    const int NSB = nb <= 4 && rts * ntt >= 1024 ? 4 : 8, RS = 8 / NSB;
-    int rpb = 1;
-    auto groups_of = [&](int s) { return ((a.seg[s].L.n_out + 31) / 32 + rpb * RS - 1) / (rpb * RS); };
-    for (;; rpb++) {
-        int rg = 0;
-        for (int s = 0; s < walk; s++) rg += groups_of(s);
-        if ((long long)rg * ntt <= 256 || rpb >= rts) break;
-    }
-    a.rpb = rpb;
+    const Plan p = plan(a, a.part && splits(a));
+    const int ntt = a.groups ? a.max_tiles : (a.T + 31) / 32, walk = a.pair ? 1 : a.nseg, RS = 8 / p.NSB;
+    a.rpb = p.rpb;
+    a.ksp = p.ksp;
+    a.pps = p.pps;
     a.n_rg = 0;
     for (int s = 0; s < walk; s++) {
         a.seg[s].rg0 = a.n_rg;
-        a.n_rg += groups_of(s);
+        a.n_rg += ((a.seg[s].L.n_out + 31) / 32 + p.rpb * RS - 1) / (p.rpb * RS);
     }
     if (a.pair) a.nseg = 1;  // (the second matrix is read through its base)
-    const unsigned grid = draco_gemmh_blocks(a.groups ? ntt : a.n_rg, a.groups ? a.n_rg : ntt);
-    return NSB == 4 ? pick<4>(a, f0, f1, grid, st) : pick<8>(a, f0, f1, grid, st);
+    const unsigned grid = draco_gemmh_blocks(a.groups ? ntt : a.ksp * a.n_rg, a.groups ? a.n_rg : ntt);
+    if (p.NSB == 4) pick<4>(a, f0, f1, grid, st);
+    else pick<8>(a, f0, f1, grid, st);
+    if (p.ksp > 1) {
+        const size_t n = (size_t)a.T * a.seg[0].L.n_out;
+        const bool v4 = n % 4 == 0 && (uintptr_t)a.seg[0].Y % 16 == 0 && (uintptr_t)a.part % 16 == 0;
+        const size_t m = v4 ? n / 4 : n;
+        const unsigned blocks = (unsigned)std::min<size_t>((m + 255) / 256, 4096);
+        if (v4)
+            hipLaunchKernelGGL(k_gemmr_sum4, dim3(blocks), dim3(256), 0, st, (const float4*)a.part, (float4*)a.seg[0].Y, m,
+                               p.ksp);
+        else
+            hipLaunchKernelGGL(k_gemmr_sum, dim3(blocks), dim3(256), 0, st, a.part, a.seg[0].Y, m, p.ksp);
+    }
+    return 0;
 }

@@ -168,3 +168,18 @@ def test_gemm_long_launches_vs_oracle(hip, oracle, code, T, n_out, n_in):
     ref = np.zeros_like(Y)
     assert oracle.lib.or_gemm(code, lib.pf(X), lib.pu8(W), T, n_out, n_in, lib.pf(ref)) == 0
     assert rel_err(Y, ref) <= TOL
+
+
+@pytest.mark.parametrize("code", [5, 4, 0, 3])
+@pytest.mark.parametrize("T,n_out,n_in", [(1, 129, 6400), (40, 511, 14336), (33, 2048, 4352), (256, 4100, 8192)])
+def test_gemm_split_rows_vs_oracle(hip, oracle, code, T, n_out, n_in):
+    """Rows of several passes whose passes run in blocks of their own: a last
+    split with fewer super-blocks, results that are no multiple of four (the
+    scalar sum), several row tiles a block."""
+    from dracohip import lib
+    W, X = _case(code, T, n_out, n_in, T + n_out + code)
+    Y = np.full((T, n_out), np.nan, np.float32)
+    assert hip.m5_gemm_auto(code, lib.pf(X), lib.pu8(W), T, n_out, n_in, lib.pf(Y)) == 0
+    ref = np.zeros_like(Y)
+    assert oracle.lib.or_gemm(code, lib.pf(X), lib.pu8(W), T, n_out, n_in, lib.pf(ref)) == 0
+    assert rel_err(Y, ref) <= TOL
