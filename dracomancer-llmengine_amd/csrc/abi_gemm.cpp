@@ -3,7 +3,7 @@
 // m5_gemm_auto: src/m5/m5_gemm_fused.c:231-241 (0 = done, -1 = code not served,
 // the caller falls back); m5_gemm: src/m5/m5_gemm.c:249-272 (Y[T x n_out] =
 // X[T x n_in] . W^T).  Host pointers.  Q4_K, Q5_K, Q6_K and Q8_0 run on the
-// f16-MFMA GEMM (gemmh.hip).
+// f16-MFMA GEMM (gemmh.hip), the shortest Q8_0 and Q5_K ones as GEMVs.
 // m5_dequant_row: src/m5/m5_gemm.c:55-235, the GEMM library's row decoder.
 #include <stdio.h>
 #include <string.h>
@@ -20,12 +20,25 @@ using namespace draco;
 
 constexpr int GEMM_PART = 18;  // scratch slot
 
+// Whether T rows of one of n matrices on the same rows go through the GEMV, a
+// launch a token, instead of the GEMM, whose operand image and 32-token tile
+// cost the same for one token as for 32.  The plain formats always; Q8_0 and
+// Q5_K where it is faster.  Host calls of one matrix, GEMVs / GEMM in us: one
+// token 29-40 / 36-50, two 32-50 / 36-51, three 35-42 / 36-49 up to 4M weights
+// and 48-58 / 46-52 beyond, four 38-69 / 37-54.  Matrices that share an image
+// and a launch (q, k and v): one token only.
+static bool by_gemv(const DracoMat& m, int T, int n) {
+    if (!draco_gemmh_serves(m.L.code)) return true;
+    if (m.L.code != DRACO_Q8_0 && m.L.code != DRACO_Q5_K) return false;
+    return T == 1 || (n == 1 && (T == 2 || (T == 3 && (long long)m.L.n_out * m.L.n_in <= 1 << 22)));
+}
+
 int draco_enqueue_gemms(const GemmTo* to, int n, const float* X, int T, uint8_t* digits, hipStream_t st) {
     bool have = false;  // X's operands are in `digits`
     GemmHArgs a = {};
     for (int i = 0; i < n; i++) {
         const DracoMat& m = *to[i].m;
-        if (!draco_gemmh_serves(m.L.code)) {  // the plain formats: one GEMV per token
+        if (by_gemv(m, T, n)) {
             for (int t = 0; t < T; t++)
                 if (draco_gemv_launch(m, X + (size_t)t * m.L.n_in, to[i].Y + (size_t)t * m.L.n_out, nullptr, 0, m.L.n_out, st))
                     return fail(-1, "gemm: gemv launch rejected");
@@ -42,7 +55,7 @@ int draco_enqueue_gemms(const GemmTo* to, int n, const float* X, int T, uint8_t*
         s.Y = to[i].Y;
         s.ldy = m.L.n_out;
         // launched when full, or when the next matrix cannot join
-        bool more = a.nseg < 3 && i + 1 < n && draco_gemmh_serves(to[i + 1].m->L.code);
+        bool more = a.nseg < 3 && i + 1 < n && !by_gemv(*to[i + 1].m, T, n);
         for (int k = 0; more && k < a.nseg; k++) more = draco_gemmh_mixes(a.seg[k].L.code, to[i + 1].m->L.code);
         if (more) continue;
         // partial sums of long rows (grow-only; a caller that captures enqueues
@@ -56,7 +69,7 @@ int draco_enqueue_gemms(const GemmTo* to, int n, const float* X, int T, uint8_t*
 
 int draco_enqueue_swiglu(const DracoMat& gate, const DracoMat& up, const float* X, int T, float* G, float* U,
                          uint8_t* digits, hipStream_t st) {
-    if (!draco_gemmh_serves(gate.L.code) || gate.L.code != up.L.code || gate.L.n_out != up.L.n_out) {
+    if (by_gemv(gate, T, 2) || gate.L.code != up.L.code || gate.L.n_out != up.L.n_out) {
         const GemmTo to[2] = {{&gate, G}, {&up, U}};
         if (int rc = draco_enqueue_gemms(to, 2, X, T, digits, st)) return rc;
         dk_swiglu(G, U, T * gate.L.n_out, st);
@@ -229,8 +242,8 @@ int draco_bench_gemm(int code, const uint8_t* W, int n_out, int n_in, int T, int
     DRACO_HIP(hipMalloc(&dd, draco_gemmh_x_bytes(T, n_in)));
     DRACO_HIP(hipMemcpy(dx, xh.data(), sizeof(float) * xh.size(), hipMemcpyHostToDevice));
     hipStream_t st = stream();
-    // one eager product first: it writes the activation operands
-    if (enqueue_gemm(mats[0], dx, T, dy, dd, st)) return -1;
+    // one eager product first, and the activation operands of the kernel alone
+    if (enqueue_gemm(mats[0], dx, T, dy, dd, st) || draco_gemmh_x_launch(dx, T, n_in, dd, st)) return -1;
     DRACO_HIP(hipStreamSynchronize(st));
     hipEvent_t e0, e1;
     DRACO_HIP(hipEventCreate(&e0));

@@ -67,7 +67,7 @@ struct DracoMat;
 // rows (X, Y device, token-major).  The block formats (draco_gemmh_serves): X's
 // activation operands (f16 hi/lo) into `digits` (draco_gemmh_x_bytes(T,
 // n_in) bytes), then f16-MFMA launches of up to three matrices each; F32 and
-// F16: one GEMV per token.
+// F16, and Q8_0 / Q5_K of the shortest calls: one GEMV per token.
 struct GemmTo {
     const DracoMat* m;
     float* Y;

@@ -183,3 +183,16 @@ def test_gemm_split_rows_vs_oracle(hip, oracle, code, T, n_out, n_in):
     ref = np.zeros_like(Y)
     assert oracle.lib.or_gemm(code, lib.pf(X), lib.pu8(W), T, n_out, n_in, lib.pf(ref)) == 0
     assert rel_err(Y, ref) <= TOL
+
+
+@pytest.mark.parametrize("code", [0, 3])
+@pytest.mark.parametrize("T,n_out,n_in", [(1, 320, 1024), (2, 4096, 4096), (3, 512, 2048), (1, 33, 256)])
+def test_short_gemm_is_stacked_gemvs(hip, code, T, n_out, n_in):
+    """One and two tokens of Q8_0 and Q5_K, and three of a small matrix, take
+    the GEMV per token (the operand image and the 32-token tile cost more):
+    the same bits as m5_gemv's."""
+    from dracohip import lib
+    W, X = _case(code, T, n_out, n_in, T + n_out)
+    Y = np.full((T, n_out), np.nan, np.float32)
+    assert hip.m5_gemm_auto(code, lib.pf(X), lib.pu8(W), T, n_out, n_in, lib.pf(Y)) == 0
+    assert np.array_equal(Y, np.stack([lib.gemv(code, X[t], W, n_out, n_in) for t in range(T)]))
