@@ -932,6 +932,23 @@ int* op_state() {
 
 }  // namespace
 
+// Decode steps per graph of a generate call (the state advances on the device,
+// so consecutive steps capture as they run).  Four steps a graph save 5 us a
+// token over one (3.6 to 6 at 1 to 16 layers of the 1B shape), sixteen 1 to 2
+// more; a captured and instantiated kernel costs 1.8 us of host time.  So four
+// pay from 1.5 tokens a kernel of the step on (measured break-evens: 10 tokens
+// at 1 layer, 54 at 4, 123 at 16) and, where a chunked prompt runs meanwhile,
+// from 16 tokens on (the 16-layer stack behind 3 to 64 prompt tokens, one / four:
+// 2.7-3.1 / 3.4-3.6 ms at 4 tokens, 4.2-4.5 / 4.5-4.7 at 8, from 16 on the same),
+// and sixteen from 14 a kernel and 64 on (205 and 370 tokens at 1 and 4 layers).
+// Steps of more than 128 kernels keep one a graph (SmolLM2-360M's 130 and a
+// 48-layer MoE stack were 0.1-0.2% slower with several).
+int draco_graph_steps(int step_nodes, int n_gen, bool prompt_runs) {
+    if (step_nodes > 128 || n_gen < 4) return 1;
+    if (n_gen >= 14 * step_nodes + 64) return 16;
+    return 2 * n_gen >= 3 * step_nodes || (prompt_runs && n_gen >= 16) ? 4 : 1;
+}
+
 extern "C" {
 
 // src/m6_engine.c:31-37
@@ -1349,9 +1366,6 @@ int draco_llama_generate(const void* layers_v, int n_layer, int h, float eps, co
         dk_advance(m->state, n_layer, cursor, st);
         return 0;
     };
-    // tokens per decode graph: a graph of 16 steps decodes 0.2% faster than one
-    // of 4 but takes 2 ms more to capture, 400 tokens' worth
-    constexpr int GEN_STEPS = 4;
     // events and graphs are released on every return path (the guard's
     // destructor waits for the stream first, so no replay is still running)
     struct Guard {
@@ -1372,6 +1386,7 @@ int draco_llama_generate(const void* layers_v, int n_layer, int h, float eps, co
     for (hipEvent_t& e : G.ev) DRACO_HIP(hipEventCreate(&e));
     hipEvent_t e0 = G.ev[0], e1 = G.ev[1], e2 = G.ev[2], ep = G.ev[3];
     hipGraphExec_t* gx = G.gx;
+    int gsteps = 1;  // tokens per launch of gx[2]
     // The chunked prompt is enqueued first, so that it runs while the host
     // captures the decode graphs.
     if (n_chunked) {
@@ -1389,21 +1404,26 @@ int draco_llama_generate(const void* layers_v, int n_layer, int h, float eps, co
             hipError_t ce = hipStreamEndCapture(st, &G.gg[k]);
             if (rc) return rc;
             if (ce != hipSuccess) return fail(-2, "graph capture: %s", hipGetErrorString(ce));
+            return 0;
+        };
+        auto make = [&](int k) -> int {
             DRACO_HIP(hipGraphInstantiate(&gx[k], G.gg[k], nullptr, nullptr, 0));
             return 0;
         };
-        if (n_chunked < n_prompt - 1)  // token-serial prompt steps
+        if (n_chunked < n_prompt - 1) {  // token-serial prompt steps
             if (int rc = capture(0, 1, false)) return report(rc, "draco_llama_generate");
+            if (int rc = make(0)) return report(rc, "draco_llama_generate");
+        }
         if (int rc = capture(1, 1, true)) return report(rc, "draco_llama_generate");
-        // GEN_STEPS generated tokens in one graph (the state advances on the
-        // device, so consecutive steps capture as they run): one graph launch
-        // per GEN_STEPS tokens instead of per token.  Steps of more than 128
-        // kernels keep one graph per token (SmolLM2-360M's 130 and the 48-layer
-        // MoE stack were 0.1-0.2% slower with several).
         size_t step_nodes = 0;
         DRACO_HIP(hipGraphGetNodes(G.gg[1], nullptr, &step_nodes));
-        if (n_gen >= GEN_STEPS && step_nodes <= 128)
-            if (int rc = capture(2, GEN_STEPS, true)) return report(rc, "draco_llama_generate");
+        gsteps = draco_graph_steps((int)step_nodes, n_gen, n_chunked > 0);
+        if (gsteps > 1) {
+            if (int rc = capture(2, gsteps, true)) return report(rc, "draco_llama_generate");
+            if (int rc = make(2)) return report(rc, "draco_llama_generate");
+        }
+        if (n_gen % gsteps || gsteps == 1)  // the tokens left over
+            if (int rc = make(1)) return report(rc, "draco_llama_generate");
     }
     if (!n_chunked) DRACO_HIP(hipEventRecord(e0, st));  // (the stats leave the capture out)
     for (int i = n_chunked; i < n_prompt - 1; i++) {
@@ -1413,9 +1433,9 @@ int draco_llama_generate(const void* layers_v, int n_layer, int h, float eps, co
     if (fused_head) dk_embed(*em, dtok, cursor, m->w.xe, st);
     DRACO_HIP(hipEventRecord(e1, st));
     for (int i = 0; i < n_gen; i++) {
-        if (use_graph && gx[2] && i + GEN_STEPS <= n_gen) {
+        if (use_graph && gx[2] && i + gsteps <= n_gen) {
             DRACO_HIP(hipGraphLaunch(gx[2], st));
-            i += GEN_STEPS - 1;
+            i += gsteps - 1;
             continue;
         }
         if (use_graph) DRACO_HIP(hipGraphLaunch(gx[1], st));

@@ -585,3 +585,23 @@ def test_device_generate_from_gguf_file(tmp_path, cfgname, fname):
     toks, hidden, _ = drv.generate_device(model.prompt(), cfg.n_gen, use_graph=True)
     assert toks == list(g["tokens"])
     assert np.max(np.abs(hidden - g["hidden"])) <= hid_tol(g["hidden"])
+
+
+@pytest.mark.parametrize("n_prompt,n_gen", [(1, 3), (1, 32), (1, 35), (40, 17), (40, 33), (1, 320), (1, 327)])
+def test_generate_graph_lengths(n_prompt, n_gen):
+    """Generations of one, four and sixteen decode steps a graph, with and
+    without tokens left over, behind a chunked prompt and not: the same tokens
+    and last hidden row as without graphs."""
+    import dataclasses
+    from dracohip import lib
+    cfg = dataclasses.replace(models.TINY_K, name=f"steps-{n_prompt}-{n_gen}", n_layer=1, max_t=384)
+    model = models.build_llama(cfg, 0)
+    prompt = np.random.default_rng(31).integers(0, cfg.vocab, n_prompt).astype(np.int32)
+    got = []
+    for use_graph in (False, True):
+        lib.load().draco_reset()
+        drv = LlamaDriver(model, hip_engine_lib())
+        toks, hidden, _ = drv.generate_device(prompt, n_gen, use_graph=use_graph)
+        assert drv.tl[0][0] == n_prompt + n_gen - 1
+        got.append((list(toks), hidden.copy()))
+    assert got[0][0] == got[1][0] and np.array_equal(got[0][1], got[1][1])
