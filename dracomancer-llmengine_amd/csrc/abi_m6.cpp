@@ -775,15 +775,19 @@ int enqueue_layer(DevModel* m, int l, float eps, hipStream_t st, const float* xi
     return 0;
 }
 
-// Whether the model's tokens can go through the batched (chunked) prefill:
+// Whether n tokens of the model go through the batched (chunked) prefill:
 // hidden rows that the chunk's norms hold, attention shapes its kernel serves
-// and FFNs that run over token rows; other models feed their prompts through
-// token-serial decode steps.
-bool chunk_ok(const DevModel* m) {
+// and FFNs that run over token rows; other prompts go through token-serial
+// decode steps.  So do the shortest of MoE models, whose tokens read experts of
+// their own in either form while the chunk's launches are more (two layers of
+// 128 experts, 1 to 4 tokens: 196, 261, 328, 394 us token by token, 345, 366,
+// 387, 391 as a chunk).
+constexpr int MOE_CHUNK_MIN = 4;
+bool chunk_ok(const DevModel* m, int n) {
     if (m->h > PF_H_MAX) return false;
     for (int l = 0; l < m->n_layer; l++) {
         if (!pf_attention_ok(m->attn[l]->NH, m->attn[l]->NKV, m->attn[l]->HD)) return false;
-        if (m->moe[l] && !draco_moe_layer_rows_ok(m->moe[l])) return false;
+        if (m->moe[l] && (n < MOE_CHUNK_MIN || !draco_moe_layer_rows_ok(m->moe[l]))) return false;
     }
     return true;
 }
@@ -885,7 +889,7 @@ int enqueue_prefill_layer(DevModel* m, int l, int T, int pos0, int row0, float e
 // host tlen counters are not advanced here).  The last token's hidden state
 // is left in pf.X row (last chunk's T - 1); returns that T (0 on error).
 int enqueue_prefill(DevModel* m, const DracoMat* em, const int* ids, int n, int pos0, float eps, hipStream_t st) {
-    if (!chunk_ok(m)) {
+    if (!chunk_ok(m, n)) {
         fail(-1, "chunked prefill: this model's layers go token by token");
         return 0;
     }
@@ -1320,8 +1324,8 @@ int draco_llama_generate(const void* layers_v, int n_layer, int h, float eps, co
     // prompt[0 .. n_prompt - 1) goes through the chunked prefill when enabled
     // (the last prompt token goes through the first decode step, which also
     // runs the head); the token cursor then starts past those tokens
-    // (models outside chunk_ok feed the prompt through token-serial decode steps)
-    const int n_chunked = (g_prefill_chunk > 0 && n_prompt - 1 >= 2 && chunk_ok(m)) ? n_prompt - 1 : 0;
+    // (prompts outside chunk_ok go through token-serial decode steps)
+    const int n_chunked = (g_prefill_chunk > 0 && n_prompt - 1 >= 2 && chunk_ok(m, n_prompt - 1)) ? n_prompt - 1 : 0;
     if (n_chunked && ensure_pf(m, g_prefill_chunk)) return report(-2, "draco_llama_generate (prefill buffers)");
     ht[ntok + 8] = n_chunked;
     DRACO_HIP(hipMemcpyAsync(dtok, ht.data(), sizeof(int) * (ntok + 64), hipMemcpyHostToDevice, st));
@@ -1532,7 +1536,7 @@ int draco_llama_prefill(const void* layers_v, int n_layer, int h, float eps, con
         return report(-2, "draco_llama_prefill");
     }
     DRACO_HIP(hipMemcpyAsync(dids, ids, sizeof(int) * n, hipMemcpyHostToDevice, st));
-    if (!chunk_ok(m)) {
+    if (!chunk_ok(m, n)) {
         // token by token through the decode layers (the state of n
         // m6_forward_token calls): embedding of ids[cursor], every layer,
         // then the cursor and every tlen advance

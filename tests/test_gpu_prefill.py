@@ -145,6 +145,21 @@ def test_moe_prefill_matches_oracle_serial(oracle, chunk, n_used):
     assert rel_err(lg, lr) <= 1e-4
 
 
+@pytest.mark.parametrize("n", [1, 2, 3])
+def test_moe_prefill_of_few_tokens_is_token_serial(n):
+    """Up to three tokens of a MoE model go through the decode layers (a chunk
+    takes more launches and reads as many experts): the hidden row and the
+    generation after them are those of the tokens one by one, bit for bit."""
+    cfg = dataclasses.replace(models.MOE_TINY, name="moe-pf-few", n_exp=16, n_used=3, exp_ff=256, vocab=256, max_t=16,
+                              wscale=0.05)
+    model = models.build_llama(cfg, 0)
+    ids = np.random.default_rng(41).integers(0, cfg.vocab, n).astype(np.int32)
+    lib.load().draco_reset()
+    one, many = LlamaDriver(model, hip_engine_lib()), LlamaDriver(model, hip_engine_lib())
+    lr = _serial_logits(one, ids, 0)
+    assert np.array_equal(many.prefill_chunk(ids, 0), lr) and np.array_equal(many.x, one.x)
+
+
 def test_moe_prefill_wider_than_the_chunk_norms(oracle):
     """A MoE model of hidden rows beyond the chunk's norms (4096): its prompt
     goes token by token through the decode layers."""
