@@ -190,6 +190,29 @@ def test_dense_prefill_wider_than_the_chunk_norms(oracle, base):
     assert rel_err(hidden, ref.x) <= 1e-4
 
 
+@pytest.mark.parametrize("qk,v,ff,hidden", [(5, 4, 5, 1024), (3, 4, 3, 1024), (4, 4, 4, 768), (0, 0, 0, 960)])
+def test_prefill_two_stream_launches(oracle, qk, v, ff, hidden):
+    """Rows of at most four super-blocks and 1024 or more (row, token) tiles:
+    q, k and v (mixed formats: Q4_K or Q5_K with Q6_K) and the gate / up pair
+    run in the GEMM's two-stream form, the pair over an odd number of row tiles
+    (129), so that a block's second stream ends past the matrix.  Every token's
+    K / V rows of the second layer see the first layer's whole output."""
+    cfg = dataclasses.replace(models.TINY_K, name=f"pf2s-{qk}-{ff}", hidden=hidden, n_layer=2, n_head=32, n_kv=8,
+                              head_dim=128, n_ff=4128, vocab=256, max_t=256, wscale=0.05,
+                              codes=dict(models.TINY_K.codes, q=qk, k=qk, v=v, gate=ff, up=ff, down=0, emb=0, out=0))
+    model, drv, ref = _pair(cfg, oracle)
+    lib.load().draco_set_prefill_chunk(256)
+    ids = np.random.default_rng(37).integers(0, cfg.vocab, 230).astype(np.int32)
+    lg = drv.prefill_chunk(ids, 0).copy()
+    lr = _serial_logits(ref, ids, 0)
+    assert rel_err(lg, lr) <= 1e-4
+    assert lib.load().draco_state_pull(ct.cast(drv.descs, ct.c_void_p), drv.NL) == 0
+    n = len(ids) * cfg.n_kv * cfg.head_dim
+    for l in range(cfg.n_layer):
+        assert rel_err(drv.kc[l][:n], ref.kc[l][:n]) <= (1e-5 if l == 0 else 1e-4)
+        assert rel_err(drv.vc[l][:n], ref.vc[l][:n]) <= (1e-5 if l == 0 else 1e-4)
+
+
 @pytest.mark.parametrize("cfgname,fname", [("tiny-kquant", "llama_tiny_k.npz"), ("tiny-q8_0", "llama_tiny_q8.npz")])
 def test_generate_token_serial_prompt(cfgname, fname):
     """draco_llama_generate with the chunked prefill switched off feeds the
