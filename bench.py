@@ -279,10 +279,9 @@ def smol_decode_configs0(lib, use_graph=True):
 def moe_stack_configs3(lib, seed=3, use_graph=True):
     """the 48-layer Qwen3-30B-A3B-shaped MoE stack (attention 32 q /
     4 kv heads of 128, Q6_K; MoE FFN 128 experts, top 8, FFN 768, Q4_K experts,
-    fp32 router) decoding at context 512: a 448-token prompt fed token by token
-    through the graph-replayed decode step, then 64 greedy tokens (positions
-    448..511) timed with HIP events.  Bytes per token = attention weights +
-    the 8 routed experts' three matrices + the router, per layer, + the K/V rows
+    fp32 router) decoding at context 512: a 448-token prompt in chunks, then 64
+    greedy tokens (positions 448..511) timed with HIP events.  Bytes per token =
+    attention weights + the 8 routed experts' three matrices + the router, per layer, + the K/V rows
     read (mean over the decode positions) + the head and one embedding row."""
     import ctypes as ct
     from dracohip import models
@@ -316,7 +315,7 @@ def moe_stack_configs3(lib, seed=3, use_graph=True):
            "bytes_per_token": int(per_tok), "GB_s": round(per_tok * tok_s / 1e9, 1),
            "frac_of_peak": round(per_tok * tok_s / 1e9 / PEAK_HBM_GBS, 4),
            "stack_bytes_per_token_no_head": int(stack), "roof_tok_s": round(PEAK_HBM_GBS * 1e9 / per_tok, 1),
-           "prompt_tokens": cfg.n_prompt, "prompt_ms_token_serial": round(pre_ms, 1),
+           "prompt_tokens": cfg.n_prompt, "prompt_ms": round(pre_ms, 1),
            "greedy_tokens_repeat": toks == toks2,
            "shape": "48 layers: attention 32q/4kv x 128 Q6_K + MoE 128 experts top-8 FFN 768 Q4_K, fp32 router; "
                     "hidden 2048, vocab 151936 (untied Q6_K head), decode at positions 448..511"}
@@ -329,7 +328,7 @@ def qwen_stack_configs4(lib, seed=4, use_graph=True):
     """the 48-layer qwen35 hybrid stack (36 GDN layers of 16 q/k
     and 32 V heads of 128, 12 full-attention layers of 16 q / 2 KV heads of
     256, 3:1 interleave, Q4_K projections, hidden 2048): a 4096-token prompt,
-    all but its last token through the chunked prefill in 64-token chunks, then
+    all but its last token through the chunked prefill, then
     64 greedy decode steps (positions 4095..4158), graph-replayed.  Bytes per
     decode token = every layer's projection weights + the GDN state read and
     written + the beta / alpha rows + the full-attention K / V rows read (mean
@@ -342,14 +341,13 @@ def qwen_stack_configs4(lib, seed=4, use_graph=True):
     log(f"configs[4] stack built in {time.time() - t0:.1f}s ({stack.nbytes() / 1e9:.2f} GB)")
     L = lib.load()
     drv = Q.QwenStackDriver(stack, Q.hip_ops(L), lib=L)
-    old = L.draco_set_qwen_chunk(64)
+    chunk = L.draco_set_qwen_chunk(-1)
     prompt = stack.prompt()
     t0 = time.time()
     toks, _, _ = drv.generate_device(prompt, cfg.n_gen, use_graph=use_graph)
     log(f"configs[4] first run (upload + prompt + decode) {time.time() - t0:.1f}s")
     drv.reset()
     toks2, _, (dec_ms, pre_ms) = drv.generate_device(prompt, cfg.n_gen, use_graph=use_graph)
-    L.draco_set_qwen_chunk(old)
     gdn_w = full_w = 0
     for il, layer in enumerate(stack.layers):
         a = layer.arrays
@@ -370,7 +368,7 @@ def qwen_stack_configs4(lib, seed=4, use_graph=True):
            "bytes_per_token": int(per_tok), "GB_s": round(per_tok * tok_s / 1e9, 1),
            "frac_of_peak": round(per_tok * tok_s / 1e9 / PEAK_HBM_GBS, 4),
            "roof_tok_s": round(PEAK_HBM_GBS * 1e9 / per_tok, 1),
-           "prefill_tokens": n_pre, "prefill_chunk": 64, "prefill_ms": round(pre_ms, 1),
+           "prefill_tokens": n_pre, "prefill_chunk": chunk, "prefill_ms": round(pre_ms, 1),
            "prefill_tok_s": round(n_pre / (pre_ms / 1e3), 1), "greedy_tokens_repeat": toks == toks2,
            "shape": "48 layers 3:1 GDN (16 q/k + 32 V heads of 128) : full attention (16 q / 2 kv heads of 256), "
                     "Q4_K projections, hidden 2048, no FFN (the configuration's mixers), vocab 151936 untied Q6_K "

@@ -33,8 +33,8 @@ static bool by_gemv(const DracoMat& m, int T, int n) {
     return T == 1 || (n == 1 && (T == 2 || (T == 3 && (long long)m.L.n_out * m.L.n_in <= 1 << 22)));
 }
 
-int draco_enqueue_gemms(const GemmTo* to, int n, const float* X, int T, uint8_t* digits, hipStream_t st) {
-    bool have = false;  // X's operands are in `digits`
+int draco_enqueue_gemms(const GemmTo* to, int n, const float* X, int T, uint8_t* xh, hipStream_t st) {
+    bool have = false;  // X's operands are in `xh`
     GemmHArgs a = {};
     for (int i = 0; i < n; i++) {
         const DracoMat& m = *to[i].m;
@@ -44,11 +44,11 @@ int draco_enqueue_gemms(const GemmTo* to, int n, const float* X, int T, uint8_t*
                     return fail(-1, "gemm: gemv launch rejected");
             continue;
         }
-        if (!have && draco_gemmh_x_launch(X, T, m.L.n_in, digits, st)) return fail(-1, "gemm: activation launch rejected");
+        if (!have && draco_gemmh_x_launch(X, T, m.L.n_in, xh, st)) return fail(-1, "gemm: activation launch rejected");
         have = true;
         a.n_in = m.L.n_in;
         a.T = T;
-        a.xh = digits;
+        a.xh = xh;
         GemmHSeg& s = a.seg[a.nseg++];
         s.W = m.dev;
         s.L = m.L;
@@ -68,20 +68,20 @@ int draco_enqueue_gemms(const GemmTo* to, int n, const float* X, int T, uint8_t*
 }
 
 int draco_enqueue_swiglu(const DracoMat& gate, const DracoMat& up, const float* X, int T, float* G, float* U,
-                         uint8_t* digits, hipStream_t st) {
+                         uint8_t* xh, hipStream_t st) {
     if (by_gemv(gate, T, 2) || gate.L.code != up.L.code || gate.L.n_out != up.L.n_out) {
         const GemmTo to[2] = {{&gate, G}, {&up, U}};
-        if (int rc = draco_enqueue_gemms(to, 2, X, T, digits, st)) return rc;
+        if (int rc = draco_enqueue_gemms(to, 2, X, T, xh, st)) return rc;
         dk_swiglu(G, U, T * gate.L.n_out, st);
         return 0;
     }
-    if (draco_gemmh_x_launch(X, T, gate.L.n_in, digits, st)) return fail(-1, "gemm: activation launch rejected");
+    if (draco_gemmh_x_launch(X, T, gate.L.n_in, xh, st)) return fail(-1, "gemm: activation launch rejected");
     GemmHArgs a = {};
     a.nseg = 2;
     a.pair = 1;
     a.n_in = gate.L.n_in;
     a.T = T;
-    a.xh = digits;
+    a.xh = xh;
     a.seg[0] = {gate.dev, nullptr, gate.L, G, gate.L.n_out, 0, 0};
     a.seg[1] = {up.dev, nullptr, up.L, nullptr, gate.L.n_out, 0, 0};
     if (draco_gemmh_launch(a, st)) return fail(-1, "gemm: launch rejected");
@@ -92,9 +92,9 @@ namespace {
 
 bool served(int code) { return draco_gemmh_serves(code); }
 
-int enqueue_gemm(const DracoMat& m, const float* X, int T, float* Y, uint8_t* digits, hipStream_t st) {
+int enqueue_gemm(const DracoMat& m, const float* X, int T, float* Y, uint8_t* xh, hipStream_t st) {
     const GemmTo to = {&m, Y};
-    return draco_enqueue_gemms(&to, 1, X, T, digits, st);
+    return draco_enqueue_gemms(&to, 1, X, T, xh, st);
 }
 
 int gemm_host(int code, const float* X, const uint8_t* W, int T, int n_out, int n_in, float* Y) {
@@ -217,7 +217,7 @@ int m5_dequant_row(int code, const uint8_t* row, int n_in, float* out) {
 
 // Graph-replayed timing of the prefill GEMM on `n_copies` weight copies:
 // out[0] us per GEMM including the activation digitization, out[1] us per
-// GEMM kernel alone (digits computed once).
+// GEMM kernel alone (operand image computed once).
 int draco_bench_gemm(int code, const uint8_t* W, int n_out, int n_in, int T, int n_copies, int iters, float* out) {
     std::lock_guard<std::recursive_mutex> g(api_mutex());
     if (!served(code)) return fail(-1, "bench gemm: code %d not on the MFMA path", code);

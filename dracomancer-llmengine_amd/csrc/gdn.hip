@@ -666,7 +666,8 @@ __global__ __launch_bounds__(256) void k_gdn_rms(const GdnArgs a) {
 }
 
 // A split decode step leaves NSPL * NW = 16 partials (the ssm_out GEMV's
-// GNORM prologue reads 16); scans of several tokens use 8 waves per block.
+// GNORM prologue reads 16); scans of several tokens run in three launches, the
+// chain in blocks of 4 waves at a split of 8.
 // k_gdn_dec's waves per block (1 or 2; 0: k_gdn_scan<true, 2, 8>)
 int g_dec_waves = 2;
 

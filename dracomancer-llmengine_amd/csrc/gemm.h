@@ -65,14 +65,14 @@ int draco_gemmh_launch(GemmHArgs& a, hipStream_t st);
 struct DracoMat;
 // Y_i[t][row] = X[t] . W_i[row] for T token rows and n matrices on the same
 // rows (X, Y device, token-major).  The block formats (draco_gemmh_serves): X's
-// activation operands (f16 hi/lo) into `digits` (draco_gemmh_x_bytes(T,
+// activation operands (f16 hi/lo) into `xh` (draco_gemmh_x_bytes(T,
 // n_in) bytes), then f16-MFMA launches of up to three matrices each; F32 and
 // F16, and Q8_0 / Q5_K of the shortest calls: one GEMV per token.
 struct GemmTo {
     const DracoMat* m;
     float* Y;
 };
-int draco_enqueue_gemms(const GemmTo* to, int n, const float* X, int T, uint8_t* digits, hipStream_t st);
+int draco_enqueue_gemms(const GemmTo* to, int n, const float* X, int T, uint8_t* xh, hipStream_t st);
 // silu(gate . x) * (up . x) of T rows into G; U is scratch for formats whose pair is not one launch
 int draco_enqueue_swiglu(const DracoMat& gate, const DracoMat& up, const float* X, int T, float* G, float* U,
-                         uint8_t* digits, hipStream_t st);
+                         uint8_t* xh, hipStream_t st);

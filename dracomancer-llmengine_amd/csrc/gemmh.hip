@@ -5,9 +5,12 @@
 // most 63*8), Q5_K sc*(q-16) (63*16), Q8_0 q, all exact; Q6_K sc*(q-32) (|.| <= 4096)
 // as its f16 rounding plus the rest (-1, 0 or 1).  Per (token, 256-value
 // super-block) the activations are scaled by 2^-e (e = ilogb(max|x|) - 14, so
-// |x'| < 2^15) and split into two f16 (hi = f16(x'), lo = f16(x' - hi));
-// x' - hi - lo is below 2^-22 |x'|, and so is the one product left out (Q6_K's
-// lo * rest).  f16 x f16 products are exact in the MFMA's fp32 accumulation.
+// |x'| < 2^15) and split into two f16 (hi = f16(x'), lo = f16(x' - hi)): 23 of
+// an fp32 value's 24 bits, x' - hi - lo at most 2^-23 |x'|, or 2^-25 where lo is
+// an f16 subnormal (values below 2^-16 of the super-block's largest: 2^-39 of
+// that one).  The product left out (Q6_K's lo * rest) is below 2^-22 of the
+// value's.  f16 x f16 products are exact; the MFMA adds them to fp32 with their
+// low bits rounded down (tile_mma, Q8_0).
 // Per super-block and row, with 2^e the token's scale:
 //   Q4_K, Q5_K: y += 2^e * (d * (sum_k (sc*(q-z))_k x'_k + 32 * z * sum_sb sc_sb S'_sb)
 //                           - 32 * dmin * sum_sb m_sb S'_sb), z = 8 or 16,
@@ -16,11 +19,13 @@
 //   Q6_K: y += 2^e * d * sum (sc*(q-32)) x';
 //   Q8_0: y += 2^e * sum_blocks d_block * (sum q x').
 // The hi and the lo products accumulate apart: the lo sums are 2^-11 of the
-// hi ones, so their roundings vanish and the hi chain is half as long.
-// Relative error against 64 bits, 2048-wide rows: Q4_K 1.7e-7 (2.3e-7 in one
-// chain, the sub-block sums added in sequence), Q5_K 1.2e-7 (a GEMV with exact
-// integer dots 1.26e-7; not centred 1.8e-7), Q6_K 1.3e-7 (1.6e-7 in one chain),
-// Q8_0 9.7e-8 at 2560 (its GEMV 1.26e-7).
+// hi ones, so their roundings vanish and the hi chain is half as long.  (In one
+// MFMA the lo products lose their low bits to the hi ones', always downwards:
+// the min and centre sums formed so left a mean error of -3e-8.)
+// Relative error against 64 bits at 256 tokens: Q4_K 1.15e-7 (2048-wide rows;
+// 2.3e-7 in one chain, not centred), Q5_K 1.17e-7 (its GEMV 1.27e-7), Q6_K
+// 1.28e-7 (1.56e-7 with scales split in two), Q8_0 9.7e-8 (2560-wide; its GEMV
+// 1.26e-7, whose fp32 x keeps the 24th bit and values of any range).
 //
 // Operand order.  v_mfma_f32_32x32x16_f16: A lane l = row (token) l%32,
 // K 8*(l/32)..+7; B lane l = column (weight row) l%32, same K; C lane l =
@@ -40,16 +45,20 @@
 // tile's bytes as they fall free; the slots' sums meet in LDS.  So
 // activations are read once per block and pass instead of once per row tile,
 // no wave waits for another inside a tile, and there is no K split over
-// blocks with partials in memory.  What bounds it: issue -- about 365 VALU and
-// 36 MFMA instructions a (row tile, super-block) for Q4_K, which overlap only
-// in part (measured: 5.4k cycles a step of two waves against 2.2k of MFMA and
-// 2.9k of VALU); a 32-token tile re-forms the weights that the next one forms
-// too.  Against the kernel it replaced (activations staged in LDS super-block
-// by super-block, K split over the grid and a reduce launch), us a product
-// incl. reduce: T=256 2048x2048 Q4_K 14.7 -> 8.8, 8192x2048 34.9 -> 27.5,
-// 16384x2048 54.5 -> 49; T=64 12288x2048 20.2 -> 11.6, 2048x4096 13.2 -> 9.4;
-// T=256 512x2048 Q6_K 12.0 -> 6.5, 2048x8192 53.6 -> 47; T=31 Q8_0 960x960
-// 11.7 -> 6.4, 5120x960 13.8 -> 7.0; T=75 2048x2048 Q5_K 11.4 -> 6.8.
+// blocks with partials in memory unless rows are long (plan).  What bounds it:
+// issue -- about 307 VALU and 36 MFMA instructions a (row tile, super-block) for
+// Q4_K, which overlap only in part (a step of two waves takes 5.4k cycles, 2.3k
+// of MFMA and 2.5k of VALU); a 32-token tile re-forms the weights that the next
+// one forms too.  Against the kernel it replaced (activations staged in LDS
+// super-block by super-block, K split over the grid and a reduce launch), us a
+// product incl. reduce: T=256 2048x2048 Q4_K 15.7 -> 10.6, 8192x2048 31.6 -> 29.2;
+// T=64 8192x2048 17.3 -> 11.5; Q6_K T=256 512x2048 12.4 -> 7.6, 2048x8192 50.9 ->
+// 41.0, T=31 2048x8192 17.9 -> 12.3.  The two MFMAs of the centre term and its
+// shifts cost Q4_K some 6%: it is slower than that kernel in launches of many
+// tokens and rows (8192x2048 from 448 tokens on, 52 against 49 us) and on
+// 768-wide rows of 8192 (T=256 17.9 against 15.1: three of four slots busy).
+// Against GEMVs, whole host calls at 24 tokens: Q8_0 960x960 146 -> 46, Q5_K
+// 2048x2048 159 -> 60.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -75,8 +84,10 @@ constexpr int XH_SB = XH_A + XH_M + 32 * 4;     // + 32 token scales = 34944 B p
 // Within each 8 the order is 0 2 1 3 4 6 5 7: the weights' bytes 0, 2 and 1, 3
 // of a dword are formed as pairs.  Rows whose
 // length is not a multiple of 256 (Q8_0) are padded with zeros.  An infinite
-// value keeps its sign in hi with lo = 0, so it meets a row's weights as the
-// fp32 dot would (inf * 0 = NaN included); a NaN stays NaN.
+// value keeps its sign in hi with lo = 0 and a NaN stays NaN, so that token's
+// results are not finite and the others' are untouched.  A Q8_0 row meets it as
+// the fp32 dot would (inf * 0 = NaN included); Q4_K, Q5_K and Q6_K give NaN where
+// the dot is infinite (their infinite min, centre and rest terms cancel).
 __device__ __forceinline__ constexpr int kord(int i) { return (i & 4) + ((i & 1) << 1) + ((i >> 1) & 1); }
 __global__ __launch_bounds__(256) void k_gemmh_x(const float* __restrict__ X, int T, int n_in,
                                                  const int* __restrict__ rows, uint8_t* __restrict__ xh) {
@@ -705,17 +716,21 @@ struct Plan {
     int NSB, rpb, ksp, pps;
 };
 
-// Row tiles per block: as few as leave at most one block per CU (256).
-// Measured at T=256: 2048x2048 256 blocks 8.8 us, 512
-// 11.5; 12288 rows at T=64 11.6 / 15.9.  Four super-block slots (two row
-// streams) where rows have at most four super-blocks and there are row tiles
-// enough for both streams (960-wide rows of 30 tiles: 6.4 us with eight slots,
-// half of them idle, 8.0 with four).
+// Row tiles per block: as few as leave at most one block per CU (256).  With
+// up to 512: T=256 2048x2048 10.6 -> 13.4 us, 12288x2048 at T=64 14.7 -> 19.9 (at
+// T=128 23.3 -> 26.7).  Four super-block slots (two row streams) where rows have
+// at most four super-blocks and there are row tiles enough for both streams:
+// Q8_0 960x960 at T=31 7.5 us with eight slots, half of them idle, 8.9 with four;
+// 5120x960 at T=31 7.7 / 9.2, at T=75 (480 tiles) 9.9 / 9.6.
 //
 // Rows of several passes load a block's activations again for every two row
 // tiles and pass.  A single matrix may have its passes in ksp blocks instead,
 // whose partial sums a second launch adds: where that is less work by the
-// costs below (us), measured at 8 waves a block.
+// costs below (us), measured at 8 waves a block.  In blocks of whole rows / as
+// split, incl. the operand launch: Q6_K 2048x8192 at T=16 25.4 / 16.2, 64 28.7 /
+// 22.5, 128 32.5 / 31.6, 192 44.5 / 44.5 (not split at 256); 512x4096 at T=16 15.7
+// / 12.9; Q4_K 4096x14336 at T=16 37.0 / 24.5, 160 96.8 / 80.2.  Over 168 sizes
+// none is 2% slower split.
 Plan plan(const GemmHArgs& a, bool may_split) {
     const int ntt = a.groups ? a.max_tiles : (a.T + 31) / 32, nb = (a.n_in + 255) / 256;
     const int walk = a.pair ? 1 : a.nseg;  // matrices whose rows the blocks walk

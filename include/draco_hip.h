@@ -253,7 +253,10 @@ int draco_bench_granite_moe(const float* x0, const uint64_t* ptrs, const int* co
 /* ---- Prefill GEMM: Y[T x n_out] = X[T x n_in] . W^T ----------------------
  * m5_gemm_auto: src/m5/m5_gemm_fused.c:231-241 (0 done, -1 code not served:
  * the caller falls back).  m5_gemm: src/m5/m5_gemm.c:249-272.  Host pointers.
- * Served: Q4_K, Q5_K, Q6_K and Q8_0 on f16 MFMA (exact operands).
+ * Served: Q4_K, Q5_K, Q6_K and Q8_0 on f16 MFMA: exact weights, activations
+ * to 23 of fp32's 24 bits (and to 2^-39 of the largest of their 256 neighbours),
+ * fp32 sums; one to three tokens of Q8_0 and Q5_K by GEMV.  An infinite
+ * activation gives the K-quants NaN where the dot is infinite.
  * `wbuf` is not used. */
 int m5_gemm_auto(int code, const float* X, const uint8_t* W, int c, int n_out, int n_in, float* Y);
 int m5_gemm(int code, const float* X, const uint8_t* W, int T, int n_out, int n_in, float* Y, float* wbuf);
