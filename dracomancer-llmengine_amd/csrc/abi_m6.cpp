@@ -775,21 +775,31 @@ int enqueue_layer(DevModel* m, int l, float eps, hipStream_t st, const float* xi
     return 0;
 }
 
-// Whether n tokens of the model go through the batched (chunked) prefill:
+// Whether the model's tokens can go through the batched (chunked) prefill:
 // hidden rows that the chunk's norms hold, attention shapes its kernel serves
-// and FFNs that run over token rows; other prompts go through token-serial
-// decode steps.  So do the shortest of MoE models, whose tokens read experts of
-// their own in either form while the chunk's launches are more (two layers of
-// 128 experts, 1 to 4 tokens: 196, 261, 328, 394 us token by token, 345, 366,
-// 387, 391 as a chunk).
-constexpr int MOE_CHUNK_MIN = 4;
-bool chunk_ok(const DevModel* m, int n) {
+// and FFNs that run over token rows; other models feed their prompts through
+// token-serial decode steps.
+bool chunk_ok(const DevModel* m) {
     if (m->h > PF_H_MAX) return false;
     for (int l = 0; l < m->n_layer; l++) {
         if (!pf_attention_ok(m->attn[l]->NH, m->attn[l]->NKV, m->attn[l]->HD)) return false;
-        if (m->moe[l] && (n < MOE_CHUNK_MIN || !draco_moe_layer_rows_ok(m->moe[l]))) return false;
+        if (m->moe[l] && !draco_moe_layer_rows_ok(m->moe[l])) return false;
     }
     return true;
+}
+
+// The fewest tokens that a prompt takes as a chunk.  A MoE model's tokens read
+// experts of their own in either form and the chunk's launches are more: two
+// layers of 128 experts, 1 to 4 tokens, 196, 261, 328, 394 us token by token and
+// 345, 366, 387, 391 as a chunk.  In a call that generates n_gen tokens the
+// chunk runs while the decode graphs are captured, and the other form needs a
+// graph of its own (us, 1 / 2 layers, token by token against a chunk: 2 tokens
+// and 4 generated 422 / 660 against 480 / 740, 26 generated 1640 / 2530 against
+// 1595 / 2480; 3 tokens and 26 generated 1 layer 1770 against 1660).
+int chunk_min(const DevModel* m, int n_gen) {
+    for (const MoeLayer* p : m->moe)
+        if (p) return !n_gen ? 4 : (n_gen < 16 ? 3 : 2);
+    return n_gen ? 2 : 1;
 }
 
 // ---- chunked prefill (configs of the reference's forward_chunk,
@@ -889,7 +899,7 @@ int enqueue_prefill_layer(DevModel* m, int l, int T, int pos0, int row0, float e
 // host tlen counters are not advanced here).  The last token's hidden state
 // is left in pf.X row (last chunk's T - 1); returns that T (0 on error).
 int enqueue_prefill(DevModel* m, const DracoMat* em, const int* ids, int n, int pos0, float eps, hipStream_t st) {
-    if (!chunk_ok(m, n)) {
+    if (!chunk_ok(m)) {
         fail(-1, "chunked prefill: this model's layers go token by token");
         return 0;
     }
@@ -1324,8 +1334,8 @@ int draco_llama_generate(const void* layers_v, int n_layer, int h, float eps, co
     // prompt[0 .. n_prompt - 1) goes through the chunked prefill when enabled
     // (the last prompt token goes through the first decode step, which also
     // runs the head); the token cursor then starts past those tokens
-    // (prompts outside chunk_ok go through token-serial decode steps)
-    const int n_chunked = (g_prefill_chunk > 0 && n_prompt - 1 >= 2 && chunk_ok(m, n_prompt - 1)) ? n_prompt - 1 : 0;
+    // (shorter prompts and models outside chunk_ok: token-serial decode steps)
+    const int n_chunked = (g_prefill_chunk > 0 && n_prompt - 1 >= chunk_min(m, n_gen) && chunk_ok(m)) ? n_prompt - 1 : 0;
     if (n_chunked && ensure_pf(m, g_prefill_chunk)) return report(-2, "draco_llama_generate (prefill buffers)");
     ht[ntok + 8] = n_chunked;
     DRACO_HIP(hipMemcpyAsync(dtok, ht.data(), sizeof(int) * (ntok + 64), hipMemcpyHostToDevice, st));
@@ -1536,7 +1546,7 @@ int draco_llama_prefill(const void* layers_v, int n_layer, int h, float eps, con
         return report(-2, "draco_llama_prefill");
     }
     DRACO_HIP(hipMemcpyAsync(dids, ids, sizeof(int) * n, hipMemcpyHostToDevice, st));
-    if (!chunk_ok(m, n)) {
+    if (!chunk_ok(m) || n < chunk_min(m, 0)) {
         // token by token through the decode layers (the state of n
         // m6_forward_token calls): embedding of ids[cursor], every layer,
         // then the cursor and every tlen advance
