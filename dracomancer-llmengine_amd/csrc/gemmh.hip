@@ -728,9 +728,9 @@ struct Plan {
 // whose partial sums a second launch adds: where that is less work by the
 // costs below (us), measured at 8 waves a block.  In blocks of whole rows / as
 // split, incl. the operand launch: Q6_K 2048x8192 at T=16 25.4 / 16.2, 64 28.7 /
-// 22.5, 128 32.5 / 31.6, 192 44.5 / 44.5 (not split at 256); 512x4096 at T=16 15.7
-// / 12.9; Q4_K 4096x14336 at T=16 37.0 / 24.5, 160 96.8 / 80.2.  Over 168 sizes
-// none is 2% slower split.
+// 22.5, 160 43.1 / 39.4 (at 128 32.5 / 31.6 and 192 44.5 / 44.5: not split, the
+// second launch costs a chain of eager launches more than that); 512x4096 at T=16
+// 15.7 / 12.9; Q4_K 4096x14336 at T=16 37.0 / 24.5, 160 96.8 / 80.2.
 Plan plan(const GemmHArgs& a, bool may_split) {
     const int ntt = a.groups ? a.max_tiles : (a.T + 31) / 32, nb = (a.n_in + 255) / 256;
     const int walk = a.pair ? 1 : a.nseg;  // matrices whose rows the blocks walk
@@ -740,7 +740,8 @@ Plan plan(const GemmHArgs& a, bool may_split) {
     p.NSB = nb <= 4 && rts * ntt >= 1024 ? 4 : 8;
     const int RS = 8 / p.NSB, passes = (nb + p.NSB - 1) / p.NSB;
     auto rpb_of = [&](int ksp) {
-        for (int rpb = 1;; rpb++) {
+        // (at least the row tiles over the streams of 256 blocks)
+        for (int rpb = std::max(1, (int)((long long)rts * ntt * ksp / (256 * RS)));; rpb++) {
             int rg = 0;
             for (int s = 0; s < walk; s++) rg += ((a.seg[s].L.n_out + 31) / 32 + rpb * RS - 1) / (rpb * RS);
             if ((long long)rg * ntt * ksp <= 256 || rpb >= rts) return rpb;
@@ -756,14 +757,16 @@ Plan plan(const GemmHArgs& a, bool may_split) {
         return q.rpb * q.pps * STEP + (q.pps > 1 ? (q.rpb + GR_NR - 1) / GR_NR * q.pps : 1) * LOAD +
                (q.ksp > 1 ? SUM + q.ksp * n * 8 / 5e6 : 0.);
     };
+    Plan best = p;
     for (int pps = passes - 1; pps >= 1; pps--) {
         Plan q = p;
         q.pps = pps;
         q.ksp = (passes + pps - 1) / pps;
         q.rpb = rpb_of(q.ksp);
-        if (q.ksp * ntt <= 256 && (size_t)q.ksp * a.T * a.seg[0].L.n_out <= PART_MAX && cost(q) < cost(p)) p = q;
+        if (q.ksp * ntt <= 256 && (size_t)q.ksp * a.T * a.seg[0].L.n_out <= PART_MAX && cost(q) < cost(best)) best = q;
     }
-    return p;
+    // (blocks of several row tiles: up to 2 us less by these costs is a tie)
+    return cost(best) + (best.rpb > 2 ? 2.2 : 0.) < cost(p) ? best : p;
 }
 bool splits(const GemmHArgs& a) { return a.nseg == 1 && !a.pair && !a.groups && a.seg[0].ldy == a.seg[0].L.n_out; }
 
