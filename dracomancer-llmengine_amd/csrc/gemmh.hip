@@ -580,13 +580,13 @@ __device__ __forceinline__ void gemmr_body(const GemmHArgs& a, const GemmHSeg& s
 }
 
 // An XCD (blocks x, x + 8, ...) runs the token tiles of one row group (of one
-// split of its rows) one after the other, so a group's weights come from HBM once per XCD; in grouped
-// launches the row groups of one tile, whose activations stay in that XCD's L2
-// (the experts' weights are read once anyway).  gemmh_place spreads what does
-// not divide by eight: with every row group whole on one XCD, launches of fewer
-// than 8 groups (more than 1024 tokens) left the other XCDs idle and those of 9
-// put two rounds on one (Q4_K: T=288 8192x2048 61.6 -> 35.4 us, T=4096
-// 2048x2048 362 -> 118).
+// split of its rows) one after the other, so a group's weights come from HBM
+// once per XCD; in grouped launches the row groups of one tile, whose
+// activations stay in that XCD's L2 (the experts' weights are read once anyway).
+// gemmh_place spreads what does not divide by eight: with every row group whole
+// on one XCD, launches of fewer than 8 groups (more than 1024 tokens) left the
+// other XCDs idle and those of 9 put a second round of blocks on one (Q4_K: T=288
+// 8192x2048 61.6 -> 35.4 us, T=4096 2048x2048 362 -> 118).
 // F0 / F1: the formats that the launch's matrices have.
 template <int F0, int F1, int NSB, bool PAIR>
 __global__ __launch_bounds__(512) void k_gemmr(const GemmHArgs a) {
